@@ -61,16 +61,19 @@ def mac_flops_m2l(p, so, harmonic=False):
     """Useful flops of one M2L pair: the full form's multiply-adds, or the
     harmonic form's (rows and columns with n_z <= 1)."""
     if harmonic:
-        return 2 * sum((2 * n + 1) * (p - n + 1) ** 2 for n in range(p + 1))
+        return 2 * sum((2 * n + 1) * ((p - n + 1) ** 2 - so * so) for n in range(p - so + 1))
     from fmmgen_amd.codegen.layout import mac_count_m2l
     return 2 * mac_count_m2l(p, so)
 
 
-def harmonic_m2l(form, mode, so):
-    """Whether the M2L of this mode runs in the harmonic form."""
-    if so != 0 or form == "full" or mode == "bh":
+def harmonic_m2l(form, mode, so, order, ngroups):
+    """Whether the M2L of this mode runs in the harmonic form (automatic:
+    the library's rule, csrc/variant_decl.h)."""
+    if form == "full" or mode == "bh":
         return False
-    return form == "harmonic" or mode != "plain"
+    if form == "harmonic" or (mode != "plain" and so == 0):
+        return True
+    return ngroups >= 1 << 17 if mode != "plain" else order >= 6 or ngroups >= 1 << 14
 
 
 def cpu_baseline(cfg):
@@ -212,7 +215,7 @@ def main():
     ap.add_argument("--learned-thetas", default="0.5,0.55",
                     help="opening angles the learned modes may choose from (comma separated; empty: the tree's)")
     ap.add_argument("--m2l-form", default="auto", choices=["auto", "full", "harmonic"],
-                    help="M2L operand form of the timed mode (auto: harmonic for the mixed modes)")
+                    help="M2L operand form of the timed mode (auto: the faster one)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
@@ -262,6 +265,7 @@ def main():
                 break
         pfix = pfix or 12
         tree.set_order(pfix)
+        tree.set_m2l_form("full")  # the generated operator's sums: the method the target compares with
         ms_plain, wall_plain, ph_plain = timed(tree, F, "plain", args.steps, args.warmup)
         e_plain, _ = field_error(F, Fref, tg, so)
         print(f"# plain FP64 order {pfix}: {ms_plain:.3f} ms/eval (median), {wall_plain:.3f} (wall mean)",
@@ -285,7 +289,7 @@ def main():
     else:
         mode = args.mode
     tree.set_m2l_form(args.m2l_form)
-    harm = harmonic_m2l(args.m2l_form, mode, so)
+    harm = harmonic_m2l(args.m2l_form, mode, so, cfg["order"], info["m2l_groups"])
     if learned:
         from fmmgen_amd import learned as LN
         params, margin, _ = LN.load(args.model or LN.MODEL_PATH)

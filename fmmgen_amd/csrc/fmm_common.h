@@ -104,7 +104,7 @@ constexpr int kTile = 16;        // target cells per M2L tile (one MFMA column b
 // Operand form of the M2L GEMM: the full graded expansions (the generated
 // operator's sums), or the harmonic layout (folded multipoles, local rows
 // with n_z <= 1, the same sums by the harmonicity of 1/R); automatic = the
-// harmonic layout for the FP32 and BF16x3 GEMMs, the full form for FP64.
+// harmonic layout wherever it is the faster one (m2l_harmonic).
 enum : int { kM2LAuto = 0, kM2LFull = 1, kM2LHarmonic = 2 };
 
 struct M2LSchedule {

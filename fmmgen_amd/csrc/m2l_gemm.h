@@ -55,10 +55,12 @@ __host__ __device__ constexpr int slot_degree(int j) {
 // Slot layouts of the GEMM's rows (L) and columns (M).
 //   kGraded: every multi-index of degree <= p in the expansions' own graded
 //     order (below).
-//   kHarmonic (charges only): the multi-indices with n_z <= 1, (p + 1)^2
-//     slots; degree d holds slots d^2 .. (d + 1)^2 - 1 in the graded order
-//     restricted to n_z <= 1 (by a = n_y + n_z, then n_z), which keeps the
-//     D slots one MFMA step reads within the 8-bit offsets of its table.
+//   kHarmonic: the multi-indices with n_z <= 1, (p + 1)^2 slots; degree d
+//     holds slots d^2 .. (d + 1)^2 - 1 in the graded order restricted to
+//     n_z <= 1 (by a = n_y + n_z, then n_z), which keeps the D slots one MFMA
+//     step reads within the 8-bit offsets of its table.  Sources of order s
+//     have multipoles of degree s and more (columns from slot s^2) and local
+//     expansions of degree up to p - s.
 // Every D_k = d^k (1/R) is harmonic, D_{k+2z} = -D_{k+2x} - D_{k+2y}, so a
 // multipole term M_m with m_z >= 2 acts on the local expansion exactly as
 // -M_m placed at m - 2z + 2x and at m - 2z + 2y (the same degree: every
@@ -67,7 +69,8 @@ __host__ __device__ constexpr int slot_degree(int j) {
 // the translation of the folded multipole gives every L_n exactly, and the
 // L_n with n_z >= 2 follow from the same identity,
 //   L_(a,b,c+2k) = (-1)^k sum_i C(k,i) L_(a+2i, b+2(k-i), c)   (the unfold).
-// The GEMM then has (p + 1)^2 rows and columns instead of C(p + 3, 3).
+// The GEMM then has (p + 1)^2 rows and columns instead of C(p + 3, 3)
+// (charges; (p - s + 1)^2 rows and (p + 1)^2 - s^2 columns in general).
 enum : int { kGraded = 0, kHarmonic = 1 };
 
 __host__ __device__ constexpr int harm_degree(int j) {
@@ -75,19 +78,21 @@ __host__ __device__ constexpr int harm_degree(int j) {
   while ((d + 1) * (d + 1) <= j) ++d;
   return d;
 }
-__host__ __device__ constexpr int harm_size(int p) { return (p + 1) * (p + 1); }
+__host__ __device__ constexpr int harm_size(int p) { return p < 0 ? 0 : (p + 1) * (p + 1); }
+__host__ __device__ constexpr int harm_msize(int p, int so) { return harm_size(p) - harm_size(so - 1); }
+__host__ __device__ constexpr int harm_lsize(int p, int so) { return harm_size(p - so); }
 
 // MFMA steps of one translation: row blocks of 16 L slots by slices of KW
 // M slots, the steps whose lowest degrees sum to more than P dropped.
 template <int P, int SO, int KW, int LAY = kGraded>
 struct StepPlan {
-  static_assert(LAY == kGraded || SO == 0, "the harmonic layout is for charges");
-  static constexpr int LS = LAY == kHarmonic ? harm_size(P) : lsize(P, SO);
-  static constexpr int MS = LAY == kHarmonic ? harm_size(P) : msize(P, SO);
+  static constexpr int LS = LAY == kHarmonic ? harm_lsize(P, SO) : lsize(P, SO);
+  static constexpr int MS = LAY == kHarmonic ? harm_msize(P, SO) : msize(P, SO);
   static constexpr int NI = (LS + 15) / 16, NK = (MS + KW - 1) / KW;
-  static constexpr int OFF = nterms(SO - 1);  // M slot -> full index
+  static constexpr int OFF = nterms(SO - 1);                         // D slot -> graded index
+  static constexpr int COFF = LAY == kHarmonic ? harm_size(SO - 1) : OFF;  // M slot -> index in the layout
   static constexpr int row_degree(int n) { return LAY == kHarmonic ? harm_degree(n) : slot_degree(n); }
-  static constexpr int col_degree(int m) { return LAY == kHarmonic ? harm_degree(m) : slot_degree(m + OFF); }
+  static constexpr int col_degree(int m) { return LAY == kHarmonic ? harm_degree(m + COFF) : slot_degree(m + COFF); }
   static constexpr bool valid(int I, int K) {
     return 16 * I < LS && KW * K < MS && row_degree(16 * I) + col_degree(KW * K) <= P;
   }
@@ -190,7 +195,7 @@ static_assert(harm_layout_ok(15), "harmonic slots: a bijection onto the multi-in
 
 template <int LAY>
 __host__ __device__ constexpr MultiIdx lay_multi(int j, int off) {
-  return LAY == kHarmonic ? harm_multi(j) : slot_multi(j + off);
+  return LAY == kHarmonic ? harm_multi(j + off) : slot_multi(j + off);
 }
 
 // D-vector slot (full index - OFF) lane l reads at step (I, K): the entry
@@ -202,7 +207,7 @@ __host__ __device__ constexpr int step_lane_slot(int I, int K, int l) {
   constexpr int LS = Plan::LS, MS = Plan::MS, OFF = Plan::OFF;
   const int n = 16 * I + (l & 15), m = 4 * K + (l >> 4);
   if (n >= LS || m >= MS) return -1;
-  const MultiIdx a = lay_multi<LAY>(n, 0), b = lay_multi<LAY>(m, OFF);
+  const MultiIdx a = lay_multi<LAY>(n, 0), b = lay_multi<LAY>(m, Plan::COFF);
   if (a.x + a.y + a.z + b.x + b.y + b.z > P) return -1;
   return multi_slot(a.x + b.x, a.y + b.y, a.z + b.z) - OFF;
 }
@@ -634,16 +639,18 @@ struct HarmTables {
 // from LDS.
 constexpr int kHarmCellsPerWave = 4;
 
-// Fold: Mh[cell][j] for the (P + 1)^2 harmonic slots j from the graded
-// multipole M[cell] (stride ms).
-template <int P, typename T>
+// Fold: Mh[cell][j] for the harmonic slots of degree SO .. P from the graded
+// multipole M[cell] (stride ms); clears the cell's local row Lh[cell] of ls
+// slots, which the GEMM adds into.
+template <int P, int SO, typename T>
 __global__ __launch_bounds__(256) void k_harm_fold(int nc, const T* __restrict__ M, int ms, T* __restrict__ Mh,
-                                                   int hs) {
+                                                   int hs, T* __restrict__ Lh, int ls) {
   using H = HarmTables<P>;
   constexpr H tab{};
+  constexpr int J0 = harm_size(SO - 1), OFF = nterms(SO - 1), MS = H::GS - OFF;
   __shared__ short s_off[H::HS + 1], s_src[H::NF];
   __shared__ signed char s_w[H::NF];
-  __shared__ T s_row[4][H::GS];
+  __shared__ T s_row[4][MS];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   for (int i = tid; i <= H::HS; i += 256) s_off[i] = tab.fold_off[i];
   for (int i = tid; i < H::NF; i += 256) {
@@ -655,14 +662,16 @@ __global__ __launch_bounds__(256) void k_harm_fold(int nc, const T* __restrict__
     const int cell = c0 + c;
     __syncthreads();  // tables staged; the previous cell's row read
     if (cell < nc)
-      for (int j = lane; j < H::GS; j += 64) s_row[w][j] = M[(size_t)cell * ms + j];
+      for (int j = lane; j < MS; j += 64) s_row[w][j] = M[(size_t)cell * ms + j];
     __syncthreads();
-    if (cell < nc)
-      for (int j = lane; j < H::HS; j += 64) {
+    if (cell < nc) {
+      for (int j = J0 + lane; j < H::HS; j += 64) {
         double v = 0.0;
-        for (int t = s_off[j]; t < s_off[j + 1]; ++t) v += (double)s_w[t] * (double)s_row[w][s_src[t]];
-        Mh[(size_t)cell * hs + j] = (T)v;
+        for (int t = s_off[j]; t < s_off[j + 1]; ++t) v += (double)s_w[t] * (double)s_row[w][s_src[t] - OFF];
+        Mh[(size_t)cell * hs + j - J0] = (T)v;
       }
+      for (int j = lane; j < ls; j += 64) Lh[(size_t)cell * ls + j] = T(0);
+    }
   }
 }
 
@@ -909,7 +918,7 @@ void fill_wave_index32(std::vector<unsigned>& t) {
           const int n = 16 * I + (l & 15), m = 32 * K + 8 * (l >> 4) + e;
           unsigned u = (unsigned)msize(P, SO);
           if (n < Plan::LS && m < Plan::MS) {
-            const MultiIdx a = lay_multi<LAY>(n, 0), b = lay_multi<LAY>(m, Plan::OFF);
+            const MultiIdx a = lay_multi<LAY>(n, 0), b = lay_multi<LAY>(m, Plan::COFF);
             if (a.x + a.y + a.z + b.x + b.y + b.z <= P)
               u = (unsigned)(multi_slot(a.x + b.x, a.y + b.y, a.z + b.z) - Plan::OFF);
           }

@@ -508,15 +508,21 @@ void evaluate(Tree& t, int mode, int mask, double* F, hipStream_t st) {
   const int n = (int)t.n;
   const int nc = t.ncells;
   const size_t ms = (size_t)msize(t.order, SO), ls = (size_t)lsize(t.order, SO);
-  t.M.alloc((size_t)nc * ms);
-  t.L.alloc((size_t)nc * ls);
+  if (mode == 0) {  // the mixed modes keep their own FP32 expansions
+    t.M.alloc((size_t)nc * ms);
+    t.L.alloc((size_t)nc * ls);
+  }
   t.Fp2p.alloc((size_t)n * OUT);
   t.pS.alloc((size_t)n * SS);
   {
     PhaseTimer pt(t, kTPrep, st);
     k_gather_S<<<nblk(n, 256), 256, 0, st>>>(n, t.perm.get(), t.user_S, t.pS.get());
-    FMM_HIP(hipMemsetAsync(t.M.get(), 0, sizeof(double) * nc * ms, st));
-    FMM_HIP(hipMemsetAsync(t.L.get(), 0, sizeof(double) * nc * ls, st));
+    // P2M and M2M write every multipole slot and the harmonic form's unfold
+    // every local slot: cleared only when one of those is left out
+    if (mode == 0 && !((mask & kPhaseP2M) && (mask & kPhaseM2M)))
+      FMM_HIP(hipMemsetAsync(t.M.get(), 0, sizeof(double) * nc * ms, st));
+    if (mode == 0 && !((mask & kPhaseM2L) && t.sched.ngroups > 0 && m2l_harmonic(t, mode, t.order)))
+      FMM_HIP(hipMemsetAsync(t.L.get(), 0, sizeof(double) * nc * ls, st));
   }
   OrderTable<PMIN>::far(t.order, t, mode, mask, st);
   if (mask & kPhaseP2P) near_field(t, mode, st);

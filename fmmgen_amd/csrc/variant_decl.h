@@ -36,10 +36,23 @@ void bh_order(Tree& t, double* F, hipStream_t st);
 // M2L of the listed chunks at order Q on expansions stored at order ps.
 template <int Q>
 void m2l_class(Tree& t, int mode, const int* chunks, int nch, int ps, hipStream_t st);
-// Whether the M2L of an evaluation in this mode runs in the harmonic layout.
-inline bool m2l_harmonic(const Tree& t, int mode) {
-  if (SO != 0 || t.m2l_form == kM2LFull) return false;
-  return t.m2l_form == kM2LHarmonic || mode != 0;  // automatic: the mixed and learned modes
+// Whether the M2L of an evaluation runs in the harmonic layout (p: the order
+// the expansions are stored at).  Automatic: charges in the mixed and learned
+// modes always; otherwise where the shorter GEMM pays for the fold and unfold
+// launches, which is everywhere but at few groups and low order.  Measured
+// (full -> harmonic, one evaluation, theta 0.5, ncrit 64):
+//   FP64 charges   2^22 blobs, order 10 147 -> 66.6 ms; 2^20 uniform, order 8
+//                  11.2 -> 8.9 ms, order 2 6.73 -> 6.55 ms; 10^5 (156k groups)
+//                  order 4 932 -> 910 us; 2000 (383 groups) order 4 275 -> 278
+//                  us, order 6 318 -> 313 us
+//   FP32 dipoles   10^6 Plummer, theta 0.4, order 6 18.5 -> 13.5 ms; 10^5
+//                  order 4 927 -> 917 us; 2000 302 -> 311 us
+constexpr int kHarmMinOrder = 6, kHarmMinGroups = 1 << 14, kHarmMinGroupsMixed = 1 << 17;
+inline bool m2l_harmonic(const Tree& t, int mode, int p) {
+  if (t.m2l_form == kM2LFull) return false;
+  if (t.m2l_form == kM2LHarmonic) return true;
+  if (mode != 0) return SO == 0 || t.sched.ngroups >= kHarmMinGroupsMixed;
+  return p >= kHarmMinOrder || t.sched.ngroups >= kHarmMinGroups;
 }
 
 // Order-independent phases (defined in the base translation unit).

@@ -555,8 +555,7 @@ void far_field_mixed(Tree& t, int mode, int mask, hipStream_t st) {
   // (its M2L adds into Lf) and when there are no M2L groups.
   if (!((mask & kPhaseP2M) && (mask & kPhaseM2M)))
     FMM_HIP(hipMemsetAsync(t.Mf.get(), 0, sizeof(float) * nc * MS, st));
-  bool unfold_all = false;
-  if constexpr (SO == 0) unfold_all = (mask & kPhaseM2L) && t.sched.ngroups > 0 && m2l_harmonic(t, mode);
+  const bool unfold_all = (mask & kPhaseM2L) && t.sched.ngroups > 0 && m2l_harmonic(t, mode, P);
   if (!unfold_all) FMM_HIP(hipMemsetAsync(t.Lf.get(), 0, sizeof(float) * nc * LS, st));
   if (mask & kPhaseP2M) {
     PhaseTimer pt(t, kTP2M, st);

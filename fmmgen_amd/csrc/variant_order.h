@@ -133,23 +133,22 @@ const unsigned* ensure_index_table(Tree& t, hipStream_t st) {
 }
 
 // Harmonic-layout M2L around the GEMM: fold every cell's multipole (M,
-// graded, stride ms) into Mh, clear Lh (stride of order ps), then, after
+// graded, stride ms) into Mh and clear Lh (rows of order PS), then, after
 // the GEMM, store the unfolded rows into L (graded, stride ls).
 template <int PS, typename T>
 void harm_fold(Tree& t, const T* M, int ms, DevBuf<T>& Mh, DevBuf<T>& Lh, hipStream_t st) {
-  const int nc = t.ncells, hs = harm_size(PS);
+  const int nc = t.ncells, hs = harm_msize(PS, SO), ls = harm_lsize(PS, SO);
   Mh.alloc((size_t)nc * hs);
-  Lh.alloc((size_t)nc * hs);
+  Lh.alloc((size_t)nc * ls);
   if (nc == 0) return;
   constexpr int per = 4 * kHarmCellsPerWave;
-  k_harm_fold<PS, T><<<(nc + per - 1) / per, 256, 0, st>>>(nc, M, ms, Mh.get(), hs);
-  FMM_HIP(hipMemsetAsync(Lh.get(), 0, sizeof(T) * (size_t)nc * hs, st));
+  k_harm_fold<PS, SO, T><<<(nc + per - 1) / per, 256, 0, st>>>(nc, M, ms, Mh.get(), hs, Lh.get(), ls);
 }
 template <int PS, typename T>
 void harm_unfold(Tree& t, const DevBuf<T>& Lh, T* L, int ls, hipStream_t st) {
   if (t.ncells == 0) return;
   constexpr int per = 4 * kHarmCellsPerWave;
-  k_harm_unfold<PS, T><<<(t.ncells + per - 1) / per, 256, 0, st>>>(t.ncells, Lh.get(), harm_size(PS), L, ls);
+  k_harm_unfold<PS - SO, T><<<(t.ncells + per - 1) / per, 256, 0, st>>>(t.ncells, Lh.get(), harm_lsize(PS, SO), L, ls);
 }
 
 template <int P, int W, int LAY = kGraded>
@@ -173,18 +172,16 @@ void m2l_plain(Tree& t, hipStream_t st) {
   S.Dtab64.alloc((size_t)S.nkeys * Op<P>::MS);
   k_dtab<P, double, false><<<nblk(S.nkeys, 64), 64, 0, st>>>(S.nkeys, S.key_dx.get(), S.key_r.get(), S.Dtab64.get());
   const int grid = ((S.nchunks + 7) / 8) * 8;
-  if constexpr (SO == 0) {
-    if (m2l_harmonic(t, 0)) {
-      constexpr int W = m2l_waves<P, SO, double, kHarmonic>();
-      const unsigned* idx = ensure_index_table<P, W, kHarmonic>(t, st);
-      harm_fold<P, double>(t, t.M.get(), Op<P>::MS, t.Mh64, t.Lh64, st);
-      k_m2l_gemm<P, SO, double, false, W, kHarmonic><<<grid, 64 * W, 0, st>>>(
-          S.nchunks, grid, S.tile_cells.get(), S.chunk_tile.get(), S.chunk_g0.get(), S.chunk_g1.get(),
-          S.group_key.get(), S.group_src.get(), S.key_dlevel.get(), S.Dtab64.get(), idx, t.tile_order_ptr(), nullptr,
-          Op<P>::MS, harm_size(P), harm_size(P), t.Mh64.get(), t.Lh64.get());
-      harm_unfold<P, double>(t, t.Lh64, t.L.get(), Op<P>::LS, st);
-      return;
-    }
+  if (m2l_harmonic(t, 0, P)) {
+    constexpr int W = m2l_waves<P, SO, double, kHarmonic>();
+    const unsigned* idx = ensure_index_table<P, W, kHarmonic>(t, st);
+    harm_fold<P, double>(t, t.M.get(), Op<P>::MS, t.Mh64, t.Lh64, st);
+    k_m2l_gemm<P, SO, double, false, W, kHarmonic><<<grid, 64 * W, 0, st>>>(
+        S.nchunks, grid, S.tile_cells.get(), S.chunk_tile.get(), S.chunk_g0.get(), S.chunk_g1.get(),
+        S.group_key.get(), S.group_src.get(), S.key_dlevel.get(), S.Dtab64.get(), idx, t.tile_order_ptr(), nullptr,
+        Op<P>::MS, harm_msize(P, SO), harm_lsize(P, SO), t.Mh64.get(), t.Lh64.get());
+    harm_unfold<P, double>(t, t.Lh64, t.L.get(), Op<P>::LS, st);
+    return;
   }
   constexpr int W = m2l_waves<P, SO, double>();
   const unsigned* idx = ensure_index_table<P, W>(t, st);
@@ -269,16 +266,14 @@ void m2l_mixed(Tree& t, int mode, hipStream_t st) {
   if (S.ngroups == 0) return;
   S.Dtab32.alloc((size_t)S.nkeys * Op<P>::MS);
   k_dtab<P, float, true><<<nblk(S.nkeys, 64), 64, 0, st>>>(S.nkeys, S.key_dx.get(), S.key_r.get(), S.Dtab32.get());
-  const bool harm = m2l_harmonic(t, mode);
-  if constexpr (SO == 0)
-    if (harm) harm_fold<P, float>(t, t.Mf.get(), Op<P>::MS, t.Mhf, t.Lhf, st);
+  const bool harm = m2l_harmonic(t, mode, P);
+  if (harm) harm_fold<P, float>(t, t.Mf.get(), Op<P>::MS, t.Mhf, t.Lhf, st);
   if (t.use_tile_order && t.m2l_classes) {  // learned order: one launch per tile-order class
     t.m2l_classes(t, mode, P, st);
   } else {
     m2l_class<P>(t, mode, nullptr, S.nchunks, P, st);
   }
-  if constexpr (SO == 0)
-    if (harm) harm_unfold<P, float>(t, t.Lhf, t.Lf.get(), Op<P>::LS, st);
+  if (harm) harm_unfold<P, float>(t, t.Lhf, t.Lf.get(), Op<P>::LS, st);
 }
 
 // FP32 / BF16x3 M2L of the listed chunks (all when chunks == nullptr) at
@@ -291,16 +286,14 @@ void m2l_class(Tree& t, int mode, const int* chunks, int nch, int ps, hipStream_
   const int grid = ((nch + 7) / 8) * 8;
   const int ms = msize(ps, SO), ls = lsize(ps, SO);
   if (mode == 2) {  // BF16x3 split precision
-    if constexpr (SO == 0) {
-      if (m2l_harmonic(t, mode)) {
-        constexpr int W32 = m2l_waves32<Q, SO, kHarmonic>();
-        const unsigned* idx = ensure_index_table32<Q, W32, kHarmonic>(t, st);
-        k_m2l_bf16x3<Q, SO, W32, kHarmonic><<<grid, 64 * W32, 0, st>>>(
-            nch, grid, S.tile_cells.get(), S.chunk_tile.get(), S.chunk_g0.get(), S.chunk_g1.get(), S.group_key.get(),
-            S.group_src.get(), S.key_dlevel.get(), S.Dtab32.get(), idx, t.tile_order_ptr(), chunks, ms,
-            harm_size(ps), harm_size(ps), t.Mhf.get(), t.Lhf.get());
-        return;
-      }
+    if (m2l_harmonic(t, mode, ps)) {
+      constexpr int W32 = m2l_waves32<Q, SO, kHarmonic>();
+      const unsigned* idx = ensure_index_table32<Q, W32, kHarmonic>(t, st);
+      k_m2l_bf16x3<Q, SO, W32, kHarmonic><<<grid, 64 * W32, 0, st>>>(
+          nch, grid, S.tile_cells.get(), S.chunk_tile.get(), S.chunk_g0.get(), S.chunk_g1.get(), S.group_key.get(),
+          S.group_src.get(), S.key_dlevel.get(), S.Dtab32.get(), idx, t.tile_order_ptr(), chunks, ms,
+          harm_msize(ps, SO), harm_lsize(ps, SO), t.Mhf.get(), t.Lhf.get());
+      return;
     }
     constexpr int W32 = m2l_waves32<Q, SO>();
     const unsigned* idx = ensure_index_table32<Q, W32>(t, st);
@@ -310,16 +303,14 @@ void m2l_class(Tree& t, int mode, const int* chunks, int nch, int ps, hipStream_
                                              ms, ms, ls, t.Mf.get(), t.Lf.get());
     return;
   }
-  if constexpr (SO == 0) {
-    if (m2l_harmonic(t, mode)) {
-      constexpr int W = m2l_waves<Q, SO, float, kHarmonic>();
-      const unsigned* idx = ensure_index_table<Q, W, kHarmonic>(t, st);
-      k_m2l_gemm<Q, SO, float, true, W, kHarmonic><<<grid, 64 * W, 0, st>>>(
-          nch, grid, S.tile_cells.get(), S.chunk_tile.get(), S.chunk_g0.get(), S.chunk_g1.get(), S.group_key.get(),
-          S.group_src.get(), S.key_dlevel.get(), S.Dtab32.get(), idx, t.tile_order_ptr(), chunks, ms,
-          harm_size(ps), harm_size(ps), t.Mhf.get(), t.Lhf.get());
-      return;
-    }
+  if (m2l_harmonic(t, mode, ps)) {
+    constexpr int W = m2l_waves<Q, SO, float, kHarmonic>();
+    const unsigned* idx = ensure_index_table<Q, W, kHarmonic>(t, st);
+    k_m2l_gemm<Q, SO, float, true, W, kHarmonic><<<grid, 64 * W, 0, st>>>(
+        nch, grid, S.tile_cells.get(), S.chunk_tile.get(), S.chunk_g0.get(), S.chunk_g1.get(), S.group_key.get(),
+        S.group_src.get(), S.key_dlevel.get(), S.Dtab32.get(), idx, t.tile_order_ptr(), chunks, ms,
+        harm_msize(ps, SO), harm_lsize(ps, SO), t.Mhf.get(), t.Lhf.get());
+    return;
   }
   constexpr int W = m2l_waves<Q, SO, float>();
   const unsigned* idx = ensure_index_table<Q, W>(t, st);
