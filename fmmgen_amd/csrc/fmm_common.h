@@ -171,6 +171,7 @@ struct Tree {
   // interaction lists (example/tree.hpp:87-88), multiset-equal to the
   // reference; CSR by target cell.
   long long n_m2l = 0, n_p2p = 0;
+  int m2l_maxq = 0;               // largest M2L centre offset per axis, in finer half-widths
   DevBuf<int> m2l_off, m2l_src;   // [ncells+1], [n_m2l]
   DevBuf<int> p2p_off, p2p_src;   // [ncells+1], [n_p2p]
   // P2P sources of each target leaf as merged particle ranges (the target

@@ -29,9 +29,16 @@ namespace {
 
 inline int blocks(long long n, int bs) { return (int)((n + bs - 1) / bs); }
 
-__global__ void k_has_m2l(int b, int e, const int* __restrict__ off, int* __restrict__ flag) {
-  const int c = b + blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < e) flag[c - b] = off[c + 1] > off[c] ? 1 : 0;
+struct HasM2L {  // cells with M2L sources
+  const int* off;
+  __host__ __device__ int operator()(int c) const { return off[c + 1] > off[c] ? 1 : 0; }
+};
+
+// cnt[l] = cells with M2L sources before level l (rank: their exclusive scan)
+__global__ void k_level_ranks(int depth, const int* __restrict__ level_off, const int* __restrict__ rank,
+                              int* __restrict__ cnt) {
+  const int l = blockIdx.x * blockDim.x + threadIdx.x;
+  if (l <= depth) cnt[l] = rank[level_off[l]];
 }
 
 // Tile order of a level's targets: (octant, parent octant) class first,
@@ -41,36 +48,42 @@ __global__ void k_has_m2l(int b, int e, const int* __restrict__ off, int* __rest
 // With a per-cell order hint (the learned order the cell is predicted to
 // run at), cells of one class are further ordered by hint, so that a tile
 // (which runs at the largest order of its cells) holds cells of one order.
-__global__ void k_tile_keys(int b, int e, const int* __restrict__ off, const int* __restrict__ octant,
-                            const int* __restrict__ parent, const int* __restrict__ hint,
-                            unsigned long long* __restrict__ key, int* __restrict__ cell) {
-  const int c = b + blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= e) return;
+__global__ void k_tile_keys(int nc, const int* __restrict__ off, const int* __restrict__ level,
+                            const int* __restrict__ octant, const int* __restrict__ parent,
+                            const int* __restrict__ hint, unsigned long long* __restrict__ key) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= nc) return;
   const bool has = off[c + 1] > off[c];
   const unsigned cls = (unsigned)(octant[c] * 8 + octant[parent[c]]);
   const unsigned h = hint ? (unsigned)min(max(hint[c], 0), 15) : 0u;
-  key[c - b] = has ? (((unsigned long long)cls << 36) | ((unsigned long long)h << 32) | (unsigned)c) : ~0ULL;
-  cell[c - b] = c;
+  key[c] = has ? (((unsigned long long)level[c] << 42) | ((unsigned long long)cls << 36) |
+                  ((unsigned long long)h << 32) | (unsigned)c)
+               : (31ull << 42);
 }
 
-__global__ void k_assign_tiles(int cnt, const int* __restrict__ cell_sorted, int tile_base,
-                               int* __restrict__ tile_of, int* __restrict__ col_of, int* __restrict__ tile_cells) {
+// Tiles of 16 in key order, starting anew on every level: level l holds sorted
+// entries from cnt[l] and tiles from base[l].
+__global__ void k_assign_tiles(int total, const unsigned long long* __restrict__ key_sorted,
+                               const int* __restrict__ cnt, const int* __restrict__ base, int* __restrict__ tile_of,
+                               int* __restrict__ col_of, int* __restrict__ tile_cells) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= cnt) return;
-  const int c = cell_sorted[i];
-  const int t = tile_base + i / kTile, col = i % kTile;
+  if (i >= total) return;
+  const unsigned long long k = key_sorted[i];
+  const int c = (int)(k & 0xffffffffu), l = (int)(k >> 42);
+  const int j = i - cnt[l], t = base[l] + j / kTile, col = j % kTile;
   tile_of[c] = t;
   col_of[c] = col;
   tile_cells[t * kTile + col] = c;
 }
 
-// Per pair: key (target level, source level, quantised offset) and the
-// pair's tile.  Offsets are integer multiples of the finer half-width.
+// Per pair: key (target level, source level, quantised offset per axis, lb and
+// qb bits a field) and the pair's target.  Offsets are integer multiples of the
+// finer half-width, at most half in size; half < 2^(qb - 1).
 __global__ void k_pair_key(long long m, const int* __restrict__ off, const int* __restrict__ src, int ncells,
                            const int* __restrict__ level, const double* __restrict__ cx,
                            const double* __restrict__ cy, const double* __restrict__ cz,
-                           const double* __restrict__ cr, unsigned long long* __restrict__ key,
-                           int* __restrict__ tgt, int* __restrict__ bad) {
+                           const double* __restrict__ cr, int lb, int qb, int half,
+                           unsigned long long* __restrict__ key, int* __restrict__ tgt) {
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (i >= m) return;
   // target of entry i by binary search in the CSR offsets
@@ -82,24 +95,21 @@ __global__ void k_pair_key(long long m, const int* __restrict__ off, const int* 
   const int A = lo, B = src[i];
   tgt[i] = A;
   const double rf = fmin(cr[A], cr[B]);
-  const long long qx = llrint((cx[A] - cx[B]) / rf);
-  const long long qy = llrint((cy[A] - cy[B]) / rf);
-  const long long qz = llrint((cz[A] - cz[B]) / rf);
-  const long long lim = 1LL << 17;
-  if (qx <= -lim || qx >= lim || qy <= -lim || qy >= lim || qz <= -lim || qz >= lim) atomicOr(bad, 1);
-  key[i] = ((unsigned long long)(level[A] & 31) << 59) | ((unsigned long long)(level[B] & 31) << 54) |
-           ((unsigned long long)((qx + lim) & 0x3ffff) << 36) | ((unsigned long long)((qy + lim) & 0x3ffff) << 18) |
-           (unsigned long long)((qz + lim) & 0x3ffff);
+  const unsigned long long qx = (unsigned long long)(llrint((cx[A] - cx[B]) / rf) + half);
+  const unsigned long long qy = (unsigned long long)(llrint((cy[A] - cy[B]) / rf) + half);
+  const unsigned long long qz = (unsigned long long)(llrint((cz[A] - cz[B]) / rf) + half);
+  unsigned long long k = (unsigned long long)level[A];
+  k = (k << lb) | (unsigned)level[B];
+  k = (k << qb) | qx;
+  k = (k << qb) | qy;
+  key[i] = (k << qb) | qz;
 }
 
-__global__ void k_iota_ll(long long m, int* __restrict__ v) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i < m) v[i] = (int)i;
-}
-
+// flag[m] = 0: the scan's last entry is the number of runs
 __global__ void k_run_flags64(long long m, const unsigned long long* __restrict__ k, int* __restrict__ flag) {
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i < m) flag[i] = (i == 0 || k[i] != k[i - 1]) ? 1 : 0;
+  if (i > m) return;
+  flag[i] = i < m && (i == 0 || k[i] != k[i - 1]) ? 1 : 0;
 }
 
 // Key ids in pair order and one representative pair per key.
@@ -124,13 +134,15 @@ __global__ void k_key_ids(long long m, const int* __restrict__ flag, const int* 
   }
 }
 
-__global__ void k_group_keys(long long m, const int* __restrict__ tgt, const int* __restrict__ keyid,
+__global__ void k_group_keys(long long m, int kb, const int* __restrict__ tgt, const int* __restrict__ keyid,
                              const int* __restrict__ tile_of, unsigned long long* __restrict__ comp) {
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i < m) comp[i] = ((unsigned long long)(unsigned)tile_of[tgt[i]] << 32) | (unsigned)keyid[i];
+  if (i < m) comp[i] = ((unsigned long long)(unsigned)tile_of[tgt[i]] << kb) | (unsigned)keyid[i];
 }
 
-__global__ void k_fill_groups(long long m, const unsigned long long* __restrict__ comp,
+// Groups and the first group of every tile (every tile has one: its cells all
+// have M2L sources); tile_first[ntiles] = the number of groups.
+__global__ void k_fill_groups(long long m, int kb, int ntiles, const unsigned long long* __restrict__ comp,
                               const int* __restrict__ order, const int* __restrict__ flag,
                               const int* __restrict__ pos, const int* __restrict__ tgt,
                               const int* __restrict__ src, const int* __restrict__ col_of,
@@ -142,20 +154,32 @@ __global__ void k_fill_groups(long long m, const unsigned long long* __restrict_
   const int i = order[j];
   const unsigned long long c = comp[j];
   if (flag[j]) {
-    group_key[g] = (int)(c & 0xffffffffu);
-    const int t = (int)(c >> 32);
-    if (j == 0 || (int)(comp[j - 1] >> 32) != t) tile_first[t] = g;
+    group_key[g] = (int)(c & ((1ull << kb) - 1));
+    const int t = (int)(c >> kb);
+    if (j == 0 || (int)(comp[j - 1] >> kb) != t) tile_first[t] = g;
   }
+  if (j == m - 1) tile_first[ntiles] = g + 1;
   group_src[(long long)g * kTile + col_of[tgt[i]]] = src[i];
 }
 
-__global__ void k_close_offsets(int n, int* __restrict__ off, int total) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  int next = total;
-  off[n] = total;
-  for (int c = n - 1; c >= 0; --c) {
-    if (off[c] < 0) off[c] = next;
-    else next = off[c];
+// Work items of a tile: its groups cut into equal runs of at most
+// kGroupsPerChunk; nch[ntiles] = 0, so that the scan's last entry is their
+// number.
+__global__ void k_chunk_count(int ntiles, const int* __restrict__ goff, int* __restrict__ nch) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t <= ntiles) nch[t] = t < ntiles ? (goff[t + 1] - goff[t] + kGroupsPerChunk - 1) / kGroupsPerChunk : 0;
+}
+__global__ void k_chunk_fill(int ntiles, const int* __restrict__ goff, const int* __restrict__ nch,
+                             const int* __restrict__ first, int* __restrict__ tile, int* __restrict__ g0,
+                             int* __restrict__ g1) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= ntiles) return;
+  const int G = goff[t + 1] - goff[t], n = nch[t];
+  for (int k = 0; k < n; ++k) {
+    const int c = first[t] + k;
+    tile[c] = t;
+    g0[c] = goff[t] + (int)((long long)G * k / n);
+    g1[c] = goff[t] + (int)((long long)G * (k + 1) / n);
   }
 }
 
@@ -174,6 +198,22 @@ int read_int(const int* d, hipStream_t st) {
   return h;
 }
 
+int bits_for(unsigned long long v) {  // bits that hold 0 .. v
+  int b = 1;
+  while (v >>= 1) ++b;
+  return b;
+}
+
+// Pair indices in the order of their keys (stable), low `bits` bits.
+void sort_order(Tree& t, const unsigned long long* key, unsigned long long* key_sorted, int* order, long long m,
+                int bits, hipStream_t st) {
+  const rocprim::counting_iterator<int> iota(0);
+  size_t bytes = 0;
+  FMM_HIP(rocprim::radix_sort_pairs(nullptr, bytes, key, key_sorted, iota, order, (size_t)m, 0, bits, st));
+  void* tmp = t.scratch.get(bytes);
+  FMM_HIP(rocprim::radix_sort_pairs(tmp, bytes, key, key_sorted, iota, order, (size_t)m, 0, bits, st));
+}
+
 }  // namespace
 
 void build_m2l_schedule(Tree& t, hipStream_t st) {
@@ -182,79 +222,68 @@ void build_m2l_schedule(Tree& t, hipStream_t st) {
   S.cell_tile_ready = false;
   const int nc = t.ncells;
   const long long m = t.n_m2l;
-  // tiles, one level at a time
-  DevBuf<int> tile_of, col_of, flag, rank;
+  FMM_CHECK(m < (1LL << 31), kOutOfMemory, "more than 2^31 M2L pairs");
+  // tiles of every level
+  DevBuf<int> tile_of, col_of, rank, lvl;
   tile_of.alloc(nc);
   col_of.alloc(nc);
-  std::vector<int> tiles_per_level(t.depth), tile_base(t.depth + 1, 0);
   {
-    DevBuf<int> fl, rk;
-    for (int l = 0; l < t.depth; ++l) {
-      const int b = t.level_off[l], e = t.level_off[l + 1], k = e - b;
-      fl.alloc(k + 1);
-      rk.alloc(k + 1);
-      k_has_m2l<<<blocks(k, 256), 256, 0, st>>>(b, e, t.m2l_off.get(), fl.get());
-      scan_ex(t.scratch, fl.get(), rk.get(), k, st);
-      const int cnt = read_int(rk.get() + k - 1, st) + read_int(fl.get() + k - 1, st);
-      tiles_per_level[l] = (cnt + kTile - 1) / kTile;
-      tile_base[l + 1] = tile_base[l] + tiles_per_level[l];
-    }
-    S.ntiles = tile_base[t.depth];
-    S.tile_cells.alloc((size_t)std::max(S.ntiles, 1) * kTile);
-    FMM_HIP(hipMemsetAsync(S.tile_cells.get(), 0xff, sizeof(int) * std::max(S.ntiles, 1) * kTile, st));
-    DevBuf<unsigned long long> k0, k1;
-    DevBuf<int> c0, c1;
-    for (int l = 0; l < t.depth; ++l) {
-      const int b = t.level_off[l], e = t.level_off[l + 1], k = e - b;
-      const int cnt = tiles_per_level[l] == 0 ? 0 : -1;
-      if (cnt == 0) continue;
-      k0.alloc(k); k1.alloc(k); c0.alloc(k); c1.alloc(k);
-      fl.alloc(k + 1);
-      rk.alloc(k + 1);
-      k_has_m2l<<<blocks(k, 256), 256, 0, st>>>(b, e, t.m2l_off.get(), fl.get());
-      scan_ex(t.scratch, fl.get(), rk.get(), k, st);
-      const int ncnt = read_int(rk.get() + k - 1, st) + read_int(fl.get() + k - 1, st);
-      k_tile_keys<<<blocks(k, 256), 256, 0, st>>>(b, e, t.m2l_off.get(), t.octant.get(), t.parent.get(),
-                                                  t.tile_hint_ptr(), k0.get(), c0.get());
-      size_t bytes = 0;
-      FMM_HIP(rocprim::radix_sort_pairs(nullptr, bytes, k0.get(), k1.get(), c0.get(), c1.get(), (size_t)k, 0, 64, st));
-      void* tmp = t.scratch.get(bytes);
-      FMM_HIP(rocprim::radix_sort_pairs(tmp, bytes, k0.get(), k1.get(), c0.get(), c1.get(), (size_t)k, 0, 64, st));
-      k_assign_tiles<<<blocks(ncnt, 256), 256, 0, st>>>(ncnt, c1.get(), tile_base[l], tile_of.get(), col_of.get(),
-                                                        S.tile_cells.get());
-      FMM_HIP(hipStreamSynchronize(st));
-    }
-  }
-  S.tile_group_off.alloc(S.ntiles + 1);
-  if (m == 0) {
-    S.ngroups = 0;
-    S.nkeys = 0;
-    FMM_HIP(hipMemsetAsync(S.tile_group_off.get(), 0, sizeof(int) * (S.ntiles + 1), st));
-    FMM_HIP(hipStreamSynchronize(st));
-    return;
-  }
-  FMM_CHECK(m < (1LL << 31), kOutOfMemory, "more than 2^31 M2L pairs");
-  DevBuf<unsigned long long> key, key_sorted;
-  DevBuf<int> tgt, order0, order, fl, pos, keyid, bad;
-  key.alloc(m); key_sorted.alloc(m); tgt.alloc(m); order0.alloc(m); order.alloc(m);
-  fl.alloc(m); pos.alloc(m); keyid.alloc(m); bad.alloc(1);
-  FMM_HIP(hipMemsetAsync(bad.get(), 0, sizeof(int), st));
-  k_pair_key<<<blocks(m, 256), 256, 0, st>>>(m, t.m2l_off.get(), t.m2l_src.get(), nc, t.level.get(), t.cx.get(),
-                                             t.cy.get(), t.cz.get(), t.cr.get(), key.get(), tgt.get(), bad.get());
-  FMM_CHECK(read_int(bad.get(), st) == 0, kUnsupported, "M2L offset beyond 2^17 half-widths (tree too deep)");
-  // distinct keys
-  k_iota_ll<<<blocks(m, 256), 256, 0, st>>>(m, order0.get());
-  {
+    const int D = t.depth;
+    rank.alloc(nc + 1);
+    lvl.alloc(3 * (D + 1));  // level offsets; ranks and first tiles of the levels
+    int* const lcnt = lvl.get() + (D + 1);
+    int* const lbase = lcnt + (D + 1);
+    FMM_HIP(hipMemcpyAsync(lvl.get(), t.level_off.data(), sizeof(int) * (D + 1), hipMemcpyHostToDevice, st));
+    auto has = rocprim::make_transform_iterator(rocprim::counting_iterator<int>(0), HasM2L{t.m2l_off.get()});
     size_t bytes = 0;
-    FMM_HIP(rocprim::radix_sort_pairs(nullptr, bytes, key.get(), key_sorted.get(), order0.get(), order.get(),
-                                      (size_t)m, 0, 64, st));
+    FMM_HIP(rocprim::inclusive_scan(nullptr, bytes, has, rank.get() + 1, (size_t)nc, rocprim::plus<int>(), st));
     void* tmp = t.scratch.get(bytes);
-    FMM_HIP(rocprim::radix_sort_pairs(tmp, bytes, key.get(), key_sorted.get(), order0.get(), order.get(),
-                                      (size_t)m, 0, 64, st));
+    FMM_HIP(rocprim::inclusive_scan(tmp, bytes, has, rank.get() + 1, (size_t)nc, rocprim::plus<int>(), st));
+    FMM_HIP(hipMemsetAsync(rank.get(), 0, sizeof(int), st));
+    k_level_ranks<<<1, 64, 0, st>>>(D, lvl.get(), rank.get(), lcnt);
+    std::vector<int> cnt(D + 1), base(D + 1, 0);
+    FMM_HIP(hipMemcpyAsync(cnt.data(), lcnt, sizeof(int) * (D + 1), hipMemcpyDeviceToHost, st));
+    FMM_HIP(hipStreamSynchronize(st));
+    for (int l = 0; l < D; ++l) base[l + 1] = base[l] + (cnt[l + 1] - cnt[l] + kTile - 1) / kTile;
+    S.ntiles = base[D];
+    S.tile_cells.alloc((size_t)std::max(S.ntiles, 1) * kTile);
+    S.tile_group_off.alloc(S.ntiles + 1);
+    if (m == 0) {
+      S.ngroups = S.nkeys = S.nchunks = 0;
+      FMM_HIP(hipMemsetAsync(S.tile_group_off.get(), 0, sizeof(int) * (S.ntiles + 1), st));
+      FMM_HIP(hipStreamSynchronize(st));
+      return;
+    }
+    FMM_HIP(hipMemsetAsync(S.tile_cells.get(), 0xff, sizeof(int) * S.ntiles * kTile, st));
+    FMM_HIP(hipMemcpyAsync(lbase, base.data(), sizeof(int) * (D + 1), hipMemcpyHostToDevice, st));
+    DevBuf<unsigned long long> k0, k1;
+    k0.alloc(nc);
+    k1.alloc(nc);
+    k_tile_keys<<<blocks(nc, 256), 256, 0, st>>>(nc, t.m2l_off.get(), t.level.get(), t.octant.get(), t.parent.get(),
+                                                 t.tile_hint_ptr(), k0.get());
+    FMM_HIP(rocprim::radix_sort_keys(nullptr, bytes, k0.get(), k1.get(), (size_t)nc, 0, 47, st));
+    tmp = t.scratch.get(bytes);
+    FMM_HIP(rocprim::radix_sort_keys(tmp, bytes, k0.get(), k1.get(), (size_t)nc, 0, 47, st));
+    k_assign_tiles<<<blocks(cnt[D], 256), 256, 0, st>>>(cnt[D], k1.get(), lcnt, lbase, tile_of.get(), col_of.get(),
+                                                        S.tile_cells.get());
+    FMM_HIP(hipStreamSynchronize(st));  // base, k0 and k1 end here
   }
-  k_run_flags64<<<blocks(m, 256), 256, 0, st>>>(m, key_sorted.get(), fl.get());
-  scan_ex(t.scratch, fl.get(), pos.get(), m, st);
-  S.nkeys = read_int(pos.get() + m - 1, st) + read_int(fl.get() + m - 1, st);
+  DevBuf<unsigned long long> key, key_sorted;
+  DevBuf<int> tgt, order, fl, pos, keyid;
+  key.alloc(m); key_sorted.alloc(m); tgt.alloc(m); order.alloc(m);
+  fl.alloc(m + 1); pos.alloc(m + 1); keyid.alloc(m);
+  // fields as wide as the largest offset needs: every 8 bits less are a pass
+  // less of the sort over all pairs
+  FMM_CHECK(t.m2l_maxq < (1 << 17), kUnsupported, "M2L offset beyond 2^17 half-widths (tree too deep)");
+  const int qb = bits_for((unsigned long long)t.m2l_maxq) + 1, lb = bits_for((unsigned long long)t.depth);
+  k_pair_key<<<blocks(m, 256), 256, 0, st>>>(m, t.m2l_off.get(), t.m2l_src.get(), nc, t.level.get(), t.cx.get(),
+                                             t.cy.get(), t.cz.get(), t.cr.get(), lb, qb, t.m2l_maxq, key.get(),
+                                             tgt.get());
+  // distinct keys
+  sort_order(t, key.get(), key_sorted.get(), order.get(), m, 2 * lb + 3 * qb, st);
+  k_run_flags64<<<blocks(m + 1, 256), 256, 0, st>>>(m, key_sorted.get(), fl.get());
+  scan_ex(t.scratch, fl.get(), pos.get(), m + 1, st);
+  S.nkeys = read_int(pos.get() + m, st);
   S.key_dx.alloc(3 * (size_t)S.nkeys);
   S.key_r.alloc(S.nkeys);
   S.key_dlevel.alloc(S.nkeys);
@@ -262,49 +291,31 @@ void build_m2l_schedule(Tree& t, hipStream_t st) {
                                             t.level.get(), t.cx.get(), t.cy.get(), t.cz.get(), t.cr.get(),
                                             keyid.get(), S.key_dx.get(), S.key_r.get(), S.key_dlevel.get());
   // groups = runs of (tile, key)
-  k_group_keys<<<blocks(m, 256), 256, 0, st>>>(m, tgt.get(), keyid.get(), tile_of.get(), key.get());
-  k_iota_ll<<<blocks(m, 256), 256, 0, st>>>(m, order0.get());
-  {
-    size_t bytes = 0;
-    FMM_HIP(rocprim::radix_sort_pairs(nullptr, bytes, key.get(), key_sorted.get(), order0.get(), order.get(),
-                                      (size_t)m, 0, 64, st));
-    void* tmp = t.scratch.get(bytes);
-    FMM_HIP(rocprim::radix_sort_pairs(tmp, bytes, key.get(), key_sorted.get(), order0.get(), order.get(),
-                                      (size_t)m, 0, 64, st));
-  }
-  k_run_flags64<<<blocks(m, 256), 256, 0, st>>>(m, key_sorted.get(), fl.get());
-  scan_ex(t.scratch, fl.get(), pos.get(), m, st);
-  S.ngroups = read_int(pos.get() + m - 1, st) + read_int(fl.get() + m - 1, st);
+  const int kb = bits_for((unsigned long long)S.nkeys - 1);
+  k_group_keys<<<blocks(m, 256), 256, 0, st>>>(m, kb, tgt.get(), keyid.get(), tile_of.get(), key.get());
+  sort_order(t, key.get(), key_sorted.get(), order.get(), m, kb + bits_for((unsigned long long)S.ntiles - 1), st);
+  k_run_flags64<<<blocks(m + 1, 256), 256, 0, st>>>(m, key_sorted.get(), fl.get());
+  scan_ex(t.scratch, fl.get(), pos.get(), m + 1, st);
+  S.ngroups = read_int(pos.get() + m, st);
   S.group_key.alloc(S.ngroups);
   S.group_src.alloc((size_t)S.ngroups * kTile);
   FMM_HIP(hipMemsetAsync(S.group_src.get(), 0xff, sizeof(int) * (size_t)S.ngroups * kTile, st));
-  FMM_HIP(hipMemsetAsync(S.tile_group_off.get(), 0xff, sizeof(int) * (S.ntiles + 1), st));
-  k_fill_groups<<<blocks(m, 256), 256, 0, st>>>(m, key_sorted.get(), order.get(), fl.get(), pos.get(), tgt.get(),
-                                                t.m2l_src.get(), col_of.get(), S.group_key.get(), S.group_src.get(),
-                                                S.tile_group_off.get());
-  k_close_offsets<<<1, 1, 0, st>>>(S.ntiles, S.tile_group_off.get(), S.ngroups);
-  FMM_HIP(hipStreamSynchronize(st));
+  k_fill_groups<<<blocks(m, 256), 256, 0, st>>>(m, kb, S.ntiles, key_sorted.get(), order.get(), fl.get(), pos.get(),
+                                                tgt.get(), t.m2l_src.get(), col_of.get(), S.group_key.get(),
+                                                S.group_src.get(), S.tile_group_off.get());
   // work items: runs of groups of one tile
-  std::vector<int> goff(S.ntiles + 1);
-  FMM_HIP(hipMemcpy(goff.data(), S.tile_group_off.get(), sizeof(int) * (S.ntiles + 1), hipMemcpyDeviceToHost));
-  std::vector<int> ct, c0, c1;
-  // a tile's groups cut into equal runs of at most kGroupsPerChunk
-  for (int tl = 0; tl < S.ntiles; ++tl) {
-    const int G = goff[tl + 1] - goff[tl];
-    const int nch = (G + kGroupsPerChunk - 1) / kGroupsPerChunk;
-    for (int k = 0; k < nch; ++k) {
-      ct.push_back(tl);
-      c0.push_back(goff[tl] + (int)((long long)G * k / nch));
-      c1.push_back(goff[tl] + (int)((long long)G * (k + 1) / nch));
-    }
-  }
-  S.nchunks = (int)ct.size();
+  DevBuf<int> nch, first;
+  nch.alloc(S.ntiles + 1);
+  first.alloc(S.ntiles + 1);
+  k_chunk_count<<<blocks(S.ntiles + 1, 256), 256, 0, st>>>(S.ntiles, S.tile_group_off.get(), nch.get());
+  scan_ex(t.scratch, nch.get(), first.get(), S.ntiles + 1, st);
+  S.nchunks = read_int(first.get() + S.ntiles, st);
   S.chunk_tile.alloc(S.nchunks);
   S.chunk_g0.alloc(S.nchunks);
   S.chunk_g1.alloc(S.nchunks);
-  FMM_HIP(hipMemcpy(S.chunk_tile.get(), ct.data(), sizeof(int) * S.nchunks, hipMemcpyHostToDevice));
-  FMM_HIP(hipMemcpy(S.chunk_g0.get(), c0.data(), sizeof(int) * S.nchunks, hipMemcpyHostToDevice));
-  FMM_HIP(hipMemcpy(S.chunk_g1.get(), c1.data(), sizeof(int) * S.nchunks, hipMemcpyHostToDevice));
+  k_chunk_fill<<<blocks(S.ntiles, 256), 256, 0, st>>>(S.ntiles, S.tile_group_off.get(), nch.get(), first.get(),
+                                                      S.chunk_tile.get(), S.chunk_g0.get(), S.chunk_g1.get());
+  FMM_HIP(hipStreamSynchronize(st));
 }
 
 }  // namespace fmm

@@ -3,8 +3,9 @@
 // Reproduces example/tree.cpp:130-233 (build_tree) and
 // example/calculate.cpp:81-133 (interact_dehnen_lazy) bit for bit on the
 // geometry, with a canonical cell numbering:
-//   * root centre = sequential FP64 mean (one lane per axis, in index
-//     order, as example/tree.cpp:145-156 sums), half-width = 1.001 x the
+//   * root centre = the FP64 mean of example/tree.cpp:145-156, whose sum runs
+//     in index order with one rounding per addition (evaluated in parallel,
+//     bit for bit, see k_mean_steps), half-width = 1.001 x the
 //     largest per-axis deviation (order-free max reduction);
 //   * a cell splits iff it holds >= ncrit particles; only non-empty octants
 //     become children; child centre = parent centre +- r/2 by the same FP64
@@ -40,64 +41,250 @@ constexpr int kMaxSplitLevels = 21;  // 3 key bits per level in 63 bits
 
 __device__ __forceinline__ double rmax_of(double r) { return sqrt_rn((3.0 * r) * r); }
 
-// Sequential mean: the block stages chunks of positions through LDS
-// (coalesced loads), lanes 0..2 add them in index order.
-// Mean of the positions with the reference's sequential FP64 sum
-// (lanes 0..2 of wave 0 sum x, y, z in particle order, one rounding per
-// addition, so the root centre is bit-exact).  Waves 1..3 stage the next
-// chunk into the other half of a double buffer while wave 0 sums the
-// current one, reading runs of 16 values before their 16 ordered additions.
-__global__ __launch_bounds__(256) void k_mean(const double* __restrict__ pos, long long n, double* __restrict__ out) {
-  constexpr int kChunk = 1024, kRun = 16;
-  __shared__ double buf[2][3 * kChunk];
-  double s = 0.0;
-  const int tid = threadIdx.x;
-  auto stage = [&](long long base, int half) {  // waves 1..3
-    const int m = (int)(n - base < kChunk ? n - base : kChunk);
-    for (int k = tid - 64; k < 3 * m; k += 192) buf[half][k] = pos[3 * base + k];
-  };
-  if (tid >= 64 && n > 0) stage(0, 0);
+// The mean of the positions with the reference's sequential FP64 sum
+// s <- RN(s + x), bit for bit, without its chain of n dependent additions.
+// While |s| stays inside one binade [2^e, 2^(e+1)) of ulp u, s = u S with S a
+// whole number and RN(s + x) = u (S + d): d = x/u rounded to the nearest whole
+// number, ties by the parity of S.  A run of additions is then a pair of whole
+// numbers (the total of the d for an even and for an odd S before the run), and
+// such pairs compose associatively.  Runs of kMeanChunk additions are summed in
+// any order first, which gives each run's range of s up to the bound E of
+// k_mean_scan; a run whose range lies in one binade is composed in parallel
+// (k_mean_steps), and k_mean_walk applies the pairs in order, 64 at a time,
+// adding one by one only in the runs that may leave their binade (a few of
+// them where s grows steadily).
+// The chain of additions, one lane per axis, took 1936 us at 300007 particles
+// and 27 ms at 2^22; this takes 110 us at 300007 (k_mean_walk 82).
+constexpr int kMeanChunk = 256;  // one wave per axis, 4 additions a lane
+constexpr int kMeanUnsafe = -100000;
+
+struct MeanRun {
+  double sum, lo, hi, abs;  // total, least and greatest partial sum (0 included), sum of |x|
+};
+
+__device__ __forceinline__ void mean_load(const double* __restrict__ pos, long long n, long long c, double* buf,
+                                          int axis, int lane, double (&x)[4]) {
+  const long long base = c * kMeanChunk;
+  const int m = 3 * (int)(n - base < kMeanChunk ? n - base : kMeanChunk);
+  for (int k = threadIdx.x; k < 3 * kMeanChunk; k += 192) buf[k] = k < m ? pos[3 * base + k] : 0.0;
   __syncthreads();
-  int half = 0;
-  for (long long base = 0; base < n; base += kChunk, half ^= 1) {
-    if (tid >= 64 && base + kChunk < n) stage(base + kChunk, half ^ 1);
-    if (tid < 3) {
-      const int m = (int)(n - base < kChunk ? n - base : kChunk);
-      const double* b = buf[half] + tid;
-      int i = 0;
-      for (; i + kRun <= m; i += kRun) {
-        double v[kRun];
 #pragma unroll
-        for (int u = 0; u < kRun; ++u) v[u] = b[3 * (i + u)];
-#pragma unroll
-        for (int u = 0; u < kRun; ++u) s = s + v[u];
-      }
-      for (; i < m; ++i) s = s + b[3 * i];
-    }
-    __syncthreads();  // this half consumed, the next one staged
-  }
-  if (tid < 3) out[tid] = s / (double)n;
+  for (int k = 0; k < 4; ++k) x[k] = buf[3 * (4 * lane + k) + axis];
 }
 
-__global__ void k_maxdev(const double* __restrict__ pos, long long n, const double* __restrict__ mean,
-                         unsigned long long* __restrict__ mx) {
+__global__ __launch_bounds__(192) void k_mean_sums(const double* __restrict__ pos, long long n, long long nrun,
+                                                   MeanRun* __restrict__ out) {
+  __shared__ double buf[3 * kMeanChunk];
+  const int lane = threadIdx.x & 63, axis = threadIdx.x >> 6;
+  double x[4];
+  mean_load(pos, n, blockIdx.x, buf, axis, lane, x);
+  double sum = (x[0] + x[1]) + (x[2] + x[3]), inc = sum;
+  double ab = (fabs(x[0]) + fabs(x[1])) + (fabs(x[2]) + fabs(x[3]));
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double v = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += v;
+  }
+  double p = inc - sum, lo = fmin(p, 0.0), hi = fmax(p, 0.0);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    p += x[k];
+    lo = fmin(lo, p);
+    hi = fmax(hi, p);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, o, 64));
+    hi = fmax(hi, __shfl_xor(hi, o, 64));
+    ab += __shfl_xor(ab, o, 64);
+  }
+  const double tot = __shfl(inc, 63, 64);
+  // NaN and infinite sums pass through `sum` and make every later run unsafe
+  if (lane == 0) out[axis * nrun + blockIdx.x] = MeanRun{tot, lo, hi, ab};
+}
+
+// Binade of every run's partial sums, or kMeanUnsafe (one block per axis).
+// E bounds the distance of the sequential sum from the sums computed here:
+// n additions each rounded by at most 2^-53 of the largest partial sum, and
+// this kernel's and k_mean_sums' own additions (a few hundred levels deep for
+// the serial parts) by 2^-53 of the sum of |x| each.
+__global__ __launch_bounds__(1024) void k_mean_scan(long long n, long long nrun, const MeanRun* __restrict__ run,
+                                                    int* __restrict__ expo) {
+  __shared__ double sh[3][1024];
+  const int tid = threadIdx.x;
+  const MeanRun* r = run + blockIdx.x * nrun;
+  const long long per = (nrun + 1023) / 1024, b = min(tid * per, nrun), e = min(b + per, nrun);
+  double sum = 0.0, ab = 0.0;
+  for (long long i = b; i < e; ++i) {
+    sum += r[i].sum;
+    ab += r[i].abs;
+  }
+  sh[0][tid] = sum;
+  sh[1][tid] = ab;
+  __syncthreads();
+  for (int o = 1; o < 1024; o <<= 1) {  // inclusive scans
+    const double v = tid >= o ? sh[0][tid - o] : 0.0, w = tid >= o ? sh[1][tid - o] : 0.0;
+    __syncthreads();
+    sh[0][tid] += v;
+    sh[1][tid] += w;
+    __syncthreads();
+  }
+  const double start = tid > 0 ? sh[0][tid - 1] : 0.0, xabs = sh[1][1023];
+  double a = start, big = 0.0;
+  for (long long i = b; i < e; ++i) {
+    big = fmax(big, fmax(fabs(a + r[i].lo), fabs(a + r[i].hi)));
+    a += r[i].sum;
+  }
+  sh[2][tid] = big;
+  __syncthreads();
+  for (int s = 512; s > 0; s >>= 1) {
+    if (tid < s) sh[2][tid] = fmax(sh[2][tid], sh[2][tid + s]);
+    __syncthreads();
+  }
+  const double E = 0x1p-52 * ((double)n * sh[2][0] + (double)(per + 64) * xabs);
+  a = start;
+  for (long long i = b; i < e; ++i) {
+    double lo = a + r[i].lo - E, hi = a + r[i].hi + E;
+    a += r[i].sum;
+    if (hi < 0.0) {
+      const double t = -lo;
+      lo = -hi;
+      hi = t;
+    }
+    int ex = kMeanUnsafe;
+    if (lo > 0x1p-900 && hi < 0x1p900) {  // false for NaN
+      const int l = ilogb(lo);
+      if (hi < ldexp(1.0, l + 1)) ex = l;
+    }
+    expo[blockIdx.x * nrun + i] = ex;
+  }
+}
+
+struct MeanStep {
+  long long d[2];  // change of S by the parity of S before
+};
+__device__ __forceinline__ MeanStep mean_then(const MeanStep& a, const MeanStep& b) {
+  return MeanStep{{a.d[0] + ((a.d[0] & 1) ? b.d[1] : b.d[0]), a.d[1] + ((a.d[1] & 1) ? b.d[0] : b.d[1])}};
+}
+__device__ __forceinline__ MeanStep mean_reduce(MeanStep s) {  // lane 0: the lanes' steps in order
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) s = mean_then(s, MeanStep{{__shfl_down(s.d[0], o, 64), __shfl_down(s.d[1], o, 64)}});
+  return s;
+}
+
+__global__ __launch_bounds__(192) void k_mean_steps(const double* __restrict__ pos, long long n, long long nrun,
+                                                    const int* __restrict__ expo, MeanStep* __restrict__ step) {
+  __shared__ double buf[3 * kMeanChunk];
+  const int lane = threadIdx.x & 63, axis = threadIdx.x >> 6;
+  double x[4];
+  mean_load(pos, n, blockIdx.x, buf, axis, lane, x);
+  const int e = expo[axis * nrun + blockIdx.x];
+  if (e == kMeanUnsafe) return;  // uniform over the wave
+  MeanStep s{{0, 0}};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const double y = ldexp(x[k], 52 - e), f = floor(y), r = y - f;  // exact: |x| < 2^(e + 2)
+    const long long i = (long long)f;
+    MeanStep t;
+    t.d[0] = i + (r > 0.5 || (r == 0.5 && (i & 1)) ? 1 : 0);
+    t.d[1] = i + (r > 0.5 || (r == 0.5 && !(i & 1)) ? 1 : 0);
+    s = mean_then(s, t);
+  }
+  s = mean_reduce(s);
+  if (lane == 0) step[axis * nrun + blockIdx.x] = s;
+}
+
+__global__ __launch_bounds__(64) void k_mean_walk(const double* __restrict__ pos, long long n, long long nrun,
+                                                  const int* __restrict__ expo, const MeanStep* __restrict__ step,
+                                                  double* __restrict__ out) {
+  __shared__ double buf[kMeanChunk];
+  const int lane = threadIdx.x, axis = blockIdx.x;
+  expo += axis * nrun;
+  step += axis * nrun;
+  double s = 0.0;
+  // runs past the last one change nothing; unsafe runs have no step
+  auto get = [&](long long base, int& e, MeanStep& m) {
+    const long long i = base + lane;
+    e = i < nrun ? expo[i] : kMeanUnsafe;
+    m = i < nrun && e != kMeanUnsafe ? step[i] : MeanStep{{0, 0}};
+  };
+  auto apply = [&](int e, long long d0, long long d1) {
+    const long long S = (long long)ldexp(s, 52 - e);
+    s = ldexp((double)(S + ((S & 1) ? d1 : d0)), e - 52);
+  };
+  int e, en;
+  MeanStep m, mn;
+  get(0, e, m);
+  for (long long base = 0; base < nrun; base += 64) {
+    if (base + 64 < nrun) get(base + 64, en, mn);  // in flight during this batch
+    const int e0 = __builtin_amdgcn_readfirstlane(e);
+    const int cnt = (int)(nrun - base < 64 ? nrun - base : 64);
+    if (__all(e0 != kMeanUnsafe && (e == e0 || lane >= cnt))) {
+      const MeanStep t = mean_reduce(m);
+      apply(e0, __shfl(t.d[0], 0, 64), __shfl(t.d[1], 0, 64));
+    } else {
+      for (int l = 0; l < cnt; ++l) {
+        const int el = __shfl(e, l, 64);
+        if (el != kMeanUnsafe) {
+          apply(el, __shfl(m.d[0], l, 64), __shfl(m.d[1], l, 64));
+          continue;
+        }
+        const long long first = (base + l) * kMeanChunk;
+        const int k = (int)(n - first < kMeanChunk ? n - first : kMeanChunk);
+        __syncthreads();
+        for (int i = lane; i < k; i += 64) buf[i] = pos[3 * (first + i) + axis];
+        __syncthreads();
+        int i = 0;
+        for (; i + 16 <= k; i += 16) {
+          double v[16];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) v[u] = buf[i + u];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) s = s + v[u];
+        }
+        for (; i < k; ++i) s = s + buf[i];
+      }
+    }
+    e = en;
+    m = mn;
+  }
+  if (lane == 0) out[axis] = s / (double)n;
+}
+
+__global__ __launch_bounds__(256) void k_maxdev(const double* __restrict__ pos, long long n,
+                                                const double* __restrict__ mean,
+                                                unsigned long long* __restrict__ mx) {
+  __shared__ double red[3][4];
   const double m0 = mean[0], m1 = mean[1], m2 = mean[2];
-  double a0 = 0, a1 = 0, a2 = 0;
+  double a[3] = {0, 0, 0};
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {
     const double x = fabs(pos[3 * i] - m0), y = fabs(pos[3 * i + 1] - m1), z = fabs(pos[3 * i + 2] - m2);
-    a0 = x > a0 ? x : a0;
-    a1 = y > a1 ? y : a1;
-    a2 = z > a2 ? z : a2;
+    a[0] = x > a[0] ? x : a[0];
+    a[1] = y > a[1] ? y : a[1];
+    a[2] = z > a[2] ? z : a[2];
   }
-  // non-negative doubles order like their bit patterns
-  atomicMax(&mx[0], (unsigned long long)__double_as_longlong(a0));
-  atomicMax(&mx[1], (unsigned long long)__double_as_longlong(a1));
-  atomicMax(&mx[2], (unsigned long long)__double_as_longlong(a2));
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const double v = __shfl_xor(a[d], o, 64);
+      a[d] = v > a[d] ? v : a[d];
+    }
+    if ((threadIdx.x & 63) == 0) red[d][threadIdx.x >> 6] = a[d];
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {  // non-negative doubles order like their bit patterns
+    const double* r = red[threadIdx.x];
+    double v = r[0];
+    for (int w = 1; w < 4; ++w) v = r[w] > v ? r[w] : v;
+    atomicMax(&mx[threadIdx.x], (unsigned long long)__double_as_longlong(v));
+  }
 }
 
 __global__ void k_root(const double* __restrict__ mean, const unsigned long long* __restrict__ mx,
-                       double* cx, double* cy, double* cz, double* cr, int* count, long long n) {
+                       double* cx, double* cy, double* cz, double* cr, int* count, int* parent, int* octant,
+                       int* ccount, long long n) {
   const double xm = __longlong_as_double((long long)mx[0]);
   const double ym = __longlong_as_double((long long)mx[1]);
   const double zm = __longlong_as_double((long long)mx[2]);
@@ -107,41 +294,71 @@ __global__ void k_root(const double* __restrict__ mean, const unsigned long long
   cz[0] = mean[2];
   cr[0] = r;
   count[0] = (int)n;
+  parent[0] = octant[0] = 0;
+  for (int o = 0; o < 8; ++o) ccount[o] = 0;
 }
 
-// Per particle still inside a split cell: octant histogram of the level.
-// Particles whose cell at this level is a leaf are finalised.
-__global__ void k_level_octants(const double* __restrict__ pos, int n, int* __restrict__ pcell,
-                                unsigned char* __restrict__ poct, int* __restrict__ leaf_of,
-                                const double* __restrict__ lcx, const double* __restrict__ lcy,
-                                const double* __restrict__ lcz, const int* __restrict__ lcount,
-                                int* __restrict__ ccount, int ncrit, int level_base) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int c = pcell[i];
-  if (c < 0) return;
-  if (lcount[c] < ncrit) {
-    leaf_of[i] = level_base + c;
-    pcell[i] = -1;
-    return;
+// Moves every particle that is still inside a split cell to its child of the
+// level (`cidx`: the previous level's numbering by (cell, octant), unused at
+// the root), then finalises the particles whose cell there is a leaf and adds
+// the others to the level's (cell, octant) histogram.  On levels of at most
+// LDS / 8 cells a block counts in LDS first: added straight into memory, the
+// eight counters of the root took all particles' additions (268 us a level on
+// average at 300007 blob particles, 3.1 ms at 2^22; now 35 us at 300007).
+template <int LDS>
+__global__ __launch_bounds__(256) void k_level_octants(const double* __restrict__ pos, int n, int level, int ncell,
+                                                       int* __restrict__ pcell, unsigned char* __restrict__ poct,
+                                                       unsigned long long* __restrict__ key,
+                                                       const int* __restrict__ cidx, int* __restrict__ leaf_of,
+                                                       const double* __restrict__ lcx, const double* __restrict__ lcy,
+                                                       const double* __restrict__ lcz, const int* __restrict__ lcount,
+                                                       int* __restrict__ ccount, int ncrit, int level_base) {
+  __shared__ int hist[LDS > 0 ? LDS : 1];
+  if constexpr (LDS > 0) {
+    for (int j = threadIdx.x; j < 8 * ncell; j += 256) hist[j] = 0;
+    __syncthreads();
   }
-  const int oct = (pos[3 * i] > lcx[c]) + ((pos[3 * i + 1] > lcy[c]) << 1) + ((pos[3 * i + 2] > lcz[c]) << 2);
-  poct[i] = (unsigned char)oct;
-  atomicAdd(&ccount[8 * c + oct], 1);
+  for (long long i = blockIdx.x * 256LL + threadIdx.x; i < n; i += gridDim.x * 256LL) {
+    int c = 0;
+    if (level > 0) {
+      c = pcell[i];
+      if (c < 0) continue;
+      const int o = poct[i];
+      c = cidx[8 * c + o];
+      const unsigned long long bit = (unsigned long long)o << (3 * (kMaxSplitLevels - level));
+      key[i] = level == 1 ? bit : key[i] | bit;
+    }
+    if (lcount[c] < ncrit) {
+      leaf_of[i] = level_base + c;
+      pcell[i] = -1;
+      if (level == 0) key[i] = 0;
+      continue;
+    }
+    const int oct = (pos[3 * i] > lcx[c]) + ((pos[3 * i + 1] > lcy[c]) << 1) + ((pos[3 * i + 2] > lcz[c]) << 2);
+    poct[i] = (unsigned char)oct;
+    pcell[i] = c;
+    if constexpr (LDS > 0) atomicAdd(&hist[8 * c + oct], 1);
+    else atomicAdd(&ccount[8 * (size_t)c + oct], 1);
+  }
+  if constexpr (LDS > 0) {
+    __syncthreads();
+    for (int j = threadIdx.x; j < 8 * ncell; j += 256)
+      if (hist[j] > 0) atomicAdd(&ccount[j], hist[j]);
+  }
 }
 
-__global__ void k_flags(const int* __restrict__ ccount, int* __restrict__ flag, int m) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < m) flag[j] = ccount[j] > 0 ? 1 : 0;
-}
+struct Occupied {  // an octant with particles becomes a child
+  __host__ __device__ int operator()(int count) const { return count > 0 ? 1 : 0; }
+};
 
-// Children of the level, numbered by the scan over (parent, octant) slots.
+// Children of the level, numbered by the scan over (parent, octant) slots;
+// clears their octant counters.
 __global__ void k_make_children(int nparent, const int* __restrict__ ccount, const int* __restrict__ cidx,
                                 const double* __restrict__ lcx, const double* __restrict__ lcy,
                                 const double* __restrict__ lcz, const double* __restrict__ lr,
                                 double* __restrict__ ncx, double* __restrict__ ncy, double* __restrict__ ncz,
                                 double* __restrict__ nr, int* __restrict__ ncount, int* __restrict__ nparent_local,
-                                int* __restrict__ noctant, int* __restrict__ first_child_local,
+                                int* __restrict__ noctant, int* __restrict__ ncc, int* __restrict__ first_child_local,
                                 int* __restrict__ nchild, int* __restrict__ octmask) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= nparent) return;
@@ -162,26 +379,11 @@ __global__ void k_make_children(int nparent, const int* __restrict__ ccount, con
     ncount[id] = k;
     nparent_local[id] = c;
     noctant[id] = o;
+    for (int q = 0; q < 8; ++q) ncc[8 * (size_t)id + q] = 0;
   }
   first_child_local[c] = first;
   nchild[c] = cnt;
   octmask[c] = mask;
-}
-
-__global__ void k_descend(int n, int* __restrict__ pcell, const unsigned char* __restrict__ poct,
-                          const int* __restrict__ cidx, unsigned long long* __restrict__ key, int level) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int c = pcell[i];
-  if (c < 0) return;
-  const int o = poct[i];
-  pcell[i] = cidx[8 * c + o];
-  key[i] |= (unsigned long long)o << (3 * (kMaxSplitLevels - 1 - level));
-}
-
-__global__ void k_iota(int* v, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) v[i] = i;
 }
 
 __global__ void k_gather_particles(int n, const int* __restrict__ perm, const double* __restrict__ pos,
@@ -190,9 +392,9 @@ __global__ void k_gather_particles(int n, const int* __restrict__ perm, const do
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   const int i = perm[j];
-  px[j] = pos[3 * i];
-  py[j] = pos[3 * i + 1];
-  pz[j] = pos[3 * i + 2];
+  px[j] = pos[3 * (size_t)i];
+  py[j] = pos[3 * (size_t)i + 1];
+  pz[j] = pos[3 * (size_t)i + 2];
   leaf_of[j] = leaf_of_orig[i];
 }
 
@@ -202,32 +404,54 @@ __global__ void k_leaf_starts(int n, const int* __restrict__ leaf_of, int* __res
   if (j == 0 || leaf_of[j] != leaf_of[j - 1]) pstart[leaf_of[j]] = j;
 }
 
-__global__ void k_internal_starts(int beg, int end, const int* __restrict__ nchild,
-                                  const int* __restrict__ first_child, int* __restrict__ pstart) {
-  const int c = beg + blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= end) return;
-  if (nchild[c] > 0) pstart[c] = pstart[first_child[c]];
-}
-
-__global__ void k_rmax(int n, const double* __restrict__ r, double* __restrict__ rmax) {
+// An internal cell starts where the leaf at the end of its chain of first
+// children does.
+__global__ void k_internal_starts(int ncells, const int* __restrict__ nchild, const int* __restrict__ first_child,
+                                  int* __restrict__ pstart) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < n) rmax[c] = rmax_of(r[c]);
+  if (c >= ncells || nchild[c] == 0) return;
+  int l = c;
+  while (nchild[l] > 0) l = first_child[l];
+  pstart[c] = pstart[l];
 }
 
-__global__ void k_offset_add(int* v, int n, int add) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && v[i] >= 0) v[i] += add;
-}
-
-__global__ void k_leaf_flags(int n, const int* __restrict__ nchild, int* __restrict__ flag) {
+// One level's cells into the canonical arrays (offset o; parents from po,
+// first children from co, both counted inside their own levels).
+struct CellArrays {
+  double *cx, *cy, *cz, *cr, *crmax;
+  int *pcount, *parent, *first_child, *nchild, *octmask, *octant, *level;
+};
+__global__ void k_place_level(int m, int o, int po, int co, int level, const double* __restrict__ x,
+                              const double* __restrict__ y, const double* __restrict__ z,
+                              const double* __restrict__ r, const int* __restrict__ count,
+                              const int* __restrict__ parent, const int* __restrict__ first_child,
+                              const int* __restrict__ nchild, const int* __restrict__ octmask,
+                              const int* __restrict__ oct, CellArrays out) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < n) flag[c] = nchild[c] == 0 ? 1 : 0;
+  if (c >= m) return;
+  const int k = o + c;
+  out.cx[k] = x[c];
+  out.cy[k] = y[c];
+  out.cz[k] = z[c];
+  out.cr[k] = r[c];
+  out.crmax[k] = rmax_of(r[c]);
+  out.pcount[k] = count[c];
+  out.parent[k] = parent[c] + po;
+  out.first_child[k] = first_child[c] < 0 ? first_child[c] : first_child[c] + co;
+  out.nchild[k] = nchild[c];
+  out.octmask[k] = octmask[c];
+  out.octant[k] = oct[c];
+  out.level[k] = level;
 }
 
-__global__ void k_leaf_compact(int n, const int* __restrict__ flag, const int* __restrict__ pos,
+struct IsLeaf {
+  __host__ __device__ int operator()(int nchild) const { return nchild == 0 ? 1 : 0; }
+};
+
+__global__ void k_leaf_compact(int n, const int* __restrict__ nchild, const int* __restrict__ pos,
                                int* __restrict__ leaves) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < n && flag[c]) leaves[pos[c]] = c;
+  if (c < n && nchild[c] == 0) leaves[pos[c]] = c;
 }
 
 // ---------------------------------------------------------------- lists
@@ -263,85 +487,101 @@ __global__ void k_pair_count(int nf, const int2* __restrict__ fr, Counts3* __res
                              const double* __restrict__ rmax, const int* __restrict__ nchild,
                              const int* __restrict__ pcount, double theta, int ncrit) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf) return;
-  const int2 ab = fr[f];
-  const int d = decide(ab.x, ab.y, cx, cy, cz, rmax, nchild, pcount, theta, ncrit);
-  dec[f] = (unsigned char)d;
+  if (f > nf) return;
   Counts3 c{0, 0, 0};
-  if (d == 0) c.m2l = 1;
-  else if (d == 1) c.p2p = 1;
-  else if (d == 2) c.nxt = nchild[ab.x];
-  else c.nxt = nchild[ab.y];
+  if (f < nf) {  // cnt[nf] = 0: the scan's last entry is the total
+    const int2 ab = fr[f];
+    const int d = decide(ab.x, ab.y, cx, cy, cz, rmax, nchild, pcount, theta, ncrit);
+    dec[f] = (unsigned char)d;
+    if (d == 0) c.m2l = 1;
+    else if (d == 1) c.p2p = 1;
+    else if (d == 2) c.nxt = nchild[ab.x];
+    else c.nxt = nchild[ab.y];
+  }
   cnt[f] = c;
 }
 
-// M2L entries are written as (target, source) like the CSR key; the
-// reference stores (source, target) (example/calculate.cpp:95).
-__global__ void k_pair_emit(int nf, const int2* __restrict__ fr, const Counts3* __restrict__ off,
-                            const unsigned char* __restrict__ dec, const int* __restrict__ first_child,
-                            const int* __restrict__ nchild, int2* __restrict__ m2l, long long m2l_base,
-                            int2* __restrict__ p2p, long long p2p_base, int2* __restrict__ next) {
+// List entries are written as the keys (target << kb) | source that the CSR
+// sort orders; the reference stores M2L as (source, target)
+// (example/calculate.cpp:95).  maxq: the largest M2L centre offset per axis in
+// units of the finer half-width, the field width of the schedule's keys.
+__global__ __launch_bounds__(256) void k_pair_emit(int nf, const int2* __restrict__ fr,
+                                                   const Counts3* __restrict__ off,
+                                                   const unsigned char* __restrict__ dec,
+                                                   const int* __restrict__ first_child,
+                                                   const int* __restrict__ nchild, const double* __restrict__ cx,
+                                                   const double* __restrict__ cy, const double* __restrict__ cz,
+                                                   const double* __restrict__ cr, int kb,
+                                                   unsigned long long* __restrict__ m2l, long long m2l_base,
+                                                   unsigned long long* __restrict__ p2p, long long p2p_base,
+                                                   int2* __restrict__ next, int* __restrict__ maxq) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf) return;
-  const int2 ab = fr[f];
-  const int d = dec[f];
-  const Counts3 o = off[f];
-  if (d == 0) {
-    m2l[m2l_base + o.m2l] = make_int2(ab.x, ab.y);
-  } else if (d == 1) {
-    p2p[p2p_base + o.p2p] = make_int2(ab.x, ab.y);
-  } else if (d == 2) {
-    const int fc = first_child[ab.x], k = nchild[ab.x];
-    for (int i = 0; i < k; ++i) next[o.nxt + i] = make_int2(fc + i, ab.y);
-  } else {
-    const int fc = first_child[ab.y], k = nchild[ab.y];
-    for (int i = 0; i < k; ++i) next[o.nxt + i] = make_int2(ab.x, fc + i);
+  int q = 0;
+  if (f < nf) {
+    const int2 ab = fr[f];
+    const int d = dec[f];
+    const Counts3 o = off[f];
+    const unsigned long long key = ((unsigned long long)(unsigned)ab.x << kb) | (unsigned)ab.y;
+    if (d == 0) {
+      m2l[m2l_base + o.m2l] = key;
+      const double rf = fmin(cr[ab.x], cr[ab.y]);
+      const double m = fmax(fmax(fabs(cx[ab.x] - cx[ab.y]), fabs(cy[ab.x] - cy[ab.y])), fabs(cz[ab.x] - cz[ab.y]));
+      q = (int)fmin(rint(m / rf), 1e9);
+    } else if (d == 1) {
+      p2p[p2p_base + o.p2p] = key;
+    } else if (d == 2) {
+      const int fc = first_child[ab.x], k = nchild[ab.x];
+      for (int i = 0; i < k; ++i) next[o.nxt + i] = make_int2(fc + i, ab.y);
+    } else {
+      const int fc = first_child[ab.y], k = nchild[ab.y];
+      for (int i = 0; i < k; ++i) next[o.nxt + i] = make_int2(ab.x, fc + i);
+    }
+  }
+  __shared__ int red[4];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) q = max(q, __shfl_xor(q, o, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = q;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    q = max(max(red[0], red[1]), max(red[2], red[3]));
+    if (q > *maxq) atomicMax(maxq, q);  // a stale read only costs an atomic
   }
 }
 
-__global__ void k_pair_keys(long long m, const int2* __restrict__ pr, unsigned long long* __restrict__ key) {
+// CSR from the sorted keys: sources, and the offset of every row (each entry
+// sets the rows after its predecessor's up to its own).  With pcount: also the
+// particle pairs nA nB of the list, self pairs of a cell with itself excluded.
+__global__ __launch_bounds__(256) void k_csr_fill(long long m, int nc, int kb,
+                                                  const unsigned long long* __restrict__ key, int* __restrict__ src,
+                                                  int* __restrict__ off, const int* __restrict__ pcount,
+                                                  unsigned long long* __restrict__ pairs) {
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i < m) key[i] = ((unsigned long long)(unsigned)pr[i].x << 32) | (unsigned)pr[i].y;
+  unsigned long long w = 0;
+  if (i < m) {
+    const unsigned long long k = key[i];
+    const int t = (int)(k >> kb), b = (int)(k & ((1ull << kb) - 1));
+    src[i] = b;
+    const int prev = i > 0 ? (int)(key[i - 1] >> kb) : -1;
+    for (int r = prev + 1; r <= t; ++r) off[r] = (int)i;
+    if (i == m - 1)
+      for (int r = t + 1; r <= nc; ++r) off[r] = (int)m;
+    if (pairs) w = (unsigned long long)pcount[t] * (unsigned)pcount[b] - (t == b ? (unsigned)pcount[t] : 0u);
+  }
+  if (!pairs) return;
+  __shared__ unsigned long long red[4];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) w += __shfl_xor(w, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(pairs, red[0] + red[1] + red[2] + red[3]);
 }
 
-__global__ void k_csr_fill(long long m, const unsigned long long* __restrict__ key, int* __restrict__ src,
-                           int* __restrict__ row_first, int* __restrict__ row_end) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const unsigned long long k = key[i];
-  const int t = (int)(k >> 32);
-  src[i] = (int)(k & 0xffffffffu);
-  if (i == 0 || (int)(key[i - 1] >> 32) != t) row_first[t] = (int)i;
-  if (i == m - 1 || (int)(key[i + 1] >> 32) != t) row_end[t] = (int)(i + 1);
-}
-
-// Entries per row (0 for rows without any: both bounds stay zero).
-__global__ void k_csr_count(int ncells, const int* __restrict__ row_first, const int* __restrict__ row_end,
-                            int* __restrict__ cnt) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < ncells) cnt[c] = row_end[c] - row_first[c];
-}
-
-__global__ void k_set_int(int* __restrict__ p, int v) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *p = v;
+__global__ void k_fill_off(int n, int* __restrict__ off) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) off[i] = 0;
 }
 
 inline int blocks(long long n, int bs) { return (int)((n + bs - 1) / bs); }
-
-// P2P particle pairs: sum over list entries of nA * nB, minus self pairs.
-__global__ void k_p2p_work(int ncells, const int* __restrict__ off, const int* __restrict__ src,
-                           const int* __restrict__ pcount, unsigned long long* __restrict__ total) {
-  const int A = blockIdx.x * blockDim.x + threadIdx.x;
-  unsigned long long w = 0;
-  if (A < ncells) {
-    const long long na = pcount[A];
-    for (int i = off[A]; i < off[A + 1]; ++i) {
-      const int B = src[i];
-      w += (unsigned long long)(na * pcount[B] - (B == A ? na : 0));
-    }
-  }
-  if (w) atomicAdd(total, w);
-}
 
 template <typename T>
 void exclusive_scan_int(Scratch& s, const T* in, T* out, long long n, hipStream_t st) {
@@ -351,96 +591,88 @@ void exclusive_scan_int(Scratch& s, const T* in, T* out, long long n, hipStream_
   FMM_HIP(rocprim::exclusive_scan(tmp, bytes, in, out, T(0), (size_t)n, rocprim::plus<T>(), st));
 }
 
-// CSR offsets off[0..nc] from each row's first and one-past-last entry
-// (both zero for a row without entries): the exclusive scan of the row
-// lengths, so an empty row's offset is the next row's start; off[nc] = m.
-void close_csr(Tree& t, const int* first, const int* end, int* off, int nc, long long m, hipStream_t st) {
-  DevBuf<int> cnt;
-  cnt.alloc(nc);
-  k_csr_count<<<blocks(nc, 256), 256, 0, st>>>(nc, first, end, cnt.get());
-  exclusive_scan_int(t.scratch, cnt.get(), off, nc, st);
-  k_set_int<<<1, 64, 0, st>>>(off + nc, (int)m);
-  FMM_HIP(hipStreamSynchronize(st));  // cnt is freed on return
+int bits_for(unsigned long long v) {  // bits that hold 0 .. v
+  int b = 1;
+  while (v >>= 1) ++b;
+  return b;
 }
 
-void build_csr(Tree& t, DevBuf<int2>& pairs, long long m, DevBuf<int>& off, DevBuf<int>& src,
+void sort_keys(Tree& t, const unsigned long long* in, unsigned long long* out, long long m, int bits,
                hipStream_t st) {
+  size_t bytes = 0;
+  FMM_HIP(rocprim::radix_sort_keys(nullptr, bytes, in, out, (size_t)m, 0, bits, st));
+  void* tmp = t.scratch.get(bytes);
+  FMM_HIP(rocprim::radix_sort_keys(tmp, bytes, in, out, (size_t)m, 0, bits, st));
+}
+
+// CSR lists from the entry keys (target << kb) | source; `sorted` keeps the
+// sorted keys, `total` (optional) adds up the particle pairs.
+void build_csr(Tree& t, const unsigned long long* keys, long long m, int kb, DevBuf<unsigned long long>& sorted,
+               DevBuf<int>& off, DevBuf<int>& src, unsigned long long* total, hipStream_t st) {
   const int nc = t.ncells;
   off.alloc(nc + 1);
   src.alloc(std::max<long long>(m, 1));
-  DevBuf<int> first, end;
-  first.alloc(nc);
-  end.alloc(nc);
-  FMM_HIP(hipMemsetAsync(first.get(), 0, sizeof(int) * nc, st));
-  FMM_HIP(hipMemsetAsync(end.get(), 0, sizeof(int) * nc, st));
-  if (m > 0) {
-    DevBuf<unsigned long long> k0, k1;
-    k0.alloc(m);
-    k1.alloc(m);
-    k_pair_keys<<<blocks(m, 256), 256, 0, st>>>(m, pairs.get(), k0.get());
-    size_t bytes = 0;
-    FMM_HIP(rocprim::radix_sort_keys(nullptr, bytes, k0.get(), k1.get(), (size_t)m, 0, 64, st));
-    void* tmp = t.scratch.get(bytes);
-    FMM_HIP(rocprim::radix_sort_keys(tmp, bytes, k0.get(), k1.get(), (size_t)m, 0, 64, st));
-    k_csr_fill<<<blocks(m, 256), 256, 0, st>>>(m, k1.get(), src.get(), first.get(), end.get());
-    FMM_HIP(hipStreamSynchronize(st));
+  if (m == 0) {
+    k_fill_off<<<blocks(nc + 1, 256), 256, 0, st>>>(nc + 1, off.get());
+    return;
   }
-  close_csr(t, first.get(), end.get(), off.get(), nc, m, st);
+  sorted.alloc(m);
+  sort_keys(t, keys, sorted.get(), m, 2 * kb, st);
+  k_csr_fill<<<blocks(m, 256), 256, 0, st>>>(m, nc, kb, sorted.get(), src.get(), off.get(), t.pcount.get(), total);
 }
 
-// Source ranges: one entry per (target, non-self source) pair keyed by
-// (target, source particle start).
-__global__ void k_rng_keys(int ncells, const int* __restrict__ off, const int* __restrict__ src,
-                           const int* __restrict__ pstart, unsigned long long* __restrict__ key,
-                           int* __restrict__ cnt_out, int* __restrict__ pos) {
-  const int A = blockIdx.x * blockDim.x + threadIdx.x;
-  if (A >= ncells) return;
-  int w = pos[A];
-  for (int i = off[A]; i < off[A + 1]; ++i) {
-    const int B = src[i];
-    if (B == A) continue;
-    key[w] = ((unsigned long long)(unsigned)A << 32) | (unsigned)pstart[B];
-    cnt_out[w] = B;
-    ++w;
-  }
-}
-
-__global__ void k_rng_count(int ncells, const int* __restrict__ off, const int* __restrict__ src,
-                            int* __restrict__ n) {
-  const int A = blockIdx.x * blockDim.x + threadIdx.x;
-  if (A >= ncells) return;
-  int c = 0;
-  for (int i = off[A]; i < off[A + 1]; ++i) c += src[i] != A;
-  n[A] = c;
-}
-
-// run starts: new target, or a gap to the previous source's end
-__global__ void k_rng_flags(long long m, const unsigned long long* __restrict__ key, const int* __restrict__ srcB,
-                            const int* __restrict__ pcount, int* __restrict__ flag) {
+// Source ranges.  Keys (target << nb) | first source particle of every P2P
+// entry, from the sorted entry keys.
+__global__ void k_rng_keys(long long m, int kb, int nb, const unsigned long long* __restrict__ entry,
+                           const int* __restrict__ pstart, unsigned long long* __restrict__ key) {
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (i >= m) return;
-  int f = 1;
-  if (i > 0 && (key[i] >> 32) == (key[i - 1] >> 32)) {
-    const unsigned prev_end = (unsigned)(key[i - 1] & 0xffffffffu) + (unsigned)pcount[srcB[i - 1]];
-    f = ((unsigned)(key[i] & 0xffffffffu) != prev_end);
+  const unsigned long long k = entry[i];
+  key[i] = ((k >> kb) << nb) | (unsigned)pstart[k & ((1ull << kb) - 1)];
+}
+
+// A range starts at an entry that is not the target itself and is the target's
+// first, follows the target itself, or does not follow on its predecessor's
+// end.  Every source is a leaf, so the cell of an entry is that of its first
+// particle.
+struct RangeEntry {
+  int A, B, start;
+};
+__device__ __forceinline__ RangeEntry range_entry(unsigned long long k, int nb, const int* __restrict__ leaf_of) {
+  const int s = (int)(k & ((1ull << nb) - 1));
+  return RangeEntry{(int)(k >> nb), leaf_of[s], s};
+}
+__global__ void k_rng_flags(long long m, int nb, const unsigned long long* __restrict__ key,
+                            const int* __restrict__ leaf_of, const int* __restrict__ pcount, int* __restrict__ flag) {
+  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (i > m) return;
+  int f = 0;  // flag[m] = 0: the scan's last entry is the number of ranges
+  if (i < m) {
+    const RangeEntry e = range_entry(key[i], nb, leaf_of);
+    f = e.B != e.A;
+    if (f && i > 0) {
+      const RangeEntry p = range_entry(key[i - 1], nb, leaf_of);
+      if (p.A == e.A && p.B != p.A && p.start + pcount[p.B] == e.start) f = 0;
+    }
   }
   flag[i] = f;
 }
 
-__global__ void k_rng_fill(long long m, const unsigned long long* __restrict__ key, const int* __restrict__ srcB,
-                           const int* __restrict__ pcount, const int* __restrict__ flag, const int* __restrict__ pos,
-                           int* __restrict__ rstart, int* __restrict__ rlen, int* __restrict__ row_first,
-                           int* __restrict__ row_end) {
+__global__ void k_rng_fill(long long m, int nb, int nc, const unsigned long long* __restrict__ key,
+                           const int* __restrict__ leaf_of, const int* __restrict__ pcount,
+                           const int* __restrict__ flag, const int* __restrict__ pos, int* __restrict__ rstart,
+                           int* __restrict__ rlen, int* __restrict__ off) {
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (i >= m) return;
+  const RangeEntry e = range_entry(key[i], nb, leaf_of);
+  const int prev = i > 0 ? (int)(key[i - 1] >> nb) : -1;
+  for (int r = prev + 1; r <= e.A; ++r) off[r] = pos[i];
+  if (i == m - 1)
+    for (int r = e.A + 1; r <= nc; ++r) off[r] = pos[m];
+  if (e.B == e.A) return;
   const int r = pos[i] + flag[i] - 1;
-  const int A = (int)(key[i] >> 32);
-  if (flag[i]) {
-    rstart[r] = (int)(key[i] & 0xffffffffu);
-    if (i == 0 || (int)(key[i - 1] >> 32) != A) row_first[A] = r;
-  }
-  if (i == m - 1 || (int)(key[i + 1] >> 32) != A) row_end[A] = r + 1;
-  atomicAdd(&rlen[r], pcount[srcB[i]]);
+  if (flag[i]) rstart[r] = e.start;
+  atomicAdd(&rlen[r], pcount[e.B]);
 }
 
 // Per leaf: number of P2P segments; per range: its length as 64-bit.
@@ -534,54 +766,37 @@ void build_p2p_items(Tree& t, hipStream_t st) {
   t.p2p_split = total > t.nleaves;
 }
 
-// Merged source particle ranges of every P2P target (self excluded).
-void build_p2p_ranges(Tree& t, hipStream_t st) {
+// Merged source particle ranges of every P2P target (self excluded), from the
+// list's sorted entry keys.
+void build_p2p_ranges(Tree& t, const unsigned long long* entry, int kb, hipStream_t st) {
   const int nc = t.ncells;
-  DevBuf<int> cnt, pos;
-  cnt.alloc(nc + 1);
-  pos.alloc(nc + 1);
-  k_rng_count<<<blocks(nc, 256), 256, 0, st>>>(nc, t.p2p_off.get(), t.p2p_src.get(), cnt.get());
-  exclusive_scan_int(t.scratch, cnt.get(), pos.get(), nc, st);
-  int a = 0, b = 0;
-  FMM_HIP(hipMemcpyAsync(&a, cnt.get() + nc - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-  FMM_HIP(hipMemcpyAsync(&b, pos.get() + nc - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-  FMM_HIP(hipStreamSynchronize(st));
-  const long long m = (long long)a + b;
+  const long long m = t.n_p2p;
   t.rng_off.alloc(nc + 1);
+  t.n_rng = 0;
   if (m == 0) {
-    t.n_rng = 0;
     t.rng_start.alloc(1);
     t.rng_len.alloc(1);
-    FMM_HIP(hipMemsetAsync(t.rng_off.get(), 0, sizeof(int) * (nc + 1), st));
-    FMM_HIP(hipStreamSynchronize(st));
+    k_fill_off<<<blocks(nc + 1, 256), 256, 0, st>>>(nc + 1, t.rng_off.get());
     return;
   }
+  const int nb = bits_for((unsigned long long)t.n - 1);
   DevBuf<unsigned long long> k0, k1;
-  DevBuf<int> b0, b1, fl, ps;
-  k0.alloc(m); k1.alloc(m); b0.alloc(m); b1.alloc(m); fl.alloc(m); ps.alloc(m);
-  k_rng_keys<<<blocks(nc, 256), 256, 0, st>>>(nc, t.p2p_off.get(), t.p2p_src.get(), t.pstart.get(), k0.get(),
-                                              b0.get(), pos.get());
-  size_t bytes = 0;
-  FMM_HIP(rocprim::radix_sort_pairs(nullptr, bytes, k0.get(), k1.get(), b0.get(), b1.get(), (size_t)m, 0, 64, st));
-  void* tmp = t.scratch.get(bytes);
-  FMM_HIP(rocprim::radix_sort_pairs(tmp, bytes, k0.get(), k1.get(), b0.get(), b1.get(), (size_t)m, 0, 64, st));
-  k_rng_flags<<<blocks(m, 256), 256, 0, st>>>(m, k1.get(), b1.get(), t.pcount.get(), fl.get());
-  exclusive_scan_int(t.scratch, fl.get(), ps.get(), m, st);
-  FMM_HIP(hipMemcpyAsync(&a, fl.get() + m - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-  FMM_HIP(hipMemcpyAsync(&b, ps.get() + m - 1, sizeof(int), hipMemcpyDeviceToHost, st));
+  DevBuf<int> fl, ps;
+  k0.alloc(m); k1.alloc(m); fl.alloc(m + 1); ps.alloc(m + 1);
+  k_rng_keys<<<blocks(m, 256), 256, 0, st>>>(m, kb, nb, entry, t.pstart.get(), k0.get());
+  sort_keys(t, k0.get(), k1.get(), m, kb + nb, st);
+  k_rng_flags<<<blocks(m + 1, 256), 256, 0, st>>>(m, nb, k1.get(), t.leaf_of.get(), t.pcount.get(), fl.get());
+  exclusive_scan_int(t.scratch, fl.get(), ps.get(), m + 1, st);
+  int total = 0;
+  FMM_HIP(hipMemcpyAsync(&total, ps.get() + m, sizeof(int), hipMemcpyDeviceToHost, st));
   FMM_HIP(hipStreamSynchronize(st));
-  t.n_rng = (long long)a + b;
-  t.rng_start.alloc(t.n_rng);
-  t.rng_len.alloc(t.n_rng);
-  FMM_HIP(hipMemsetAsync(t.rng_len.get(), 0, sizeof(int) * t.n_rng, st));
-  DevBuf<int> first, end;
-  first.alloc(nc);
-  end.alloc(nc);
-  FMM_HIP(hipMemsetAsync(first.get(), 0, sizeof(int) * nc, st));
-  FMM_HIP(hipMemsetAsync(end.get(), 0, sizeof(int) * nc, st));
-  k_rng_fill<<<blocks(m, 256), 256, 0, st>>>(m, k1.get(), b1.get(), t.pcount.get(), fl.get(), ps.get(),
-                                             t.rng_start.get(), t.rng_len.get(), first.get(), end.get());
-  close_csr(t, first.get(), end.get(), t.rng_off.get(), nc, t.n_rng, st);
+  t.n_rng = total;
+  t.rng_start.alloc(std::max(total, 1));
+  t.rng_len.alloc(std::max(total, 1));
+  FMM_HIP(hipMemsetAsync(t.rng_len.get(), 0, sizeof(int) * std::max(total, 1), st));
+  k_rng_fill<<<blocks(m, 256), 256, 0, st>>>(m, nb, nc, k1.get(), t.leaf_of.get(), t.pcount.get(), fl.get(), ps.get(),
+                                             t.rng_start.get(), t.rng_len.get(), t.rng_off.get());
+  FMM_HIP(hipStreamSynchronize(st));  // the temporaries are freed on return
 }
 
 // Builds the tree of `t` from caller positions (device, [n*3]).
@@ -593,8 +808,18 @@ void build_tree_device(Tree& t, const double* d_pos, hipStream_t st) {
   mean.alloc(3);
   mx.alloc(3);
   FMM_HIP(hipMemsetAsync(mx.get(), 0, 3 * sizeof(unsigned long long), st));
-  k_mean<<<1, 256, 0, st>>>(d_pos, n, mean.get());
-  k_maxdev<<<std::min(blocks(n, 256), 2048), 256, 0, st>>>(d_pos, n, mean.get(), mx.get());
+  const long long nrun = ((long long)n + kMeanChunk - 1) / kMeanChunk;
+  DevBuf<MeanRun> mrun;
+  DevBuf<int> mexp;
+  DevBuf<MeanStep> mstep;
+  mrun.alloc(3 * nrun);
+  mexp.alloc(3 * nrun);
+  mstep.alloc(3 * nrun);
+  k_mean_sums<<<(int)nrun, 192, 0, st>>>(d_pos, n, nrun, mrun.get());
+  k_mean_scan<<<3, 1024, 0, st>>>(n, nrun, mrun.get(), mexp.get());
+  k_mean_steps<<<(int)nrun, 192, 0, st>>>(d_pos, n, nrun, mexp.get(), mstep.get());
+  k_mean_walk<<<3, 64, 0, st>>>(d_pos, n, nrun, mexp.get(), mstep.get(), mean.get());
+  k_maxdev<<<std::min(blocks(n, 256), 1024), 256, 0, st>>>(d_pos, n, mean.get(), mx.get());
 
   // per-level arrays
   struct Level {
@@ -605,15 +830,11 @@ void build_tree_device(Tree& t, const double* d_pos, hipStream_t st) {
   std::vector<Level*> lv;
   auto new_level = [&](int m) {
     Level* L = new Level();
+    lv.push_back(L);
     L->n = m;
     L->cx.alloc(m); L->cy.alloc(m); L->cz.alloc(m); L->r.alloc(m);
     L->count.alloc(m); L->parent.alloc(m); L->first_child.alloc(m); L->nchild.alloc(m); L->octmask.alloc(m);
     L->oct.alloc(m);
-    FMM_HIP(hipMemsetAsync(L->oct.get(), 0, sizeof(int) * m, st));
-    FMM_HIP(hipMemsetAsync(L->nchild.get(), 0, sizeof(int) * m, st));
-    FMM_HIP(hipMemsetAsync(L->octmask.get(), 0, sizeof(int) * m, st));
-    FMM_HIP(hipMemsetAsync(L->first_child.get(), 0xff, sizeof(int) * m, st));
-    lv.push_back(L);
     return L;
   };
   struct Cleanup {
@@ -621,50 +842,55 @@ void build_tree_device(Tree& t, const double* d_pos, hipStream_t st) {
     ~Cleanup() { for (auto* p : v) delete p; }
   } cleanup{lv};
 
-  Level* root = new_level(1);
-  FMM_HIP(hipMemsetAsync(root->parent.get(), 0, sizeof(int), st));
-  k_root<<<1, 1, 0, st>>>(mean.get(), mx.get(), root->cx.get(), root->cy.get(), root->cz.get(), root->r.get(),
-                          root->count.get(), n);
-
-  DevBuf<int> pcell, leaf_orig, ccount, flag, cidx;
+  DevBuf<int> pcell, leaf_orig, ccount[2], cidx[2];  // counters and numbering of this level and the last
   DevBuf<unsigned char> poct;
   DevBuf<unsigned long long> key;
   pcell.alloc(n);
   leaf_orig.alloc(n);
   poct.alloc(n);
   key.alloc(n);
-  FMM_HIP(hipMemsetAsync(pcell.get(), 0, sizeof(int) * n, st));
-  FMM_HIP(hipMemsetAsync(key.get(), 0, sizeof(unsigned long long) * n, st));
+  Level* root = new_level(1);
+  ccount[0].alloc(8);
+  k_root<<<1, 1, 0, st>>>(mean.get(), mx.get(), root->cx.get(), root->cy.get(), root->cz.get(), root->r.get(),
+                          root->count.get(), root->parent.get(), root->oct.get(), ccount[0].get(), n);
 
   std::vector<int> level_off{0};
   int level = 0;
+  constexpr int kHist = 4096;  // octant counters of a block (16 KB): levels of up to 512 cells
   while (true) {
     Level* cur = lv.back();
-    const int m = cur->n;
+    const int m = cur->n, h = level & 1;
     level_off.push_back(level_off.back() + m);
-    ccount.alloc(8 * (size_t)m);
-    FMM_HIP(hipMemsetAsync(ccount.get(), 0, sizeof(int) * 8 * (size_t)m, st));
-    k_level_octants<<<blocks(n, 256), 256, 0, st>>>(d_pos, n, pcell.get(), poct.get(), leaf_orig.get(),
-                                                    cur->cx.get(), cur->cy.get(), cur->cz.get(),
-                                                    cur->count.get(), ccount.get(), ncrit, level_off[level]);
-    flag.alloc(8 * (size_t)m);
-    cidx.alloc(8 * (size_t)m + 1);
-    k_flags<<<blocks(8LL * m, 256), 256, 0, st>>>(ccount.get(), flag.get(), 8 * m);
-    exclusive_scan_int(t.scratch, flag.get(), cidx.get(), 8LL * m, st);
-    int last_flag = 0, last_idx = 0;
-    FMM_HIP(hipMemcpyAsync(&last_flag, flag.get() + 8 * (size_t)m - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-    FMM_HIP(hipMemcpyAsync(&last_idx, cidx.get() + 8 * (size_t)m - 1, sizeof(int), hipMemcpyDeviceToHost, st));
+    auto octants = [&](auto kern, int grid) {
+      kern<<<grid, 256, 0, st>>>(d_pos, n, level, m, pcell.get(), poct.get(), key.get(), cidx[h ^ 1].get(),
+                                 leaf_orig.get(), cur->cx.get(), cur->cy.get(), cur->cz.get(), cur->count.get(),
+                                 ccount[h].get(), ncrit, level_off[level]);
+    };
+    if (8LL * m <= kHist) octants(k_level_octants<kHist>, std::min(blocks(n, 256), 1024));
+    else octants(k_level_octants<0>, std::min(blocks(n, 256), 1 << 16));
+    cidx[h].alloc(8 * (size_t)m + 1);
+    // numbering of the occupied octants: cidx[j] = how many come before j
+    auto occ = rocprim::make_transform_iterator(ccount[h].get(), Occupied());
+    size_t bytes = 0;
+    FMM_HIP(rocprim::inclusive_scan(nullptr, bytes, occ, cidx[h].get() + 1, 8 * (size_t)m, rocprim::plus<int>(), st));
+    void* tmp = t.scratch.get(bytes);
+    FMM_HIP(rocprim::inclusive_scan(tmp, bytes, occ, cidx[h].get() + 1, 8 * (size_t)m, rocprim::plus<int>(), st));
+    FMM_HIP(hipMemsetAsync(cidx[h].get(), 0, sizeof(int), st));
+    int nnext = 0;
+    FMM_HIP(hipMemcpyAsync(&nnext, cidx[h].get() + 8 * (size_t)m, sizeof(int), hipMemcpyDeviceToHost, st));
     FMM_HIP(hipStreamSynchronize(st));
-    const int nnext = last_idx + last_flag;
-    if (nnext == 0) break;
-    FMM_CHECK(level < kMaxSplitLevels, kTreeTooDeep,
+    FMM_CHECK(nnext == 0 || level < kMaxSplitLevels, kTreeTooDeep,
               "tree deeper than 21 split levels (coincident particles?)");
-    Level* nx = new_level(nnext);
+    Level* nx = nnext > 0 ? new_level(nnext) : nullptr;
+    if (nx) ccount[h ^ 1].alloc(8 * (size_t)nnext);
+    // on the last level: no children, their arrays are not touched
     k_make_children<<<blocks(m, 256), 256, 0, st>>>(
-        m, ccount.get(), cidx.get(), cur->cx.get(), cur->cy.get(), cur->cz.get(), cur->r.get(), nx->cx.get(),
-        nx->cy.get(), nx->cz.get(), nx->r.get(), nx->count.get(), nx->parent.get(), nx->oct.get(),
-        cur->first_child.get(), cur->nchild.get(), cur->octmask.get());
-    k_descend<<<blocks(n, 256), 256, 0, st>>>(n, pcell.get(), poct.get(), cidx.get(), key.get(), level);
+        m, ccount[h].get(), cidx[h].get(), cur->cx.get(), cur->cy.get(), cur->cz.get(), cur->r.get(),
+        nx ? nx->cx.get() : nullptr, nx ? nx->cy.get() : nullptr, nx ? nx->cz.get() : nullptr,
+        nx ? nx->r.get() : nullptr, nx ? nx->count.get() : nullptr, nx ? nx->parent.get() : nullptr,
+        nx ? nx->oct.get() : nullptr, ccount[h ^ 1].get(), cur->first_child.get(), cur->nchild.get(),
+        cur->octmask.get());
+    if (!nx) break;
     ++level;
   }
   t.depth = (int)lv.size();
@@ -672,155 +898,131 @@ void build_tree_device(Tree& t, const double* d_pos, hipStream_t st) {
   t.ncells = level_off.back();
   const int nc = t.ncells;
 
-  // concatenate levels into canonical global arrays
+  // levels into the canonical global arrays
   t.cx.alloc(nc); t.cy.alloc(nc); t.cz.alloc(nc); t.cr.alloc(nc); t.crmax.alloc(nc);
   t.parent.alloc(nc); t.first_child.alloc(nc); t.nchild.alloc(nc); t.octmask.alloc(nc);
   t.level.alloc(nc); t.pstart.alloc(nc); t.pcount.alloc(nc); t.octant.alloc(nc);
-  std::vector<int> hlevel(nc);
+  const CellArrays out{t.cx.get(), t.cy.get(), t.cz.get(), t.cr.get(), t.crmax.get(), t.pcount.get(), t.parent.get(),
+                       t.first_child.get(), t.nchild.get(), t.octmask.get(), t.octant.get(), t.level.get()};
   for (int l = 0; l < t.depth; ++l) {
     Level* L = lv[l];
-    const int o = level_off[l], m = L->n;
-    auto cp = [&](void* dst, const void* src, size_t bytes) {
-      FMM_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, st));
-    };
-    cp(t.cx.get() + o, L->cx.get(), sizeof(double) * m);
-    cp(t.cy.get() + o, L->cy.get(), sizeof(double) * m);
-    cp(t.cz.get() + o, L->cz.get(), sizeof(double) * m);
-    cp(t.cr.get() + o, L->r.get(), sizeof(double) * m);
-    cp(t.pcount.get() + o, L->count.get(), sizeof(int) * m);
-    cp(t.parent.get() + o, L->parent.get(), sizeof(int) * m);
-    cp(t.first_child.get() + o, L->first_child.get(), sizeof(int) * m);
-    cp(t.nchild.get() + o, L->nchild.get(), sizeof(int) * m);
-    cp(t.octmask.get() + o, L->octmask.get(), sizeof(int) * m);
-    cp(t.octant.get() + o, L->oct.get(), sizeof(int) * m);
-    if (l > 0) k_offset_add<<<blocks(m, 256), 256, 0, st>>>(t.parent.get() + o, m, level_off[l - 1]);
-    if (l + 1 < t.depth) k_offset_add<<<blocks(m, 256), 256, 0, st>>>(t.first_child.get() + o, m, level_off[l + 1]);
-    for (int c = 0; c < m; ++c) hlevel[o + c] = l;
+    k_place_level<<<blocks(L->n, 256), 256, 0, st>>>(
+        L->n, level_off[l], l > 0 ? level_off[l - 1] : 0, level_off[l + 1], l, L->cx.get(), L->cy.get(), L->cz.get(),
+        L->r.get(), L->count.get(), L->parent.get(), L->first_child.get(), L->nchild.get(), L->octmask.get(),
+        L->oct.get(), out);
   }
-  FMM_HIP(hipMemcpyAsync(t.level.get(), hlevel.data(), sizeof(int) * nc, hipMemcpyHostToDevice, st));
-  k_rmax<<<blocks(nc, 256), 256, 0, st>>>(nc, t.cr.get(), t.crmax.get());
 
   // stable sort of particles by path key
   {
     DevBuf<unsigned long long> k1;
-    DevBuf<int> v0;
     k1.alloc(n);
-    v0.alloc(n);
     t.perm.alloc(n);
-    k_iota<<<blocks(n, 256), 256, 0, st>>>(v0.get(), n);
     const unsigned begin_bit = 3u * (unsigned)(kMaxSplitLevels - std::max(level, 1));
+    const rocprim::counting_iterator<int> iota(0);
     size_t bytes = 0;
-    FMM_HIP(rocprim::radix_sort_pairs(nullptr, bytes, key.get(), k1.get(), v0.get(), t.perm.get(), (size_t)n,
-                                      begin_bit, 63u, st));
+    FMM_HIP(rocprim::radix_sort_pairs(nullptr, bytes, key.get(), k1.get(), iota, t.perm.get(), (size_t)n, begin_bit,
+                                      63u, st));
     void* tmp = t.scratch.get(bytes);
-    FMM_HIP(rocprim::radix_sort_pairs(tmp, bytes, key.get(), k1.get(), v0.get(), t.perm.get(), (size_t)n,
-                                      begin_bit, 63u, st));
+    FMM_HIP(rocprim::radix_sort_pairs(tmp, bytes, key.get(), k1.get(), iota, t.perm.get(), (size_t)n, begin_bit, 63u,
+                                      st));
     FMM_HIP(hipStreamSynchronize(st));
   }
   t.px.alloc(n); t.py.alloc(n); t.pz.alloc(n); t.leaf_of.alloc(n);
   k_gather_particles<<<blocks(n, 256), 256, 0, st>>>(n, t.perm.get(), d_pos, leaf_orig.get(), t.px.get(),
                                                      t.py.get(), t.pz.get(), t.leaf_of.get());
   k_leaf_starts<<<blocks(n, 256), 256, 0, st>>>(n, t.leaf_of.get(), t.pstart.get());
-  for (int l = t.depth - 2; l >= 0; --l) {
-    const int b = level_off[l], e = level_off[l + 1];
-    k_internal_starts<<<blocks(e - b, 256), 256, 0, st>>>(b, e, t.nchild.get(), t.first_child.get(),
-                                                          t.pstart.get());
-  }
+  k_internal_starts<<<blocks(nc, 256), 256, 0, st>>>(nc, t.nchild.get(), t.first_child.get(), t.pstart.get());
   // leaves in canonical order
   {
-    DevBuf<int> lf, lp;
-    lf.alloc(nc + 1);
+    DevBuf<int> lp;
     lp.alloc(nc + 1);
-    k_leaf_flags<<<blocks(nc, 256), 256, 0, st>>>(nc, t.nchild.get(), lf.get());
-    exclusive_scan_int(t.scratch, lf.get(), lp.get(), nc, st);
-    int a = 0, b = 0;
-    FMM_HIP(hipMemcpyAsync(&a, lf.get() + nc - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-    FMM_HIP(hipMemcpyAsync(&b, lp.get() + nc - 1, sizeof(int), hipMemcpyDeviceToHost, st));
+    auto leaf = rocprim::make_transform_iterator(t.nchild.get(), IsLeaf());
+    size_t bytes = 0;
+    FMM_HIP(rocprim::inclusive_scan(nullptr, bytes, leaf, lp.get() + 1, (size_t)nc, rocprim::plus<int>(), st));
+    void* tmp = t.scratch.get(bytes);
+    FMM_HIP(rocprim::inclusive_scan(tmp, bytes, leaf, lp.get() + 1, (size_t)nc, rocprim::plus<int>(), st));
+    FMM_HIP(hipMemsetAsync(lp.get(), 0, sizeof(int), st));
+    FMM_HIP(hipMemcpyAsync(&t.nleaves, lp.get() + nc, sizeof(int), hipMemcpyDeviceToHost, st));
     FMM_HIP(hipStreamSynchronize(st));
-    t.nleaves = a + b;
     t.leaves.alloc(t.nleaves);
-    k_leaf_compact<<<blocks(nc, 256), 256, 0, st>>>(nc, lf.get(), lp.get(), t.leaves.get());
+    k_leaf_compact<<<blocks(nc, 256), 256, 0, st>>>(nc, t.nchild.get(), lp.get(), t.leaves.get());
     FMM_HIP(hipStreamSynchronize(st));
   }
-  FMM_HIP(hipStreamSynchronize(st));
 }
 
 // Breadth-first dual traversal from (root, root) and CSR lists by target.
 void build_lists_device(Tree& t, hipStream_t st) {
-  DevBuf<int2> cur, nxt, m2l, p2p;
+  DevBuf<int2> cur, nxt;
+  DevBuf<unsigned long long> m2l, p2p, sorted;
   DevBuf<Counts3> cnt, off;
   DevBuf<unsigned char> dec;
+  DevBuf<unsigned long long> total;
+  DevBuf<int> maxq;
+  const int kb = bits_for((unsigned long long)t.ncells - 1);
   long long n_m2l = 0, n_p2p = 0;
-  long long cap_m2l = 1 << 20, cap_p2p = 1 << 20;
+  // about 27 M2L and 9 P2P entries a particle at 64 particles a leaf
+  long long cap_m2l = std::max<long long>(1 << 16, 16LL * (long long)t.n), cap_p2p = cap_m2l / 2;
   m2l.alloc(cap_m2l);
   p2p.alloc(cap_p2p);
   cur.alloc(1);
-  int2 rootpair = make_int2(0, 0);
-  FMM_HIP(hipMemcpyAsync(cur.get(), &rootpair, sizeof(int2), hipMemcpyHostToDevice, st));
+  total.alloc(1);
+  maxq.alloc(1);
+  FMM_HIP(hipMemsetAsync(cur.get(), 0, sizeof(int2), st));  // the pair (root, root)
+  FMM_HIP(hipMemsetAsync(total.get(), 0, sizeof(unsigned long long), st));
+  FMM_HIP(hipMemsetAsync(maxq.get(), 0, sizeof(int), st));
   int nf = 1;
-  auto grow = [&](DevBuf<int2>& b, long long& cap, long long used, long long need) {
+  auto grow = [&](DevBuf<unsigned long long>& b, long long& cap, long long used, long long need) {
     if (need <= cap) return;
-    long long nc = std::max(need, 2 * cap);
-    DevBuf<int2> nb;
-    nb.alloc(nc);
-    if (used > 0) FMM_HIP(hipMemcpyAsync(nb.get(), b.get(), sizeof(int2) * used, hipMemcpyDeviceToDevice, st));
+    const long long c = std::max(need, 2 * cap);
+    DevBuf<unsigned long long> nb;
+    nb.alloc(c);
+    if (used > 0)
+      FMM_HIP(hipMemcpyAsync(nb.get(), b.get(), sizeof(unsigned long long) * used, hipMemcpyDeviceToDevice, st));
     FMM_HIP(hipStreamSynchronize(st));
     std::swap(b.p, nb.p);
     std::swap(b.n, nb.n);
-    cap = nc;
+    cap = c;
   };
   while (nf > 0) {
     cnt.alloc(nf + 1);
     off.alloc(nf + 1);
     dec.alloc(nf);
-    k_pair_count<<<blocks(nf, 256), 256, 0, st>>>(nf, cur.get(), cnt.get(), dec.get(), t.cx.get(), t.cy.get(),
-                                                  t.cz.get(), t.crmax.get(), t.nchild.get(), t.pcount.get(),
-                                                  t.theta, (int)t.ncrit);
-    {
-      size_t bytes = 0;
-      FMM_HIP(rocprim::exclusive_scan(nullptr, bytes, cnt.get(), off.get(), Counts3{0, 0, 0}, (size_t)nf, Plus3(), st));
-      void* tmp = t.scratch.get(bytes);
-      FMM_HIP(rocprim::exclusive_scan(tmp, bytes, cnt.get(), off.get(), Counts3{0, 0, 0}, (size_t)nf, Plus3(), st));
-    }
-    Counts3 lastc, lasto;
-    FMM_HIP(hipMemcpyAsync(&lastc, cnt.get() + nf - 1, sizeof(Counts3), hipMemcpyDeviceToHost, st));
-    FMM_HIP(hipMemcpyAsync(&lasto, off.get() + nf - 1, sizeof(Counts3), hipMemcpyDeviceToHost, st));
+    k_pair_count<<<blocks(nf + 1, 256), 256, 0, st>>>(nf, cur.get(), cnt.get(), dec.get(), t.cx.get(), t.cy.get(),
+                                                      t.cz.get(), t.crmax.get(), t.nchild.get(), t.pcount.get(),
+                                                      t.theta, (int)t.ncrit);
+    size_t bytes = 0;
+    FMM_HIP(rocprim::exclusive_scan(nullptr, bytes, cnt.get(), off.get(), Counts3{0, 0, 0}, (size_t)nf + 1, Plus3(),
+                                    st));
+    void* tmp = t.scratch.get(bytes);
+    FMM_HIP(rocprim::exclusive_scan(tmp, bytes, cnt.get(), off.get(), Counts3{0, 0, 0}, (size_t)nf + 1, Plus3(), st));
+    Counts3 add;
+    FMM_HIP(hipMemcpyAsync(&add, off.get() + nf, sizeof(Counts3), hipMemcpyDeviceToHost, st));
     FMM_HIP(hipStreamSynchronize(st));
-    const long long add_m2l = (long long)lastc.m2l + lasto.m2l;
-    const long long add_p2p = (long long)lastc.p2p + lasto.p2p;
-    const long long add_nxt = (long long)lastc.nxt + lasto.nxt;
-    grow(m2l, cap_m2l, n_m2l, n_m2l + add_m2l);
-    grow(p2p, cap_p2p, n_p2p, n_p2p + add_p2p);
-    nxt.alloc(std::max<long long>(add_nxt, 1));
+    FMM_CHECK(add.m2l >= 0 && add.p2p >= 0 && add.nxt >= 0, kOutOfMemory, "traversal frontier exceeds 2^31 pairs");
+    grow(m2l, cap_m2l, n_m2l, n_m2l + add.m2l);
+    grow(p2p, cap_p2p, n_p2p, n_p2p + add.p2p);
+    nxt.alloc(std::max(add.nxt, 1));
     k_pair_emit<<<blocks(nf, 256), 256, 0, st>>>(nf, cur.get(), off.get(), dec.get(), t.first_child.get(),
-                                                 t.nchild.get(), m2l.get(), n_m2l, p2p.get(), n_p2p, nxt.get());
-    FMM_HIP(hipStreamSynchronize(st));
-    n_m2l += add_m2l;
-    n_p2p += add_p2p;
-    FMM_CHECK(add_nxt < (1LL << 31), kOutOfMemory, "traversal frontier exceeds 2^31 pairs");
-    nf = (int)add_nxt;
+                                                 t.nchild.get(), t.cx.get(), t.cy.get(), t.cz.get(), t.cr.get(), kb,
+                                                 m2l.get(), n_m2l, p2p.get(), n_p2p, nxt.get(), maxq.get());
+    n_m2l += add.m2l;
+    n_p2p += add.p2p;
+    nf = add.nxt;
     std::swap(cur.p, nxt.p);
     std::swap(cur.n, nxt.n);
   }
-  FMM_HIP(hipStreamSynchronize(st));
+  FMM_CHECK(n_m2l < (1LL << 31) && n_p2p < (1LL << 31), kOutOfMemory, "more than 2^31 list entries");
   t.n_m2l = n_m2l;
   t.n_p2p = n_p2p;
-  build_csr(t, m2l, n_m2l, t.m2l_off, t.m2l_src, st);
-  build_csr(t, p2p, n_p2p, t.p2p_off, t.p2p_src, st);
-  build_p2p_ranges(t, st);
+  FMM_HIP(hipMemcpyAsync(&t.m2l_maxq, maxq.get(), sizeof(int), hipMemcpyDeviceToHost, st));
+  build_csr(t, m2l.get(), n_m2l, kb, sorted, t.m2l_off, t.m2l_src, nullptr, st);
+  build_csr(t, p2p.get(), n_p2p, kb, sorted, t.p2p_off, t.p2p_src, total.get(), st);
+  unsigned long long h = 0;
+  FMM_HIP(hipMemcpyAsync(&h, total.get(), sizeof(h), hipMemcpyDeviceToHost, st));
+  build_p2p_ranges(t, sorted.get(), kb, st);
   build_p2p_items(t, st);
-  {
-    DevBuf<unsigned long long> tot;
-    tot.alloc(1);
-    FMM_HIP(hipMemsetAsync(tot.get(), 0, sizeof(unsigned long long), st));
-    k_p2p_work<<<blocks(t.ncells, 256), 256, 0, st>>>(t.ncells, t.p2p_off.get(), t.p2p_src.get(), t.pcount.get(),
-                                                      tot.get());
-    unsigned long long h = 0;
-    FMM_HIP(hipMemcpyAsync(&h, tot.get(), sizeof(h), hipMemcpyDeviceToHost, st));
-    FMM_HIP(hipStreamSynchronize(st));
-    t.p2p_particle_pairs = (long long)h;
-  }
   FMM_HIP(hipStreamSynchronize(st));
+  t.p2p_particle_pairs = (long long)h;
 }
 
 }  // namespace fmm
