@@ -19,39 +19,146 @@ __global__ void k_gather_S(int n, const int* __restrict__ perm, const double* __
   for (int k = 0; k < SS; ++k) pS[(size_t)j * SS + k] = S[(size_t)i * SS + k];
 }
 
-// FP64 direct sum on sampled targets (example/calculate.cpp:252-264): one
-// block per target, sources strided over the lanes, tree reduction in LDS.
-__global__ void k_direct(int n, const double* __restrict__ pos, const double* __restrict__ S,
-                         const long long* __restrict__ tg, int nt, double* __restrict__ F) {
-  const int t = blockIdx.x;
-  if (t >= nt) return;
-  const long long i = tg[t];
-  if (i < 0 || i >= n) {  // out-of-range target: NaN row, no access
-    if (threadIdx.x == 0)
-      for (int k = 0; k < OUT; ++k) F[(size_t)t * OUT + k] = __longlong_as_double(0x7ff8000000000000LL);
-    return;
+// One charge pair in FP64 (the example's P2P, example/calculate.cpp:24-40):
+// q/r and q r^-3 (dx, dy, dz) from the hardware estimate y of x^(-1/2), x = r^2,
+// corrected by the series of (1 - e)^(-1/2), e = 1 - x y^2, which cubes the
+// estimate's relative error.  No case of x is treated apart: where x or a power
+// of y leaves the finite range (coincident particles above all) the result is
+// NaN, and the callers repeat such sums with the generated body.  19
+// instructions and the estimate, against 23 in the generated body (its select
+// of zero and infinite x).
+__device__ __forceinline__ void charge_pair(double dx, double dy, double dz, double q, double* acc) {
+  const double x = fma(dx, dx, fma(dy, dy, dz * dz));
+  const double y = __builtin_amdgcn_rsq(x);
+  const double y2 = y * y;
+  const double e = fma(-x, y2, 1.0);
+  double s3;
+  if constexpr (OUT == 3) {
+    const double q3 = q * (y2 * y), t = q3 * e;
+    s3 = fma(t * e, 1.875, fma(t, 1.5, q3));
+  } else {
+    const double r = fma(y * e, fma(e, 0.375, 0.5), y), s = q * r;
+    acc[0] += s;
+    s3 = s * (r * r);
   }
-  const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-  double acc[OUT];
-#pragma unroll
-  for (int k = 0; k < OUT; ++k) acc[k] = 0.0;
-  for (int j = threadIdx.x; j < n; j += blockDim.x) {
-    if (j == i) continue;
-    fmmgen_ops::P2P<double>(xi - pos[3 * j], yi - pos[3 * j + 1], zi - pos[3 * j + 2], S + (size_t)j * SS, acc);
+  if constexpr (OUT != 1) {
+    constexpr int F0 = OUT == 4 ? 1 : 0;
+    acc[F0] = fma(s3, dx, acc[F0]);
+    acc[F0 + 1] = fma(s3, dy, acc[F0 + 1]);
+    acc[F0 + 2] = fma(s3, dz, acc[F0 + 2]);
   }
-  __shared__ double red[256][OUT];
+}
+
+// FP64 direct sum on sampled targets (example/calculate.cpp:252-264): a block
+// holds TT targets in registers, so that each source read serves TT pairs, and
+// strides its BS threads over the sources, the next source loaded during the
+// pairs of this one; wave sums, then a sum over the waves, in a fixed order.
+// Charges take charge_pair, the target itself as a zero charge at unit
+// distance; a row that comes out as NaN is summed again with the generated
+// body.  Bound by the FP64 pairs: 4096 targets x 2^20 charges 6.9 ms with one
+// target a block, 4.1 ms with four.
+template <int TT, int BS>
+__global__ __launch_bounds__(BS, 4) void k_direct(int n, const double* __restrict__ pos, const double* __restrict__ S,
+                                                  const long long* __restrict__ tg, int nt, double* __restrict__ F) {
+  const int t0 = blockIdx.x * TT;
+  int ti[TT];
+  double tx[TT], ty[TT], tz[TT], acc[TT][OUT];
 #pragma unroll
-  for (int k = 0; k < OUT; ++k) red[threadIdx.x][k] = acc[k];
+  for (int u = 0; u < TT; ++u) {
+    const long long i = t0 + u < nt ? tg[t0 + u] : -1;
+    const bool in = i >= 0 && i < n;  // an out-of-range target: NaN row, no access
+    ti[u] = in ? (int)i : -1;
+    tx[u] = in ? pos[3 * i] : 0.0;
+    ty[u] = in ? pos[3 * i + 1] : 0.0;
+    tz[u] = in ? pos[3 * i + 2] : 0.0;
+#pragma unroll
+    for (int k = 0; k < OUT; ++k) acc[u][k] = 0.0;
+  }
+  double nx[3], ns[SS];
+  auto load = [&](unsigned j) {
+    const size_t i = j < (unsigned)n ? j : n - 1;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) nx[k] = pos[3 * i + k];
+#pragma unroll
+    for (int k = 0; k < SS; ++k) ns[k] = S[i * SS + k];
+  };
+  load(threadIdx.x);
+  for (unsigned b = 0; b < (unsigned)n; b += BS) {
+    const unsigned j = b + threadIdx.x;
+    const double x = nx[0], y = nx[1], z = nx[2];
+    double s[SS];
+#pragma unroll
+    for (int k = 0; k < SS; ++k) s[k] = ns[k];
+    load(j + BS);
+    if (j >= (unsigned)n) continue;
+    if constexpr (SO == 0) {
+      bool own = false;  // uniform: this step holds a target of the block
+#pragma unroll
+      for (int u = 0; u < TT; ++u) own = own || (unsigned)ti[u] - b < (unsigned)BS;
+      if (own) {
+#pragma unroll
+        for (int u = 0; u < TT; ++u) {
+          const bool self = j == (unsigned)ti[u];
+          charge_pair(self ? 1.0 : tx[u] - x, ty[u] - y, tz[u] - z, self ? 0.0 : s[0], acc[u]);
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < TT; ++u) charge_pair(tx[u] - x, ty[u] - y, tz[u] - z, s[0], acc[u]);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < TT; ++u)
+        if (j != (unsigned)ti[u]) fmmgen_ops::P2P<double>(tx[u] - x, ty[u] - y, tz[u] - z, s, acc[u]);
+    }
+  }
+  constexpr int NW = BS / 64;
+  __shared__ double red[NW][TT * OUT], sum[TT * OUT];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  auto fold = [&](const double (&a)[OUT], int u) {  // wave sums of target u
+#pragma unroll
+    for (int k = 0; k < OUT; ++k) {
+      double v = a[k];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+      if (lane == 0) red[w][u * OUT + k] = v;
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < TT; ++u) fold(acc[u], u);
   __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s)
-#pragma unroll
-      for (int k = 0; k < OUT; ++k) red[threadIdx.x][k] += red[threadIdx.x + s][k];
-    __syncthreads();
+  const int i = threadIdx.x;
+  if (i < TT * OUT) {
+    double v = 0.0;
+    for (int k = 0; k < NW; ++k) v += red[k][i];
+    sum[i] = v;
   }
-  if (threadIdx.x == 0)
+  __syncthreads();
+  if constexpr (SO == 0) {
+    for (int u = 0; u < TT && t0 + u < nt; ++u) {  // uniform over the block
+      const long long t = tg[t0 + u];
+      bool bad = false;
+      for (int k = 0; k < OUT; ++k) bad = bad || sum[u * OUT + k] != sum[u * OUT + k];
+      if (!bad || t < 0 || t >= n) continue;
+      const double xt = pos[3 * t], yt = pos[3 * t + 1], zt = pos[3 * t + 2];
+      double a[OUT];
 #pragma unroll
-    for (int k = 0; k < OUT; ++k) F[(size_t)t * OUT + k] = red[0][k];
+      for (int k = 0; k < OUT; ++k) a[k] = 0.0;
+      for (long long j = threadIdx.x; j < n; j += BS)
+        if (j != t) fmmgen_ops::P2P<double>(xt - pos[3 * j], yt - pos[3 * j + 1], zt - pos[3 * j + 2], S + j, a);
+      fold(a, u);
+      __syncthreads();
+      if (i < OUT) {
+        double v = 0.0;
+        for (int k = 0; k < NW; ++k) v += red[k][u * OUT + i];
+        sum[u * OUT + i] = v;
+      }
+      __syncthreads();
+    }
+  }
+  if (i < TT * OUT && t0 + i / OUT < nt) {
+    const long long t = tg[t0 + i / OUT];
+    F[(size_t)t0 * OUT + i] = t >= 0 && t < n ? sum[i] : __longlong_as_double(0x7ff8000000000000LL);
+  }
 }
 
 __global__ void k_op_p2p(int n, const double* __restrict__ xyz, const double* __restrict__ in, int in_stride,
@@ -779,9 +886,21 @@ void op_batch(int op, int order, int n, const double* xyz, const double* in, int
   OrderTable<PMIN>::op(order, op, n, xyz, in, in_stride, out, out_stride, st);
 }
 
+// Targets per block: four (eight spill beside the registers of two blocks a
+// SIMD, or run at half the waves: 49 and 4.2 ms against 4.1 for 4096 targets x
+// 2^20 charges), fewer targets and more threads where there are too few
+// targets for two blocks a compute unit (300 targets: 1.54 -> 0.87 ms).  Small
+// sets keep one target a block: a wider block's sums cost more than its reads
+// save (2000 particles, 2000 targets: 15.6 us against 18.1).
 void direct(int n, const double* pos, const double* S, const long long* targets, int nt, double* F,
             hipStream_t st) {
-  if (nt > 0) k_direct<<<nt, 256, 0, st>>>(n, pos, S, targets, nt, F);
+  if (nt <= 0) return;
+  auto run = [&](auto kern, int tt, int bs) { kern<<<nblk(nt, tt), bs, 0, st>>>(n, pos, S, targets, nt, F); };
+  if (n < 16384) run(k_direct<1, 256>, 1, 256);
+  else if (nt >= 1024) run(k_direct<4, 512>, 4, 512);
+  else if (nt >= 768) run(k_direct<2, 512>, 2, 512);
+  else if (nt >= 512) run(k_direct<1, 512>, 1, 512);
+  else run(k_direct<1, 1024>, 1, 1024);
 }
 
 }  // namespace FMM_VARIANT_NS
