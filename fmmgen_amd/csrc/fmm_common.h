@@ -143,6 +143,19 @@ struct M2LSchedule {
 };
 constexpr int kGroupsPerChunk = 96;  // measured: 48 -> 96 cut the learned M2L by 11%
 
+// ------------------------------------------------------------ near field
+// P2P work items: the source sequence of a target leaf (own particles, then
+// its merged ranges) cut into segments of at most kSegment source particles,
+// so that a leaf next to a dense cluster is spread over many waves.  Item =
+// (leaf, first range (rb - 1 = own leaf), offset in that range, source count);
+// split leaves accumulate with atomics into a zeroed output.
+struct P2PItems {
+  static constexpr int kSegment = 8192;
+  long long count = 0;
+  int split = 0;  // some leaf has more than one item
+  DevBuf<int> leaf, r, o, n;
+};
+
 // ------------------------------------------------------------ tree handle
 struct Tree {
   // configuration (example/tree.hpp:78-95 + generated macros)
@@ -178,16 +191,11 @@ struct Tree {
   // leaf itself excluded), sorted by start: CSR over cells
   long long n_rng = 0;
   DevBuf<int> rng_off, rng_start, rng_len;
-  // P2P work items: the source sequence of a target leaf (own particles,
-  // then its merged ranges) cut into segments of at most kP2PSegment
-  // source particles, so that a leaf next to a dense cluster is spread
-  // over many waves.  Item = (leaf, first range (rb - 1 = own leaf),
-  // offset in that range, source count); split leaves accumulate with
-  // atomics into a zeroed output.
-  static constexpr int kP2PSegment = 8192;
-  long long n_p2p_items = 0;
-  int p2p_split = 0;  // some leaf has more than one item
-  DevBuf<int> p2p_item_leaf, p2p_item_r, p2p_item_o, p2p_item_n;
+  // P2P work items (p2p_items): of the FP32 near field, whose compensated
+  // sums depend on where a sequence is cut, and of the FP64 one where it is cut
+  // finer (count 0: the same items)
+  P2PItems p2p, p2p64;
+  const P2PItems& p2p_items(bool f64) const { return f64 && p2p64.count > 0 ? p2p64 : p2p; }
   M2LSchedule sched;
 
   // learned order: per leaf features and order, per cell order (the
@@ -258,8 +266,6 @@ struct Tree {
   std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> events;
   std::vector<hipEvent_t> event_pool;
 
-  DevBuf<int> p2p_next;            // work counters of the persistent near-field kernel
-  int num_cu = 0;                  // compute units of the device (queried once)
   double phase_ms[kNumPhaseTimers] = {0};
   long long phase_count[kNumPhaseTimers] = {0};
 };
@@ -289,19 +295,6 @@ __device__ __forceinline__ double sqrt_rn(double s) {
 __device__ inline double norm3_rn(double dx, double dy, double dz) {
 #pragma clang fp contract(off)
   return sqrt_rn(dx * dx + dy * dy + dz * dz);
-}
-
-// Blocks of the persistent near-field kernel: kP2PWavesPerSimd one-wave
-// blocks per SIMD of every compute unit.
-constexpr int kP2PWavesPerSimd = 8;
-inline int p2p_grid(Tree& t) {
-  if (t.num_cu == 0) {
-    int dev = 0;
-    FMM_HIP(hipGetDevice(&dev));
-    FMM_HIP(hipDeviceGetAttribute(&t.num_cu, hipDeviceAttributeMultiprocessorCount, dev));
-    if (t.num_cu <= 0) t.num_cu = 256;
-  }
-  return t.num_cu * 4 * kP2PWavesPerSimd;
 }
 
 // RAII helper: records a start/stop event pair for one phase when timing

@@ -675,16 +675,26 @@ __global__ void k_rng_fill(long long m, int nb, int nc, const unsigned long long
   atomicAdd(&rlen[r], pcount[e.B]);
 }
 
+// Sources of a segment: `seg` (P2PItems::kSegment), or with `even` a
+// leaf's sequence of `tot` in as few segments of at most `seg` as hold it, all
+// of one length, in whole staged chunks of 128.
+__device__ __forceinline__ long long seg_length(long long tot, int seg, int even) {
+  if (!even) return seg;
+  const long long k = (tot + seg - 1) / seg;
+  return ((tot + k - 1) / k + 127) / 128 * 128;
+}
+
 // Per leaf: number of P2P segments; per range: its length as 64-bit.
 __global__ void k_seg_count(int ncells, const int* __restrict__ nchild, const int* __restrict__ pcount,
                             const int* __restrict__ rng_off, const long long* __restrict__ cum,
-                            long long* __restrict__ nseg, int seg) {
+                            long long* __restrict__ nseg, int seg, int even) {
   const int A = blockIdx.x * blockDim.x + threadIdx.x;
   if (A >= ncells) return;
   long long k = 0;
   if (nchild[A] == 0 && pcount[A] > 0) {
     const long long tot = pcount[A] + cum[rng_off[A + 1]] - cum[rng_off[A]];
-    k = (tot + seg - 1) / seg;
+    const long long len = seg_length(tot, seg, even);
+    k = (tot + len - 1) / len;
   }
   nseg[A] = k;
 }
@@ -694,19 +704,19 @@ __global__ void k_widen(long long m, const int* __restrict__ in, long long* __re
   if (i < m) out[i] = in[i];
 }
 
-// Items of one leaf: segment s starts at position s * seg of the source
+// Items of one leaf: segment s starts at position s * len of the source
 // sequence (own particles first, then the ranges in order).
 __global__ void k_seg_fill(int ncells, const int* __restrict__ nchild, const int* __restrict__ pcount,
                            const int* __restrict__ rng_off, const long long* __restrict__ cum,
-                           const long long* __restrict__ nseg, const long long* __restrict__ seg_off, int seg,
+                           const long long* __restrict__ nseg, const long long* __restrict__ seg_off, int seg, int even,
                            int* __restrict__ it_leaf, int* __restrict__ it_r, int* __restrict__ it_o,
                            int* __restrict__ it_n) {
   const int A = blockIdx.x * blockDim.x + threadIdx.x;
   if (A >= ncells || nseg[A] == 0) return;
   const int nt = pcount[A], rb = rng_off[A], re = rng_off[A + 1];
-  const long long base = cum[rb], tot = nt + cum[re] - base;
+  const long long base = cum[rb], tot = nt + cum[re] - base, len = seg_length(tot, seg, even);
   for (long long s = 0; s < nseg[A]; ++s) {
-    const long long P = s * seg, w = seg_off[A] + s;
+    const long long P = s * len, w = seg_off[A] + s;
     int r, o;
     if (P < nt) {
       r = rb - 1;
@@ -726,44 +736,57 @@ __global__ void k_seg_fill(int ncells, const int* __restrict__ nchild, const int
     it_leaf[w] = A;
     it_r[w] = r;
     it_o[w] = o;
-    it_n[w] = (int)((tot - P < seg) ? tot - P : seg);
+    it_n[w] = (int)((tot - P < len) ? tot - P : len);
   }
 }
 
 }  // namespace
 
-// P2P work items (segments of each leaf's source sequence).
+// P2P work items (segments of each leaf's source sequence).  FP32: segments of
+// P2PItems::kSegment.  FP64: the same where they fill the GPU many times over;
+// smaller sets are cut until there are about kP2PItems items, of at least a
+// staged chunk each.  One item a leaf -> this rule, FP64 near field: 2000
+// particles (64 leaves) 144 -> 21 us, 10^5 (4096 leaves) 686 -> 364 us, 300007
+// blobs 2.53 -> 1.41 ms.  (The FP32 items are not cut: the compensated sums of a
+// finer cut differ by 4e-9 of the field.)
+constexpr int kP2PItems = 65536;
 void build_p2p_items(Tree& t, hipStream_t st) {
   const int nc = t.ncells;
   const long long nr = t.n_rng;
   DevBuf<long long> len, cum, nseg, soff;
   len.alloc(nr + 1);
   cum.alloc(nr + 1);
-  FMM_HIP(hipMemsetAsync(len.get(), 0, sizeof(long long) * (nr + 1), st));
+  FMM_HIP(hipMemsetAsync(len.get() + nr, 0, sizeof(long long), st));
   if (nr > 0) k_widen<<<blocks(nr, 256), 256, 0, st>>>(nr, t.rng_len.get(), len.get());
   exclusive_scan_int(t.scratch, len.get(), cum.get(), nr + 1, st);
   nseg.alloc(nc + 1);
   soff.alloc(nc + 1);
-  FMM_HIP(hipMemsetAsync(nseg.get(), 0, sizeof(long long) * (nc + 1), st));
-  const int seg = Tree::kP2PSegment;
-  k_seg_count<<<blocks(nc, 256), 256, 0, st>>>(nc, t.nchild.get(), t.pcount.get(), t.rng_off.get(), cum.get(),
-                                               nseg.get(), seg);
-  exclusive_scan_int(t.scratch, nseg.get(), soff.get(), nc + 1, st);
-  long long total = 0;
-  FMM_HIP(hipMemcpyAsync(&total, soff.get() + nc, sizeof(long long), hipMemcpyDeviceToHost, st));
-  FMM_HIP(hipStreamSynchronize(st));
-  FMM_CHECK(total < (1LL << 31), kOutOfMemory, "P2P work items exceed 2^31");
-  t.n_p2p_items = total;
-  const long long na = std::max<long long>(total, 1);
-  t.p2p_item_leaf.alloc(na);
-  t.p2p_item_r.alloc(na);
-  t.p2p_item_o.alloc(na);
-  t.p2p_item_n.alloc(na);
-  k_seg_fill<<<blocks(nc, 256), 256, 0, st>>>(nc, t.nchild.get(), t.pcount.get(), t.rng_off.get(), cum.get(),
-                                              nseg.get(), soff.get(), seg, t.p2p_item_leaf.get(), t.p2p_item_r.get(),
-                                              t.p2p_item_o.get(), t.p2p_item_n.get());
-  FMM_HIP(hipStreamSynchronize(st));
-  t.p2p_split = total > t.nleaves;
+  auto cut = [&](P2PItems& I, int seg, int even) {
+    FMM_HIP(hipMemsetAsync(nseg.get() + nc, 0, sizeof(long long), st));
+    k_seg_count<<<blocks(nc, 256), 256, 0, st>>>(nc, t.nchild.get(), t.pcount.get(), t.rng_off.get(), cum.get(),
+                                                 nseg.get(), seg, even);
+    exclusive_scan_int(t.scratch, nseg.get(), soff.get(), nc + 1, st);
+    long long total = 0;
+    FMM_HIP(hipMemcpyAsync(&total, soff.get() + nc, sizeof(long long), hipMemcpyDeviceToHost, st));
+    FMM_HIP(hipStreamSynchronize(st));
+    FMM_CHECK(total < (1LL << 31), kOutOfMemory, "P2P work items exceed 2^31");
+    I.count = total;
+    I.split = total > t.nleaves;
+    const long long na = std::max<long long>(total, 1);
+    I.leaf.alloc(na);
+    I.r.alloc(na);
+    I.o.alloc(na);
+    I.n.alloc(na);
+    k_seg_fill<<<blocks(nc, 256), 256, 0, st>>>(nc, t.nchild.get(), t.pcount.get(), t.rng_off.get(), cum.get(),
+                                                nseg.get(), soff.get(), seg, even, I.leaf.get(), I.r.get(),
+                                                I.o.get(), I.n.get());
+  };
+  cut(t.p2p, P2PItems::kSegment, 0);
+  // source sequences in all: the pairs over the mean leaf size
+  const double sources = (double)t.p2p_particle_pairs * t.nleaves / (double)t.n;
+  const long long seg = 128 * (1 + (long long)(sources / (128.0 * kP2PItems)));
+  if (seg < P2PItems::kSegment) cut(t.p2p64, (int)seg, 1);
+  FMM_HIP(hipStreamSynchronize(st));  // the temporaries are freed on return
 }
 
 // Merged source particle ranges of every P2P target (self excluded), from the
@@ -1020,9 +1043,9 @@ void build_lists_device(Tree& t, hipStream_t st) {
   unsigned long long h = 0;
   FMM_HIP(hipMemcpyAsync(&h, total.get(), sizeof(h), hipMemcpyDeviceToHost, st));
   build_p2p_ranges(t, sorted.get(), kb, st);
-  build_p2p_items(t, st);
   FMM_HIP(hipStreamSynchronize(st));
   t.p2p_particle_pairs = (long long)h;
+  build_p2p_items(t, st);
 }
 
 }  // namespace fmm

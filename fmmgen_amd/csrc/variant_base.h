@@ -347,7 +347,21 @@ __device__ __forceinline__ void p2p_pair(int j, int tslot, double xt, double yt,
 #pragma unroll
     for (int k = 0; k < SS; ++k) sj[k] = T(0);
   }
-  fmmgen_ops::P2P<T>(dx, dy, dz, sj, part);
+  if constexpr (SO == 0 && sizeof(T) == 8) charge_pair(dx, dy, dz, sj[0], part);
+  else fmmgen_ops::P2P<T>(dx, dy, dz, sj, part);
+}
+
+// The chunk's sum with the generated body, for a chunk whose charge_pair sum
+// has come out as NaN in some lane.
+template <typename T>
+__device__ __forceinline__ void p2p_chunk_exact(int ns, int filled, int sl, int tslot, double xt, double yt,
+                                                double zt, const double* sx, const double* sy, const double* sz,
+                                                const T* sS, const int* sid, T (&part)[OUT]) {
+#pragma unroll
+  for (int k = 0; k < OUT; ++k) part[k] = T(0);
+#pragma unroll 1
+  for (int j = sl; j < filled; j += ns)
+    if (sid[j] != tslot) fmmgen_ops::P2P<T>((T)(xt - sx[j]), (T)(yt - sy[j]), (T)(zt - sz[j]), sS + j * SS, part);
 }
 
 // Sources sl, sl + NS, sl + 2 NS, ... of a chunk of `filled`: a uniform trip
@@ -378,6 +392,12 @@ __device__ __forceinline__ void p2p_chunk_any(int nslice, int filled, int sl, in
     break;
     FMM_P2P_NS(1) FMM_P2P_NS(2) FMM_P2P_NS(4) FMM_P2P_NS(8) FMM_P2P_NS(16) FMM_P2P_NS(32) FMM_P2P_NS(64)
 #undef FMM_P2P_NS
+  }
+  if constexpr (SO == 0 && sizeof(T) == 8) {
+    bool bad = false;
+#pragma unroll
+    for (int k = 0; k < OUT; ++k) bad = bad || part[k] != part[k];
+    if (__any(bad)) p2p_chunk_exact<T>(nslice, filled, sl, tslot, xt, yt, zt, sx, sy, sz, sS, sid, part);
   }
 }
 
@@ -512,38 +532,31 @@ __device__ __forceinline__ void p2p_item(int it, int nitems, const int* __restri
   }
 }
 
-// Persistent form: a grid of a few waves per SIMD takes work items
-// from eight counters, one per XCD range of items (blocks are dealt to the
-// XCDs round robin, and neighbouring leaves share their sources in that
-// XCD's L2); a block whose range is exhausted takes items of the next
-// XCDs'.  next[8] is zero before the launch.
+// One block an item, dispatched by the hardware as waves free up.  Blocks are
+// dealt to the eight XCDs round robin; runs of kP2PRun items go to one XCD
+// (neighbouring leaves share their sources in its L2) and the runs to the XCDs
+// in turn, so that dense regions are spread over all of them: at 2^22 blobs one
+// eighth of the items per XCD took 13.3 ms (FP32), runs of 256, 64 and 16 items
+// 11.1, 11.1 and 11.0 ms.  (Waves that stay and take items from eight counters
+// took 12.2 ms, and the counters themselves up to half the time of small sets:
+// 10^5 particles 547 us, now 255.)
+// FP64: four waves a SIMD (128 registers) against three, 18.5 -> 17.8 ms.
+constexpr int kP2PRun = 16;
 template <typename T>
-__global__ __launch_bounds__(64) void k_p2p_leaf(int nitems, int* __restrict__ next, const int* __restrict__ it_leaf,
-                                                 const int* __restrict__ it_r, const int* __restrict__ it_o,
-                                                 const int* __restrict__ it_n, const int* __restrict__ pstart,
-                                                 const int* __restrict__ pcount, const int* __restrict__ rng_off,
-                                                 const int* __restrict__ rng_start, const int* __restrict__ rng_len,
-                                                 const double* __restrict__ px, const double* __restrict__ py,
-                                                 const double* __restrict__ pz, const double* __restrict__ pS,
-                                                 int split, double* __restrict__ F) {
-  constexpr bool kKahan = sizeof(T) == 4;
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_p2p_leaf(
+    int nitems, const int* __restrict__ it_leaf, const int* __restrict__ it_r, const int* __restrict__ it_o,
+    const int* __restrict__ it_n, const int* __restrict__ pstart, const int* __restrict__ pcount,
+    const int* __restrict__ rng_off, const int* __restrict__ rng_start, const int* __restrict__ rng_len,
+    const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
+    const double* __restrict__ pS, int split, double* __restrict__ F) {
   __shared__ double sx[kP2PChunk], sy[kP2PChunk], sz[kP2PChunk];
   __shared__ T sS[kP2PChunk * SS];
   __shared__ int sid[kP2PChunk];
-  const int lane = threadIdx.x;
-  const int per = (nitems + 7) / 8;
-  for (int k = 0; k < 8; ++k) {
-    const int x = (blockIdx.x + k) & 7;
-    const int lo = x * per, hi = min(nitems, lo + per);
-    for (;;) {
-      int got = 0;
-      if (lane == 0) got = atomicAdd(&next[x], 1);
-      const int it = lo + __shfl(got, 0, 64);
-      if (it >= hi) break;
-      p2p_item<T>(it, nitems, it_leaf, it_r, it_o, it_n, pstart, pcount, rng_off, rng_start, rng_len, px, py, pz,
-                  pS, split, F, sx, sy, sz, sS, sid);
-    }
-  }
+  const int k = blockIdx.x >> 3;
+  const int it = ((k / kP2PRun) * 8 + (int)(blockIdx.x & 7)) * kP2PRun + k % kP2PRun;
+  if (it < nitems)
+    p2p_item<T>(it, nitems, it_leaf, it_r, it_o, it_n, pstart, pcount, rng_off, rng_start, rng_len, px, py, pz, pS,
+                split, F, sx, sy, sz, sS, sid);
 }
 
 __global__ void k_fill_zero(long long n, double* __restrict__ a) {
@@ -552,21 +565,19 @@ __global__ void k_fill_zero(long long n, double* __restrict__ a) {
 }
 
 void near_field(Tree& t, int mode, hipStream_t st) {
-  const int ni = (int)t.n_p2p_items;
+  const P2PItems& I = t.p2p_items(mode == 0);
+  const int ni = (int)I.count;
   PhaseTimer pt(t, kTP2P, st);
-  if (t.p2p_split) {
+  if (I.split) {
     const long long m = (long long)t.n * OUT;
     k_fill_zero<<<(int)((m + 255) / 256), 256, 0, st>>>(m, t.Fp2p.get());
   }
   if (ni == 0) return;
-  t.p2p_next.alloc(8);
-  k_fill_int<<<1, 64, 0, st>>>(8, t.p2p_next.get());
-  const int grid = std::min(ni, p2p_grid(t));
+  const int grid = nblk(ni, 8 * kP2PRun) * 8 * kP2PRun;
   auto launch = [&](auto kern) {
-    kern<<<grid, 64, 0, st>>>(ni, t.p2p_next.get(), t.p2p_item_leaf.get(), t.p2p_item_r.get(), t.p2p_item_o.get(),
-                              t.p2p_item_n.get(), t.pstart.get(), t.pcount.get(), t.rng_off.get(),
-                              t.rng_start.get(), t.rng_len.get(), t.px.get(), t.py.get(), t.pz.get(), t.pS.get(),
-                              t.p2p_split, t.Fp2p.get());
+    kern<<<grid, 64, 0, st>>>(ni, I.leaf.get(), I.r.get(), I.o.get(), I.n.get(), t.pstart.get(), t.pcount.get(),
+                              t.rng_off.get(), t.rng_start.get(), t.rng_len.get(), t.px.get(), t.py.get(),
+                              t.pz.get(), t.pS.get(), I.split, t.Fp2p.get());
   };
   if (mode == 0) launch(k_p2p_leaf<double>);
   else launch(k_p2p_leaf<float>);
