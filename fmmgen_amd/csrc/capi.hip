@@ -129,6 +129,8 @@ int fmm_tree_build(const double* d_pos, const double* d_S, size_t n, size_t ncri
       t.theta = theta;
       t.n = n;
       t.user_S = d_S;
+      FMM_HIP(hipGetDevice(&t.device));
+      MemScope scope(st);
       build_tree_device(t, d_pos, st);
       build_lists_device(t, st);
       build_m2l_schedule(t, st);
@@ -142,18 +144,27 @@ int fmm_tree_build(const double* d_pos, const double* d_S, size_t n, size_t ncri
 
 int fmm_tree_destroy(fmm_tree_t tree) {
   return guarded([&] {
-    if (tree) {
-      (void)hipDeviceSynchronize();
-      for (auto& e : tree->t.events) {
-        (void)hipEventDestroy(e.second.first);
-        (void)hipEventDestroy(e.second.second);
-      }
-      for (auto e : tree->t.event_pool) (void)hipEventDestroy(e);
-      if (tree->t.side) (void)hipStreamDestroy(tree->t.side);
-      if (tree->t.side_fork) (void)hipEventDestroy(tree->t.side_fork);
-      if (tree->t.side_join) (void)hipEventDestroy(tree->t.side_join);
+    if (!tree) return;
+    const int own = tree->t.device;
+    int dev = own;
+    (void)hipGetDevice(&dev);
+    if (dev != own) (void)hipSetDevice(own);
+    const bool idle = hipDeviceSynchronize() == hipSuccess;
+    for (auto& e : tree->t.events) {
+      (void)hipEventDestroy(e.second.first);
+      (void)hipEventDestroy(e.second.second);
     }
-    delete tree;
+    for (auto e : tree->t.event_pool) (void)hipEventDestroy(e);
+    if (tree->t.side) (void)hipStreamDestroy(tree->t.side);
+    if (tree->t.side_fork) (void)hipEventDestroy(tree->t.side_fork);
+    if (tree->t.side_join) (void)hipEventDestroy(tree->t.side_join);
+    if (idle) {
+      MemScope scope(nullptr);  // nothing is pending: the buffers are kept for later trees
+      delete tree;
+    } else {
+      delete tree;
+    }
+    if (dev != own) (void)hipSetDevice(dev);
   });
 }
 
@@ -477,6 +488,7 @@ int fmm_tree_set_model(fmm_tree_t tree, const float* d_params, double tol, doubl
     Tree& t = tree->t;
     // no evaluation on any stream may still read the buffers re-formed here
     FMM_HIP(hipDeviceSynchronize());
+    MemScope scope(nullptr);
     t.mlp_half.alloc(kMlpParams);
     mlp_to_half(d_params, t.mlp_half.get(), nullptr);
     FMM_HIP(hipStreamSynchronize(nullptr));

@@ -122,11 +122,11 @@ const unsigned* ensure_index_table(Tree& t, hipStream_t st) {
   M2LSchedule& S = t.sched;
   const int wi = W == 8 ? 1 : (W == 2 ? 2 : 0);
   if (!S.idx_ready[LAY][P][wi]) {
-    const std::vector<unsigned> tab = m2l_index_table<P, SO, W, LAY>();
+    static const std::vector<unsigned> tab = m2l_index_table<P, SO, W, LAY>();  // once per process
     S.idxtab[LAY][P][wi].alloc(tab.size());
     FMM_HIP(hipMemcpyAsync(S.idxtab[LAY][P][wi].get(), tab.data(), sizeof(unsigned) * tab.size(),
                            hipMemcpyHostToDevice, st));
-    FMM_HIP(hipStreamSynchronize(st));
+    FMM_HIP(hipStreamSynchronize(st));  // evaluations on other streams may follow
     S.idx_ready[LAY][P][wi] = true;
   }
   return S.idxtab[LAY][P][wi].get();
@@ -155,11 +155,11 @@ template <int P, int W, int LAY = kGraded>
 const unsigned* ensure_index_table32(Tree& t, hipStream_t st) {
   M2LSchedule& S = t.sched;
   if (!S.idx32_ready[LAY][P]) {
-    const std::vector<unsigned> tab = m2l_index_table32<P, SO, W, LAY>();
+    static const std::vector<unsigned> tab = m2l_index_table32<P, SO, W, LAY>();  // once per process
     S.idxtab32[LAY][P].alloc(tab.size());
     FMM_HIP(hipMemcpyAsync(S.idxtab32[LAY][P].get(), tab.data(), sizeof(unsigned) * tab.size(),
                            hipMemcpyHostToDevice, st));
-    FMM_HIP(hipStreamSynchronize(st));
+    FMM_HIP(hipStreamSynchronize(st));  // evaluations on other streams may follow
     S.idx32_ready[LAY][P] = true;
   }
   return S.idxtab32[LAY][P].get();
