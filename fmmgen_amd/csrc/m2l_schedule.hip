@@ -163,11 +163,10 @@ __global__ void k_fill_groups(long long m, int kb, int ntiles, const unsigned lo
 }
 
 // Work items of a tile: its groups cut into equal runs of at most
-// kGroupsPerChunk; nch[ntiles] = 0, so that the scan's last entry is their
-// number.
-__global__ void k_chunk_count(int ntiles, const int* __restrict__ goff, int* __restrict__ nch) {
+// len; nch[ntiles] = 0, so that the scan's last entry is their number.
+__global__ void k_chunk_count(int ntiles, int len, const int* __restrict__ goff, int* __restrict__ nch) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t <= ntiles) nch[t] = t < ntiles ? (goff[t + 1] - goff[t] + kGroupsPerChunk - 1) / kGroupsPerChunk : 0;
+  if (t <= ntiles) nch[t] = t < ntiles ? (goff[t + 1] - goff[t] + len - 1) / len : 0;
 }
 __global__ void k_chunk_fill(int ntiles, const int* __restrict__ goff, const int* __restrict__ nch,
                              const int* __restrict__ first, int* __restrict__ tile, int* __restrict__ g0,
@@ -307,7 +306,8 @@ void build_m2l_schedule(Tree& t, hipStream_t st) {
   DevBuf<int> nch, first;
   nch.alloc(S.ntiles + 1);
   first.alloc(S.ntiles + 1);
-  k_chunk_count<<<blocks(S.ntiles + 1, 256), 256, 0, st>>>(S.ntiles, S.tile_group_off.get(), nch.get());
+  const int len = std::max(kGroupsPerChunkMin, std::min(kGroupsPerChunk, S.ngroups / kChunkTarget));
+  k_chunk_count<<<blocks(S.ntiles + 1, 256), 256, 0, st>>>(S.ntiles, len, S.tile_group_off.get(), nch.get());
   scan_ex(t.scratch, nch.get(), first.get(), S.ntiles + 1, st);
   S.nchunks = read_int(first.get() + S.ntiles, st);
   S.chunk_tile.alloc(S.nchunks);
