@@ -5,6 +5,7 @@
 #include <algorithm>
 
 #include "learned.h"
+#include "pair.h"
 #include "variant_decl.h"
 
 namespace fmm {
@@ -19,41 +20,11 @@ __global__ void k_gather_S(int n, const int* __restrict__ perm, const double* __
   for (int k = 0; k < SS; ++k) pS[(size_t)j * SS + k] = S[(size_t)i * SS + k];
 }
 
-// One charge pair in FP64 (the example's P2P, example/calculate.cpp:24-40):
-// q/r and q r^-3 (dx, dy, dz) from the hardware estimate y of x^(-1/2), x = r^2,
-// corrected by the series of (1 - e)^(-1/2), e = 1 - x y^2, which cubes the
-// estimate's relative error.  No case of x is treated apart: where x or a power
-// of y leaves the finite range (coincident particles above all) the result is
-// NaN, and the callers repeat such sums with the generated body.  19
-// instructions and the estimate, against 23 in the generated body (its select
-// of zero and infinite x).
-__device__ __forceinline__ void charge_pair(double dx, double dy, double dz, double q, double* acc) {
-  const double x = fma(dx, dx, fma(dy, dy, dz * dz));
-  const double y = __builtin_amdgcn_rsq(x);
-  const double y2 = y * y;
-  const double e = fma(-x, y2, 1.0);
-  double s3;
-  if constexpr (OUT == 3) {
-    const double q3 = q * (y2 * y), t = q3 * e;
-    s3 = fma(t * e, 1.875, fma(t, 1.5, q3));
-  } else {
-    const double r = fma(y * e, fma(e, 0.375, 0.5), y), s = q * r;
-    acc[0] += s;
-    s3 = s * (r * r);
-  }
-  if constexpr (OUT != 1) {
-    constexpr int F0 = OUT == 4 ? 1 : 0;
-    acc[F0] = fma(s3, dx, acc[F0]);
-    acc[F0 + 1] = fma(s3, dy, acc[F0 + 1]);
-    acc[F0 + 2] = fma(s3, dz, acc[F0 + 2]);
-  }
-}
-
 // FP64 direct sum on sampled targets (example/calculate.cpp:252-264): a block
 // holds TT targets in registers, so that each source read serves TT pairs, and
 // strides its BS threads over the sources, the next source loaded during the
 // pairs of this one; wave sums, then a sum over the waves, in a fixed order.
-// Charges take charge_pair, the target itself as a zero charge at unit
+// Pairs take source_pair, the target itself as a zero source at unit
 // distance; a row that comes out as NaN is summed again with the generated
 // body.  Bound by the FP64 pairs: 4096 targets x 2^20 charges 6.9 ms with one
 // target a block, 4.1 ms with four.
@@ -91,24 +62,21 @@ __global__ __launch_bounds__(BS, 4) void k_direct(int n, const double* __restric
     for (int k = 0; k < SS; ++k) s[k] = ns[k];
     load(j + BS);
     if (j >= (unsigned)n) continue;
-    if constexpr (SO == 0) {
-      bool own = false;  // uniform: this step holds a target of the block
+    bool own = false;  // uniform: this step holds a target of the block
 #pragma unroll
-      for (int u = 0; u < TT; ++u) own = own || (unsigned)ti[u] - b < (unsigned)BS;
-      if (own) {
+    for (int u = 0; u < TT; ++u) own = own || (unsigned)ti[u] - b < (unsigned)BS;
+    if (own) {
 #pragma unroll
-        for (int u = 0; u < TT; ++u) {
-          const bool self = j == (unsigned)ti[u];
-          charge_pair(self ? 1.0 : tx[u] - x, ty[u] - y, tz[u] - z, self ? 0.0 : s[0], acc[u]);
-        }
-      } else {
+      for (int u = 0; u < TT; ++u) {
+        const bool self = j == (unsigned)ti[u];
+        double w[SS];
 #pragma unroll
-        for (int u = 0; u < TT; ++u) charge_pair(tx[u] - x, ty[u] - y, tz[u] - z, s[0], acc[u]);
+        for (int k = 0; k < SS; ++k) w[k] = self ? 0.0 : s[k];
+        source_pair<double>(self ? 1.0 : tx[u] - x, ty[u] - y, tz[u] - z, w, acc[u]);
       }
     } else {
 #pragma unroll
-      for (int u = 0; u < TT; ++u)
-        if (j != (unsigned)ti[u]) fmmgen_ops::P2P<double>(tx[u] - x, ty[u] - y, tz[u] - z, s, acc[u]);
+      for (int u = 0; u < TT; ++u) source_pair<double>(tx[u] - x, ty[u] - y, tz[u] - z, s, acc[u]);
     }
   }
   constexpr int NW = BS / 64;
@@ -133,27 +101,25 @@ __global__ __launch_bounds__(BS, 4) void k_direct(int n, const double* __restric
     sum[i] = v;
   }
   __syncthreads();
-  if constexpr (SO == 0) {
-    for (int u = 0; u < TT && t0 + u < nt; ++u) {  // uniform over the block
-      const long long t = tg[t0 + u];
-      bool bad = false;
-      for (int k = 0; k < OUT; ++k) bad = bad || sum[u * OUT + k] != sum[u * OUT + k];
-      if (!bad || t < 0 || t >= n) continue;
-      const double xt = pos[3 * t], yt = pos[3 * t + 1], zt = pos[3 * t + 2];
-      double a[OUT];
+  for (int u = 0; u < TT && t0 + u < nt; ++u) {  // uniform over the block
+    const long long t = tg[t0 + u];
+    bool bad = false;
+    for (int k = 0; k < OUT; ++k) bad = bad || sum[u * OUT + k] != sum[u * OUT + k];
+    if (!bad || t < 0 || t >= n) continue;
+    const double xt = pos[3 * t], yt = pos[3 * t + 1], zt = pos[3 * t + 2];
+    double a[OUT];
 #pragma unroll
-      for (int k = 0; k < OUT; ++k) a[k] = 0.0;
-      for (long long j = threadIdx.x; j < n; j += BS)
-        if (j != t) fmmgen_ops::P2P<double>(xt - pos[3 * j], yt - pos[3 * j + 1], zt - pos[3 * j + 2], S + j, a);
-      fold(a, u);
-      __syncthreads();
-      if (i < OUT) {
-        double v = 0.0;
-        for (int k = 0; k < NW; ++k) v += red[k][u * OUT + i];
-        sum[u * OUT + i] = v;
-      }
-      __syncthreads();
+    for (int k = 0; k < OUT; ++k) a[k] = 0.0;
+    for (long long j = threadIdx.x; j < n; j += BS)
+      if (j != t) fmmgen_ops::P2P<double>(xt - pos[3 * j], yt - pos[3 * j + 1], zt - pos[3 * j + 2], S + j * SS, a);
+    fold(a, u);
+    __syncthreads();
+    if (i < OUT) {
+      double v = 0.0;
+      for (int k = 0; k < NW; ++k) v += red[k][u * OUT + i];
+      sum[u * OUT + i] = v;
     }
+    __syncthreads();
   }
   if (i < TT * OUT && t0 + i / OUT < nt) {
     const long long t = tg[t0 + i / OUT];
@@ -328,7 +294,7 @@ __global__ void k_fill_int(long long n, int* __restrict__ a) {
 // lanes idle than with one pow2(r) piece (40 of 64 lanes busy for r = 40).
 //   T = double: FP64 throughout (the reference arithmetic).
 //   T = float : dx = float(x_t - x_s) from FP64 positions (no cancellation
-//               loss for close pairs), the generated P2P body in FP32, and
+//               loss for close pairs), the pair in FP32 (source_pair), and
 //               compensated (Kahan) accumulation of each chunk's partial
 //               sum into the running total.
 // The result is written in FP64 per sorted slot.
@@ -347,12 +313,11 @@ __device__ __forceinline__ void p2p_pair(int j, int tslot, double xt, double yt,
 #pragma unroll
     for (int k = 0; k < SS; ++k) sj[k] = T(0);
   }
-  if constexpr (SO == 0 && sizeof(T) == 8) charge_pair(dx, dy, dz, sj[0], part);
-  else fmmgen_ops::P2P<T>(dx, dy, dz, sj, part);
+  source_pair<T>(dx, dy, dz, sj, part);
 }
 
-// The chunk's sum with the generated body, for a chunk whose charge_pair sum
-// has come out as NaN in some lane.
+// The chunk's sum with the generated body, for a chunk whose FP64 source_pair
+// sum has come out as NaN in some lane.
 template <typename T>
 __device__ __forceinline__ void p2p_chunk_exact(int ns, int filled, int sl, int tslot, double xt, double yt,
                                                 double zt, const double* sx, const double* sy, const double* sz,
@@ -393,7 +358,7 @@ __device__ __forceinline__ void p2p_chunk_any(int nslice, int filled, int sl, in
     FMM_P2P_NS(1) FMM_P2P_NS(2) FMM_P2P_NS(4) FMM_P2P_NS(8) FMM_P2P_NS(16) FMM_P2P_NS(32) FMM_P2P_NS(64)
 #undef FMM_P2P_NS
   }
-  if constexpr (SO == 0 && sizeof(T) == 8) {
+  if constexpr (sizeof(T) == 8) {
     bool bad = false;
 #pragma unroll
     for (int k = 0; k < OUT; ++k) bad = bad || part[k] != part[k];
