@@ -12,6 +12,7 @@
 
 #include "m2l_gemm.h"
 #include "variant_decl.h"
+#include "wave_ops.h"
 
 namespace fmm {
 namespace FMM_VARIANT_NS {
@@ -64,6 +65,89 @@ __global__ __launch_bounds__(64) void k_p2m(int nleaves, const int* __restrict__
 #pragma unroll
     for (int k = 0; k < HI - LO; ++k) Mc[LO + k] = acc.v[k];
   });
+}
+
+// The same for charges with one wave a leaf: lanes own slots, and 32 particles
+// at a time stage q and u^k / k! (k <= P) in LDS, M_n += q X Y Z.  A thread a
+// (leaf, chunk) leaves most of the chip idle on small sets and loops each lane
+// over its own leaf: 2000 particles, order 4 17.5 -> 5.5 us; 2^20, order 8 117 ->
+// 82 us.  Bound by the three LDS reads a slot and particle.
+template <int P>
+__global__ __launch_bounds__(64) void k_p2m_leaf(int nleaves, const int* __restrict__ leaves, const int* __restrict__ pstart,
+                      const int* __restrict__ pcount, const double* __restrict__ cx, const double* __restrict__ cy,
+                      const double* __restrict__ cz, const double* __restrict__ px, const double* __restrict__ py,
+                      const double* __restrict__ pz, const double* __restrict__ pS, double* __restrict__ M) {
+  static_assert(SO == 0 || P < 0, "charges only");
+  constexpr int MS = Op<P>::MS, NPL = (MS + 63) / 64, NB = 32, PW = (3 * (P + 1)) | 1;
+  __shared__ double pw[NB * PW];  // particle k: q X[0..P], Y[0..P], Z[0..P]
+  const int lane = threadIdx.x, c = leaves[blockIdx.x];
+  const double x0 = cx[c], y0 = cy[c], z0 = cz[c];
+  int ea[NPL], eb[NPL], ec[NPL];
+  double acc[NPL];
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) {
+    const MultiIdx m = slot_multi_rt(min(lane + 64 * i, MS - 1));
+    ea[i] = m.x;
+    eb[i] = P + 1 + m.y;
+    ec[i] = 2 * (P + 1) + m.z;
+    acc[i] = 0.0;
+  }
+  const int b = pstart[c], e = b + pcount[c];
+  for (int base = b; base < e; base += NB) {
+    const int nk = min(NB, e - base);
+    wave_lds_fence();  // previous particles consumed
+    for (int t = lane; t < 3 * nk; t += 64) {  // one (particle, axis) a lane
+      const int k = t / 3, d = t - 3 * k, j = base + k;
+      const double u = d == 0 ? x0 - px[j] : d == 1 ? y0 - py[j] : z0 - pz[j];
+      double v = d == 0 ? pS[j] : 1.0;
+      double* o = pw + k * PW + d * (P + 1);
+      o[0] = v;
+      static_for<P>([&](auto K) {
+        v *= u * (1.0 / (K + 1));
+        o[K + 1] = v;
+      });
+    }
+    wave_lds_fence();
+    for (int k = 0; k < nk; ++k) {
+      const double* w = pw + k * PW;
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) acc[i] = fma(w[ea[i]] * w[eb[i]], w[ec[i]], acc[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NPL; ++i)
+    if (lane + 64 * i < MS) M[(size_t)c * MS + lane + 64 * i] = acc[i];
+}
+
+// M2M of the levels of few parents: a block a parent, a wave a child.  Each wave
+// shifts its child's multipole along the three axes in LDS (at most P + 1 terms
+// a slot and axis), and the block adds the children in order.  A thread a
+// (parent, chunk) takes the children one after the other: 10^5 particles, order 4
+// 8.5 -> 4.7 us a level; levels of up to 512 parents, order 8 29 -> 10 us.  From
+// 4096 parents on its generated bodies, the chip full, are as fast (37 us).
+constexpr int kM2MWaveParents = 1024;
+template <int P>
+__global__ __launch_bounds__(512) void k_m2m_wave(int beg, const int* __restrict__ first_child, const int* __restrict__ nchild,
+                      const double* __restrict__ cx, const double* __restrict__ cy, const double* __restrict__ cz,
+                      double* __restrict__ M) {
+  constexpr int MS = Op<P>::MS, NT = nterms(P), OFF = NT - MS;
+  __shared__ double sA[8][NT], sB[8][NT], sP[8][3 * (P + 1)];
+  const int p = beg + blockIdx.x, k = nchild[p];
+  if (k == 0) return;  // uniform over the block
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (w < k) {
+    const int c = first_child[p] + w;
+    for (int j = lane; j < NT; j += 64) sA[w][j] = j >= OFF ? M[(size_t)c * MS + j - OFF] : 0.0;
+    wave_powers<P>(lane, cx[p] - cx[c], cy[p] - cy[c], cz[p] - cz[c], sP[w]);
+    wave_lds_fence();
+    wave_shift3<P, true>(lane, sA[w], sB[w], sP[w]);
+  }
+  __syncthreads();
+  for (int j = threadIdx.x; j < MS; j += 512) {
+    double v = 0.0;
+    for (int c = 0; c < k; ++c) v += sB[c][j + OFF];
+    M[(size_t)p * MS + j] = v;
+  }
 }
 
 // M2M (example/calculate.cpp:163-187), x = parent - child, one thread per
@@ -329,14 +413,22 @@ void far_field_order(Tree& t, int mode, int mask, hipStream_t st) {
   const int nc = t.ncells;
   if (mask & kPhaseP2M) {
     PhaseTimer pt(t, kTP2M, st);
-    k_p2m<P><<<dim3(nblk(t.nleaves, 64), (Op<P>::MS + kChunk - 1) / kChunk), 64, 0, st>>>(t.nleaves, t.leaves.get(), t.pstart.get(), t.pcount.get(),
-                                                 t.cx.get(), t.cy.get(), t.cz.get(), t.px.get(), t.py.get(),
-                                                 t.pz.get(), t.pS.get(), t.M.get());
+    auto run = [&](auto kern, dim3 grid) {
+      kern<<<grid, 64, 0, st>>>(t.nleaves, t.leaves.get(), t.pstart.get(), t.pcount.get(), t.cx.get(), t.cy.get(),
+                                t.cz.get(), t.px.get(), t.py.get(), t.pz.get(), t.pS.get(), t.M.get());
+    };
+    if constexpr (SO == 0) run(k_p2m_leaf<P>, t.nleaves);
+    else run(k_p2m<P>, dim3(nblk(t.nleaves, 64), (Op<P>::MS + kChunk - 1) / kChunk));
   }
   if (mask & kPhaseM2M) {
     PhaseTimer pt(t, kTM2M, st);
     for (int l = t.depth - 2; l >= 0; --l) {
       const int b = t.level_off[l], e = t.level_off[l + 1];
+      if (e - b <= kM2MWaveParents) {
+        k_m2m_wave<P><<<e - b, 512, 0, st>>>(b, t.first_child.get(), t.nchild.get(), t.cx.get(), t.cy.get(),
+                                             t.cz.get(), t.M.get());
+        continue;
+      }
       k_m2m<P><<<dim3(nblk(e - b, 64), (Op<P>::MS + kChunk - 1) / kChunk), 64, 0, st>>>(b, e, t.first_child.get(), t.nchild.get(), t.cx.get(),
                                                t.cy.get(), t.cz.get(), t.M.get());
     }
