@@ -295,6 +295,7 @@ struct Tree {
   int m2l_form = 0;
   DevBuf<float> Mhf, Lhf;
   DevBuf<double> Mh64, Lh64;
+  DevBuf<double> Qbh;             // Barnes-Hut: solid-harmonic coefficient rows of every cell (bh.h)
   DevBuf<double> Mtop, Ltop;
   DevBuf<double> Fp2p;            // per-target near-field result, sorted order
   Scratch scratch;
