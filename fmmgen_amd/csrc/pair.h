@@ -17,7 +17,6 @@ __device__ __forceinline__ double inv_norm(double x) {
   const double e = fma(-x, y * y, 1.0);
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
-__device__ __forceinline__ float inv_norm(float x) { return __builtin_amdgcn_rsqf(x); }
 
 // One charge pair in FP64: q/r and q r^-3 (dx, dy, dz).  19 instructions and the
 // estimate, against 23 in the generated body (its select of zero and infinite
@@ -50,32 +49,30 @@ __device__ __forceinline__ void charge_pair(double dx, double dy, double dz, dou
 //   quadrupole  phi = r^-3 (3 Q - T),         F = 3 r^-4 ((5 Q - T) u - v),
 //               v = grad of u.S.u, Q = u.S.u = u.v / 2, T = trace S.
 // No second and third derivatives one by one as in the generated bodies.  200000
-// uniform particles, near field FP64 | FP32: dipoles 3.99 -> 1.66 | 2.55 -> 1.68
-// ms, quadrupoles 7.18 -> 2.48 | 4.45 -> 2.21 ms; 4096 targets x 2^18 sources:
-// dipoles 2.73 -> 1.43 ms, quadrupoles 6.02 -> 4.34 ms.
-template <typename T>
-__device__ __forceinline__ void multipole_pair(T dx, T dy, T dz, const T* S, T* acc) {
-  static_assert(SO == 1 || SO == 2, "dipoles and quadrupoles");
+// uniform particles, FP64 near field: dipoles 3.99 -> 1.66 ms, quadrupoles 7.18 ->
+// 2.48 ms; 4096 targets x 2^18 sources: dipoles 2.73 -> 1.43 ms, quadrupoles 6.02
+// -> 4.34 ms.
+__device__ __forceinline__ void multipole_pair(double dx, double dy, double dz, const double* S, double* acc) {
   constexpr int F0 = OUT == 4 ? 1 : 0;
-  const T r = inv_norm(fma(dx, dx, fma(dy, dy, dz * dz)));
-  const T x = dx * r, y = dy * r, z = dz * r, r2 = r * r, r3 = r2 * r;
+  const double r = inv_norm(fma(dx, dx, fma(dy, dy, dz * dz)));
+  const double x = dx * r, y = dy * r, z = dz * r, r2 = r * r, r3 = r2 * r;
   if constexpr (SO == 1) {
-    const T s = fma(S[0], x, fma(S[1], y, S[2] * z));
+    const double s = fma(S[0], x, fma(S[1], y, S[2] * z));
     if constexpr (OUT != 3) acc[0] = fma(-r2, s, acc[0]);
     if constexpr (OUT != 1) {
-      const T t = T(-3) * s;
+      const double t = -3.0 * s;
       acc[F0] = fma(r3, fma(t, x, S[0]), acc[F0]);
       acc[F0 + 1] = fma(r3, fma(t, y, S[1]), acc[F0 + 1]);
       acc[F0 + 2] = fma(r3, fma(t, z, S[2]), acc[F0 + 2]);
     }
   } else {
-    const T vx = fma(S[0] + S[0], x, fma(S[1], y, S[2] * z));
-    const T vy = fma(S[1], x, fma(S[3] + S[3], y, S[4] * z));
-    const T vz = fma(S[2], x, fma(S[4], y, (S[5] + S[5]) * z));
-    const T q = fma(x, vx, fma(y, vy, z * vz)), tr = S[0] + S[3] + S[5];
-    if constexpr (OUT != 3) acc[0] = fma(r3, fma(T(1.5), q, -tr), acc[0]);
+    const double vx = fma(S[0] + S[0], x, fma(S[1], y, S[2] * z));
+    const double vy = fma(S[1], x, fma(S[3] + S[3], y, S[4] * z));
+    const double vz = fma(S[2], x, fma(S[4], y, (S[5] + S[5]) * z));
+    const double q = fma(x, vx, fma(y, vy, z * vz)), tr = S[0] + S[3] + S[5];
+    if constexpr (OUT != 3) acc[0] = fma(r3, fma(1.5, q, -tr), acc[0]);
     if constexpr (OUT != 1) {
-      const T a = T(3) * (r3 * r), b = fma(T(2.5), q, -tr);
+      const double a = 3.0 * (r3 * r), b = fma(2.5, q, -tr);
       acc[F0] = fma(a, fma(b, x, -vx), acc[F0]);
       acc[F0 + 1] = fma(a, fma(b, y, -vy), acc[F0 + 1]);
       acc[F0 + 2] = fma(a, fma(b, z, -vz), acc[F0 + 2]);
@@ -84,12 +81,14 @@ __device__ __forceinline__ void multipole_pair(T dx, T dy, T dz, const T* S, T* 
 }
 
 // The pair of the near field, the direct sum and the Barnes-Hut leaves.  FP32
-// charges take the generated body (no shorter form).
+// pairs take the generated body: charges have no shorter form, and the closed
+// dipole form rounds otherwise (8e-8 of the field apart; 3.97 instead of 5.70 ms
+// at 10^6 Plummer dipoles).
 template <typename T>
 __device__ __forceinline__ void source_pair(T dx, T dy, T dz, const T* S, T* acc) {
-  if constexpr (SO == 0 && sizeof(T) == 8) charge_pair(dx, dy, dz, S[0], acc);
-  else if constexpr (SO == 0) fmmgen_ops::P2P<T>(dx, dy, dz, S, acc);
-  else multipole_pair<T>(dx, dy, dz, S, acc);
+  if constexpr (sizeof(T) == 4) fmmgen_ops::P2P<T>(dx, dy, dz, S, acc);
+  else if constexpr (SO == 0) charge_pair(dx, dy, dz, S[0], acc);
+  else multipole_pair(dx, dy, dz, S, acc);
 }
 
 }  // namespace FMM_VARIANT_NS
