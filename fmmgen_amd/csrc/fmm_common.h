@@ -173,14 +173,16 @@ struct M2LSchedule {
   bool tile_pairs_ready = false;
   DevBuf<int> cell_tile;         // cell -> its M2L tile (-1: none)
   bool cell_tile_ready = false;
-  // work items: chunks of at most kGroupsPerChunk groups of one tile
-  int nchunks = 0;
+  // work items: chunks of at most kGroupsPerChunk groups of one tile; of the
+  // FP64 M2L where it is cut finer (nchunks64 0: the same ones)
+  int nchunks = 0, nchunks64 = 0;
   DevBuf<int> chunk_tile, chunk_g0, chunk_g1;
+  DevBuf<int> chunk64_tile, chunk64_g0, chunk64_g1;
 };
 constexpr int kGroupsPerChunk = 96;  // measured: 48 -> 96 cut the learned M2L by 11%
-// Sets with fewer than kChunkTarget such chunks are cut finer, so that the chip
-// fills: M2L of 2000 particles at order 4 (383 groups) 50 -> 8 us, of 10^5 (156k
-// groups) 151 -> 134 us.
+// The FP64 M2L of sets with fewer than kChunkTarget such chunks is cut finer, so
+// that the chip fills: 2000 particles at order 4 (383 groups) 50 -> 8 us, 10^5
+// (156k groups) 151 -> 134 us.  FP32 sums depend on where a tile is cut.
 constexpr int kChunkTarget = 4096, kGroupsPerChunkMin = 2;
 
 // ------------------------------------------------------------ near field

@@ -248,7 +248,7 @@ void build_m2l_schedule(Tree& t, hipStream_t st) {
     S.tile_cells.alloc((size_t)std::max(S.ntiles, 1) * kTile);
     S.tile_group_off.alloc(S.ntiles + 1);
     if (m == 0) {
-      S.ngroups = S.nkeys = S.nchunks = 0;
+      S.ngroups = S.nkeys = S.nchunks = S.nchunks64 = 0;
       FMM_HIP(hipMemsetAsync(S.tile_group_off.get(), 0, sizeof(int) * (S.ntiles + 1), st));
       FMM_HIP(hipStreamSynchronize(st));
       return;
@@ -306,15 +306,20 @@ void build_m2l_schedule(Tree& t, hipStream_t st) {
   DevBuf<int> nch, first;
   nch.alloc(S.ntiles + 1);
   first.alloc(S.ntiles + 1);
-  const int len = std::max(kGroupsPerChunkMin, std::min(kGroupsPerChunk, S.ngroups / kChunkTarget));
-  k_chunk_count<<<blocks(S.ntiles + 1, 256), 256, 0, st>>>(S.ntiles, len, S.tile_group_off.get(), nch.get());
-  scan_ex(t.scratch, nch.get(), first.get(), S.ntiles + 1, st);
-  S.nchunks = read_int(first.get() + S.ntiles, st);
-  S.chunk_tile.alloc(S.nchunks);
-  S.chunk_g0.alloc(S.nchunks);
-  S.chunk_g1.alloc(S.nchunks);
-  k_chunk_fill<<<blocks(S.ntiles, 256), 256, 0, st>>>(S.ntiles, S.tile_group_off.get(), nch.get(), first.get(),
-                                                      S.chunk_tile.get(), S.chunk_g0.get(), S.chunk_g1.get());
+  auto cut = [&](int len, int& count, DevBuf<int>& tile, DevBuf<int>& g0, DevBuf<int>& g1) {
+    k_chunk_count<<<blocks(S.ntiles + 1, 256), 256, 0, st>>>(S.ntiles, len, S.tile_group_off.get(), nch.get());
+    scan_ex(t.scratch, nch.get(), first.get(), S.ntiles + 1, st);
+    count = read_int(first.get() + S.ntiles, st);
+    tile.alloc(count);
+    g0.alloc(count);
+    g1.alloc(count);
+    k_chunk_fill<<<blocks(S.ntiles, 256), 256, 0, st>>>(S.ntiles, S.tile_group_off.get(), nch.get(), first.get(),
+                                                        tile.get(), g0.get(), g1.get());
+  };
+  cut(kGroupsPerChunk, S.nchunks, S.chunk_tile, S.chunk_g0, S.chunk_g1);
+  const int len = std::max(kGroupsPerChunkMin, S.ngroups / kChunkTarget);
+  S.nchunks64 = 0;
+  if (len < kGroupsPerChunk) cut(len, S.nchunks64, S.chunk64_tile, S.chunk64_g0, S.chunk64_g1);
   FMM_HIP(hipStreamSynchronize(st));
 }
 

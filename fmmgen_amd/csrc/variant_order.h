@@ -255,13 +255,17 @@ void m2l_plain(Tree& t, hipStream_t st) {
   if (S.ngroups == 0) return;
   S.Dtab64.alloc((size_t)S.nkeys * Op<P>::MS);
   k_dtab<P, double, false><<<nblk(S.nkeys, 64), 64, 0, st>>>(S.nkeys, S.key_dx.get(), S.key_r.get(), S.Dtab64.get());
-  const int grid = ((S.nchunks + 7) / 8) * 8;
+  const bool fine = S.nchunks64 > 0;
+  const int n = fine ? S.nchunks64 : S.nchunks, grid = ((n + 7) / 8) * 8;
+  const int* tile = fine ? S.chunk64_tile.get() : S.chunk_tile.get();
+  const int* g0 = fine ? S.chunk64_g0.get() : S.chunk_g0.get();
+  const int* g1 = fine ? S.chunk64_g1.get() : S.chunk_g1.get();
   if (m2l_harmonic(t, 0, P)) {
     constexpr int W = m2l_waves<P, SO, double, kHarmonic>();
     const unsigned* idx = ensure_index_table<P, W, kHarmonic>(t, st);
     harm_fold<P, double>(t, t.M.get(), Op<P>::MS, t.Mh64, t.Lh64, st);
     k_m2l_gemm<P, SO, double, false, W, kHarmonic><<<grid, 64 * W, 0, st>>>(
-        S.nchunks, grid, S.tile_cells.get(), S.chunk_tile.get(), S.chunk_g0.get(), S.chunk_g1.get(),
+        n, grid, S.tile_cells.get(), tile, g0, g1,
         S.group_key.get(), S.group_src.get(), S.key_dlevel.get(), S.Dtab64.get(), idx, t.tile_order_ptr(), nullptr,
         Op<P>::MS, harm_msize(P, SO), harm_lsize(P, SO), t.Mh64.get(), t.Lh64.get());
     harm_unfold<P, double>(t, t.Lh64, t.L.get(), Op<P>::LS, st);
@@ -270,7 +274,7 @@ void m2l_plain(Tree& t, hipStream_t st) {
   constexpr int W = m2l_waves<P, SO, double>();
   const unsigned* idx = ensure_index_table<P, W>(t, st);
   k_m2l_gemm<P, SO, double, false, W><<<grid, 64 * W, 0, st>>>(
-      S.nchunks, grid, S.tile_cells.get(), S.chunk_tile.get(), S.chunk_g0.get(), S.chunk_g1.get(), S.group_key.get(),
+      n, grid, S.tile_cells.get(), tile, g0, g1, S.group_key.get(),
       S.group_src.get(), S.key_dlevel.get(), S.Dtab64.get(), idx, t.tile_order_ptr(), nullptr, Op<P>::MS,
       Op<P>::MS, Op<P>::LS, t.M.get(), t.L.get());
 }
