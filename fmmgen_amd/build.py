@@ -56,7 +56,7 @@ def generate():
     units = []
     for stem, kw in VARIANTS.items():
         text = device_source(kw["order"], kw["potential"], kw["field"], kw["source_order"],
-                             harmonic_derivs=True)
+                             harmonic_derivs=True, full_bodies_max_order=-1)  # the kernels use the chunks
         _write_if_changed(os.path.join(GEN, f"dev_{stem}.h"), text)
         head = (f'#include "_gen/dev_{stem}.h"\n'
                 f"#define FMM_VARIANT_NS v_{stem}\n")
