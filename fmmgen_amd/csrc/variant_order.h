@@ -123,9 +123,11 @@ __global__ __launch_bounds__(64) void k_p2m_leaf(int nleaves, const int* __restr
 // shifts its child's multipole along the three axes in LDS (at most P + 1 terms
 // a slot and axis), and the block adds the children in order.  A thread a
 // (parent, chunk) takes the children one after the other: 10^5 particles, order 4
-// 8.5 -> 4.7 us a level; levels of up to 512 parents, order 8 29 -> 10 us.  From
-// 4096 parents on its generated bodies, the chip full, are as fast (37 us).
-constexpr int kM2MWaveParents = 1024;
+// 8.5 -> 4.7 us a level; levels of up to 512 parents, order 8 29 -> 10 us.  On 4096
+// parents of eight children its generated bodies, the chip full, are faster (37
+// against 73 us); from order 10 on they are not (2^22 blobs, all levels 1.9 -> 1.2
+// ms).
+constexpr int kM2MWaveParents = 1024, kM2MWaveOrder = 10;
 template <int P>
 __global__ __launch_bounds__(512) void k_m2m_wave(int beg, const int* __restrict__ first_child, const int* __restrict__ nchild,
                       const double* __restrict__ cx, const double* __restrict__ cy, const double* __restrict__ cz,
@@ -301,6 +303,28 @@ __global__ __launch_bounds__(64) void k_l2l(int beg, int end, const int* __restr
   });
 }
 
+// The same with a wave a child, four children a block: the parent's expansion is
+// shifted axis by axis in LDS.  From local order 8 on the generated bodies cost
+// more than the loops' indices: 2^20 particles, order 8 264 -> 82 us over all
+// levels, 2^22 blobs, order 10 1.13 -> 0.72 ms.  At local orders 5 to 7 the bodies
+// are the faster ones (2^20, order 6 72 against 98 us).
+constexpr int kL2LWaveOrder = 8;
+template <int P>
+__global__ __launch_bounds__(256) void k_l2l_wave(int beg, int end, const int* __restrict__ parent, const double* __restrict__ cx,
+                      const double* __restrict__ cy, const double* __restrict__ cz, double* __restrict__ L) {
+  constexpr int LS = Op<P>::LS, Q = P - SO;
+  __shared__ double sA[4][LS], sB[4][LS], sP[4][3 * (Q + 1)];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = beg + blockIdx.x * 4 + w;
+  if (c >= end) return;  // no barrier below
+  const int p = parent[c];
+  for (int j = lane; j < LS; j += 64) sA[w][j] = L[(size_t)p * LS + j];
+  wave_powers<Q>(lane, cx[c] - cx[p], cy[c] - cy[p], cz[c] - cz[p], sP[w]);
+  wave_lds_fence();
+  wave_shift3<Q, false>(lane, sA[w], sB[w], sP[w]);
+  double* Lc = L + (size_t)c * LS;
+  for (int j = lane; j < LS; j += 64) Lc[j] += sB[w][j];
+}
+
 template <int P>
 __global__ __launch_bounds__(64) void k_l2p_final(int n, const int* __restrict__ leaf_of, const int* __restrict__ perm,
                             const double* __restrict__ cx, const double* __restrict__ cy,
@@ -412,13 +436,14 @@ void far_field_order(Tree& t, int mode, int mask, hipStream_t st) {
     PhaseTimer pt(t, kTM2M, st);
     for (int l = t.depth - 2; l >= 0; --l) {
       const int b = t.level_off[l], e = t.level_off[l + 1];
-      if (e - b <= kM2MWaveParents) {
+      if (P >= kM2MWaveOrder || e - b <= kM2MWaveParents) {
         k_m2m_wave<P><<<e - b, 512, 0, st>>>(b, t.first_child.get(), t.nchild.get(), t.cx.get(), t.cy.get(),
                                              t.cz.get(), t.M.get());
         continue;
       }
-      k_m2m<P><<<dim3(nblk(e - b, 64), (Op<P>::MS + kChunk - 1) / kChunk), 64, 0, st>>>(b, e, t.first_child.get(), t.nchild.get(), t.cx.get(),
-                                               t.cy.get(), t.cz.get(), t.M.get());
+      if constexpr (P < kM2MWaveOrder)
+        k_m2m<P><<<dim3(nblk(e - b, 64), (Op<P>::MS + kChunk - 1) / kChunk), 64, 0, st>>>(
+            b, e, t.first_child.get(), t.nchild.get(), t.cx.get(), t.cy.get(), t.cz.get(), t.M.get());
     }
   }
   if (mask & kPhaseM2L) {
@@ -429,8 +454,12 @@ void far_field_order(Tree& t, int mode, int mask, hipStream_t st) {
     PhaseTimer pt(t, kTL2L, st);
     for (int l = 1; l < t.depth; ++l) {
       const int b = t.level_off[l], e = t.level_off[l + 1];
-      k_l2l<P><<<dim3(nblk(e - b, 64), (Op<P>::LS + kChunk - 1) / kChunk), 64, 0, st>>>(b, e, t.parent.get(), t.cx.get(), t.cy.get(), t.cz.get(),
-                                               t.L.get());
+      if constexpr (P - SO >= kL2LWaveOrder)
+        k_l2l_wave<P><<<nblk(e - b, 4), 256, 0, st>>>(b, e, t.parent.get(), t.cx.get(), t.cy.get(), t.cz.get(),
+                                                      t.L.get());
+      else
+        k_l2l<P><<<dim3(nblk(e - b, 64), (Op<P>::LS + kChunk - 1) / kChunk), 64, 0, st>>>(
+            b, e, t.parent.get(), t.cx.get(), t.cy.get(), t.cz.get(), t.L.get());
     }
   }
 }

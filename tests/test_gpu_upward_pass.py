@@ -1,6 +1,6 @@
-"""FP64 upward pass: leaves of one particle, of a staged batch of 32 and around it,
-and levels below and above the number of parents where M2M changes its form,
-through whole evaluations against the oracle (1e-12)."""
+"""FP64 upward and downward passes: leaves of one particle, of a staged batch of 32 and around it,
+and levels below and above the number of parents, and orders, where M2M and L2L change
+their form, through whole evaluations against the oracle (1e-12)."""
 import numpy as np
 import pytest
 import torch
@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,ncrit,order,so", [(9, 2, 4, 0), (300, 32, 2, 0), (300, 33, 12, 0), (3000, 200, 5, 0),
+                                              (3000, 16, 8, 0), (20000, 8, 9, 0), (20000, 8, 10, 0),
                                               (40000, 8, 3, 0), (40000, 8, 3, 1), (5000, 32, 4, 2)])
 def test_evaluation_matches_oracle(gpu, n, ncrit, order, so):
     from fmmgen_amd import build_tree
