@@ -51,7 +51,7 @@ __device__ __forceinline__ void charge_pair(double dx, double dy, double dz, dou
 // No second and third derivatives one by one as in the generated bodies.  200000
 // uniform particles, FP64 near field: dipoles 3.99 -> 1.66 ms, quadrupoles 7.18 ->
 // 2.48 ms; 4096 targets x 2^18 sources: dipoles 2.73 -> 1.43 ms, quadrupoles 6.02
-// -> 4.34 ms.
+// -> 2.16 ms.
 __device__ __forceinline__ void multipole_pair(double dx, double dy, double dz, const double* S, double* acc) {
   constexpr int F0 = OUT == 4 ? 1 : 0;
   const double r = inv_norm(fma(dx, dx, fma(dy, dy, dz * dz)));

@@ -866,14 +866,17 @@ void op_batch(int op, int order, int n, const double* xyz, const double* in, int
 // SIMD, or run at half the waves: 49 and 4.2 ms against 4.1 for 4096 targets x
 // 2^20 charges), fewer targets and more threads where there are too few
 // targets for two blocks a compute unit (300 targets: 1.54 -> 0.87 ms).  Small
-// sets keep one target a block: a wider block's sums cost more than its reads
-// save (2000 particles, 2000 targets: 15.6 us against 18.1).
+// sets take two targets a block where there are many, else one (5000 x 4000 one |
+// two | four: 39.1 | 29.7 | 29.8 us, 8000 x 1000: 17.1 | 15.1 | 19.6 us, 5000 x
+// 600: 11.3 | 10.7 | 14.8 us, quadrupoles 14.2 | 15.8 | 29.0 us).  Quadrupoles
+// spill at four.
 void direct(int n, const double* pos, const double* S, const long long* targets, int nt, double* F,
             hipStream_t st) {
   if (nt <= 0) return;
   auto run = [&](auto kern, int tt, int bs) { kern<<<nblk(nt, tt), bs, 0, st>>>(n, pos, S, targets, nt, F); };
-  if (n < 16384) run(k_direct<1, 256>, 1, 256);
-  else if (nt >= 1024) run(k_direct<4, 512>, 4, 512);
+  if (n < 16384 && nt >= 768) run(k_direct<2, 256>, 2, 256);
+  else if (n < 16384) run(k_direct<1, 256>, 1, 256);
+  else if (SO < 2 && nt >= 1024) run(k_direct<SO < 2 ? 4 : 2, 512>, 4, 512);
   else if (nt >= 768) run(k_direct<2, 512>, 2, 512);
   else if (nt >= 512) run(k_direct<1, 512>, 1, 512);
   else run(k_direct<1, 1024>, 1, 1024);
