@@ -53,7 +53,7 @@ __global__ __launch_bounds__(BS, 4) void k_direct(int n, const double* __restric
 #pragma unroll
     for (int k = 0; k < SS; ++k) ns[k] = S[i * SS + k];
   };
-  load(threadIdx.x);
+  if (n > 0) load(threadIdx.x);  // no sources: no access, every target is out of range
   for (unsigned b = 0; b < (unsigned)n; b += BS) {
     const unsigned j = b + threadIdx.x;
     const double x = nx[0], y = nx[1], z = nx[2];
