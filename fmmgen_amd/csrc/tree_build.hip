@@ -183,11 +183,13 @@ __global__ __launch_bounds__(192) void k_mean_steps(const double* __restrict__ p
   MeanStep s{{0, 0}};
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const double y = ldexp(x[k], 52 - e), f = floor(y), r = y - f;  // exact: |x| < 2^(e + 2)
+    // y in units of the sum's last place; y - rint(y) is exact (y - floor(y) is
+    // not just above a negative half), so it shows ties and nothing else
+    const double y = ldexp(x[k], 52 - e), f = rint(y), r = y - f;
     const long long i = (long long)f;
     MeanStep t;
-    t.d[0] = i + (r > 0.5 || (r == 0.5 && (i & 1)) ? 1 : 0);
-    t.d[1] = i + (r > 0.5 || (r == 0.5 && !(i & 1)) ? 1 : 0);
+    t.d[0] = i;                                              // rint takes a tie to the even side
+    t.d[1] = i + (r == 0.5 ? 1 : (r == -0.5 ? -1 : 0));      // an odd S takes the odd side
     s = mean_then(s, t);
   }
   s = mean_reduce(s);
