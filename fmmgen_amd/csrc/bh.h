@@ -329,8 +329,8 @@ __global__ __launch_bounds__(64 * W) void k_bh(int n, const int* __restrict__ fi
         if (j != s) source_pair<double>(xi - px[j], yi - py[j], zi - pz[j], pS + (size_t)j * SS, part);
       bool bad = false;
 #pragma unroll
-      for (int k = 0; k < OUT; ++k) bad = bad || part[k] != part[k];
-      if (bad) {  // coincident particles: the generated body
+      for (int k = 0; k < OUT; ++k) bad = bad || not_finite(part[k]);
+      if (bad) {  // coincident particles above all: the generated body
 #pragma unroll
         for (int k = 0; k < OUT; ++k) part[k] = 0.0;
         for (int j = b; j < e; ++j)

@@ -9,18 +9,22 @@ namespace FMM_VARIANT_NS {
 
 // 1/r from the hardware estimate y of x^(-1/2), x = r^2, corrected in FP64 by
 // the series of (1 - e)^(-1/2), e = 1 - x y^2, which cubes the estimate's
-// relative error.  No case of x is treated apart: where x or a power of y leaves
-// the finite range (coincident particles above all) an FP64 pair comes out as
-// NaN, and the callers repeat such sums with the generated body.
+// relative error.  No case of x is treated apart: x = 0 (coincident particles)
+// and infinite x give NaN, subnormal x (y^2 overflows) gives NaN or infinity.
+// The callers repeat a sum that has come out as not finite with the generated
+// body, which also settles the sums that are infinite by right.
 __device__ __forceinline__ double inv_norm(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-x, y * y, 1.0);
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
+__device__ __forceinline__ bool not_finite(double v) { return !(fabs(v) < __builtin_huge_val()); }
+
 // One charge pair in FP64: q/r and q r^-3 (dx, dy, dz).  19 instructions and the
 // estimate, against 23 in the generated body (its select of zero and infinite
-// x).
+// x).  The products are taken in the generated body's order, (q y) y y: y^3 by
+// itself leaves the range before q r^-3 does.
 __device__ __forceinline__ void charge_pair(double dx, double dy, double dz, double q, double* acc) {
   const double x = fma(dx, dx, fma(dy, dy, dz * dz));
   double s3;
@@ -28,7 +32,7 @@ __device__ __forceinline__ void charge_pair(double dx, double dy, double dz, dou
     const double y = __builtin_amdgcn_rsq(x);
     const double y2 = y * y;
     const double e = fma(-x, y2, 1.0);
-    const double q3 = q * (y2 * y), t = q3 * e;
+    const double q3 = (q * y) * y2, t = q3 * e;
     s3 = fma(t * e, 1.875, fma(t, 1.5, q3));
   } else {
     const double r = inv_norm(x), s = q * r;

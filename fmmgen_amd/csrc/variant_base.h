@@ -25,8 +25,8 @@ __global__ void k_gather_S(int n, const int* __restrict__ perm, const double* __
 // strides its BS threads over the sources, the next source loaded during the
 // pairs of this one; wave sums, then a sum over the waves, in a fixed order.
 // Pairs take source_pair, the target itself as a zero source at unit
-// distance; a row that comes out as NaN is summed again with the generated
-// body.  Bound by the FP64 pairs: 4096 targets x 2^20 charges 6.9 ms with one
+// distance; a row that comes out as not finite is summed again with the
+// generated body.  Bound by the FP64 pairs: 4096 targets x 2^20 charges 6.9 ms with one
 // target a block, 4.1 ms with four.
 template <int TT, int BS>
 __global__ __launch_bounds__(BS, 4) void k_direct(int n, const double* __restrict__ pos, const double* __restrict__ S,
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(BS, 4) void k_direct(int n, const double* __restric
   for (int u = 0; u < TT && t0 + u < nt; ++u) {  // uniform over the block
     const long long t = tg[t0 + u];
     bool bad = false;
-    for (int k = 0; k < OUT; ++k) bad = bad || sum[u * OUT + k] != sum[u * OUT + k];
+    for (int k = 0; k < OUT; ++k) bad = bad || not_finite(sum[u * OUT + k]);
     if (!bad || t < 0 || t >= n) continue;
     const double xt = pos[3 * t], yt = pos[3 * t + 1], zt = pos[3 * t + 2];
     double a[OUT];
@@ -317,7 +317,7 @@ __device__ __forceinline__ void p2p_pair(int j, int tslot, double xt, double yt,
 }
 
 // The chunk's sum with the generated body, for a chunk whose FP64 source_pair
-// sum has come out as NaN in some lane.
+// sum is not finite in some lane.
 template <typename T>
 __device__ __forceinline__ void p2p_chunk_exact(int ns, int filled, int sl, int tslot, double xt, double yt,
                                                 double zt, const double* sx, const double* sy, const double* sz,
@@ -361,7 +361,7 @@ __device__ __forceinline__ void p2p_chunk_any(int nslice, int filled, int sl, in
   if constexpr (sizeof(T) == 8) {
     bool bad = false;
 #pragma unroll
-    for (int k = 0; k < OUT; ++k) bad = bad || part[k] != part[k];
+    for (int k = 0; k < OUT; ++k) bad = bad || not_finite(part[k]);
     if (__any(bad)) p2p_chunk_exact<T>(nslice, filled, sl, tslot, xt, yt, zt, sx, sy, sz, sS, sid, part);
   }
 }
