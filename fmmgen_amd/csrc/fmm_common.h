@@ -189,13 +189,20 @@ constexpr int kChunkTarget = 4096, kGroupsPerChunkMin = 2;
 // P2P work items: the source sequence of a target leaf (own particles, then
 // its merged ranges) cut into segments of at most kSegment source particles,
 // so that a leaf next to a dense cluster is spread over many waves.  Item =
-// (leaf, first range (rb - 1 = own leaf), offset in that range, source count);
-// split leaves accumulate with atomics into a zeroed output.
+// (leaf, first range (rb - 1 = own leaf), offset in that range, source count).
+// Where some leaf is split, the items of a leaf either store their sums in rows
+// of their own, which the final sum adds in the items' order (rows > 0: the finer
+// FP64 items, so that an evaluation repeats bit for bit), or add them with atomics
+// into a zeroed output.
 struct P2PItems {
   static constexpr int kSegment = 8192;
+  static constexpr long long kMaxRows = 1LL << 23;  // 256 MB of four outputs
   long long count = 0;
-  int split = 0;  // some leaf has more than one item
+  int split = 0;       // some leaf has more than one item
+  long long rows = 0;  // partial rows: the targets of every item
   DevBuf<int> leaf, r, o, n;
+  DevBuf<int> row;            // [count] first row of an item
+  DevBuf<long long> row_off;  // [ncells + 1] first row of a leaf's items
 };
 
 // ------------------------------------------------------------ tree handle
@@ -300,6 +307,7 @@ struct Tree {
   DevBuf<double> Qbh;             // Barnes-Hut: solid-harmonic coefficient rows of every cell (bh.h)
   DevBuf<double> Mtop, Ltop;
   DevBuf<double> Fp2p;            // per-target near-field result, sorted order
+  DevBuf<double> Fseg;            // the same by items (P2PItems::rows)
   Scratch scratch;
 
   // work counters (list build)

@@ -686,19 +686,21 @@ __device__ __forceinline__ long long seg_length(long long tot, int seg, int even
   return ((tot + k - 1) / k + 127) / 128 * 128;
 }
 
-// Per leaf: number of P2P segments; per range: its length as 64-bit.
+// Per leaf: number of P2P segments and of the rows they store (a target a
+// segment); both 0 at ncells, so that the scans' last entries are the totals.
 __global__ void k_seg_count(int ncells, const int* __restrict__ nchild, const int* __restrict__ pcount,
                             const int* __restrict__ rng_off, const long long* __restrict__ cum,
-                            long long* __restrict__ nseg, int seg, int even) {
+                            long long* __restrict__ nseg, long long* __restrict__ nrow, int seg, int even) {
   const int A = blockIdx.x * blockDim.x + threadIdx.x;
-  if (A >= ncells) return;
+  if (A > ncells) return;
   long long k = 0;
-  if (nchild[A] == 0 && pcount[A] > 0) {
+  if (A < ncells && nchild[A] == 0 && pcount[A] > 0) {
     const long long tot = pcount[A] + cum[rng_off[A + 1]] - cum[rng_off[A]];
     const long long len = seg_length(tot, seg, even);
     k = (tot + len - 1) / len;
   }
   nseg[A] = k;
+  nrow[A] = k > 0 ? k * pcount[A] : 0;
 }
 
 __global__ void k_widen(long long m, const int* __restrict__ in, long long* __restrict__ out) {
@@ -710,9 +712,10 @@ __global__ void k_widen(long long m, const int* __restrict__ in, long long* __re
 // sequence (own particles first, then the ranges in order).
 __global__ void k_seg_fill(int ncells, const int* __restrict__ nchild, const int* __restrict__ pcount,
                            const int* __restrict__ rng_off, const long long* __restrict__ cum,
-                           const long long* __restrict__ nseg, const long long* __restrict__ seg_off, int seg, int even,
-                           int* __restrict__ it_leaf, int* __restrict__ it_r, int* __restrict__ it_o,
-                           int* __restrict__ it_n) {
+                           const long long* __restrict__ nseg, const long long* __restrict__ seg_off,
+                           const long long* __restrict__ row_off, int seg, int even, int* __restrict__ it_leaf,
+                           int* __restrict__ it_r, int* __restrict__ it_o, int* __restrict__ it_n,
+                           int* __restrict__ it_row) {
   const int A = blockIdx.x * blockDim.x + threadIdx.x;
   if (A >= ncells || nseg[A] == 0) return;
   const int nt = pcount[A], rb = rng_off[A], re = rng_off[A + 1];
@@ -739,6 +742,7 @@ __global__ void k_seg_fill(int ncells, const int* __restrict__ nchild, const int
     it_r[w] = r;
     it_o[w] = o;
     it_n[w] = (int)((tot - P < len) ? tot - P : len);
+    if (it_row) it_row[w] = (int)(row_off[A] + s * nt);
   }
 }
 
@@ -755,7 +759,7 @@ constexpr int kP2PItems = 65536;
 void build_p2p_items(Tree& t, hipStream_t st) {
   const int nc = t.ncells;
   const long long nr = t.n_rng;
-  DevBuf<long long> len, cum, nseg, soff;
+  DevBuf<long long> len, cum, nseg, soff, nrow;
   len.alloc(nr + 1);
   cum.alloc(nr + 1);
   FMM_HIP(hipMemsetAsync(len.get() + nr, 0, sizeof(long long), st));
@@ -763,25 +767,32 @@ void build_p2p_items(Tree& t, hipStream_t st) {
   exclusive_scan_int(t.scratch, len.get(), cum.get(), nr + 1, st);
   nseg.alloc(nc + 1);
   soff.alloc(nc + 1);
+  nrow.alloc(nc + 1);
   auto cut = [&](P2PItems& I, int seg, int even) {
-    FMM_HIP(hipMemsetAsync(nseg.get() + nc, 0, sizeof(long long), st));
-    k_seg_count<<<blocks(nc, 256), 256, 0, st>>>(nc, t.nchild.get(), t.pcount.get(), t.rng_off.get(), cum.get(),
-                                                 nseg.get(), seg, even);
+    k_seg_count<<<blocks(nc + 1, 256), 256, 0, st>>>(nc, t.nchild.get(), t.pcount.get(), t.rng_off.get(), cum.get(),
+                                                     nseg.get(), nrow.get(), seg, even);
     exclusive_scan_int(t.scratch, nseg.get(), soff.get(), nc + 1, st);
-    long long total = 0;
+    long long total = 0, rows = 0;
     FMM_HIP(hipMemcpyAsync(&total, soff.get() + nc, sizeof(long long), hipMemcpyDeviceToHost, st));
+    if (even) {
+      I.row_off.alloc(nc + 1);
+      exclusive_scan_int(t.scratch, nrow.get(), I.row_off.get(), nc + 1, st);
+      FMM_HIP(hipMemcpyAsync(&rows, I.row_off.get() + nc, sizeof(long long), hipMemcpyDeviceToHost, st));
+    }
     FMM_HIP(hipStreamSynchronize(st));
     FMM_CHECK(total < (1LL << 31), kOutOfMemory, "P2P work items exceed 2^31");
     I.count = total;
     I.split = total > t.nleaves;
+    I.rows = I.split && rows <= P2PItems::kMaxRows ? rows : 0;
     const long long na = std::max<long long>(total, 1);
     I.leaf.alloc(na);
     I.r.alloc(na);
     I.o.alloc(na);
     I.n.alloc(na);
+    if (I.rows > 0) I.row.alloc(na);
     k_seg_fill<<<blocks(nc, 256), 256, 0, st>>>(nc, t.nchild.get(), t.pcount.get(), t.rng_off.get(), cum.get(),
-                                                nseg.get(), soff.get(), seg, even, I.leaf.get(), I.r.get(),
-                                                I.o.get(), I.n.get());
+                                                nseg.get(), soff.get(), I.row_off.get(), seg, even, I.leaf.get(),
+                                                I.r.get(), I.o.get(), I.n.get(), I.rows > 0 ? I.row.get() : nullptr);
   };
   cut(t.p2p, P2PItems::kSegment, 0);
   // source sequences in all: the pairs over the mean leaf size

@@ -286,8 +286,9 @@ __global__ void k_fill_int(long long n, int* __restrict__ a) {
 // The sources of a target leaf are its own particles (self pairs masked)
 // and the merged particle ranges of its other P2P leaves; they are staged
 // 128 at a time through LDS with coalesced loads.  A leaf whose sources span
-// several items (a small leaf beside a dense cluster) adds its partial sums
-// atomically into a zeroed output; other leaves store.  Targets go 64 to a
+// several items (a small leaf beside a dense cluster) stores each item's sums in
+// rows of their own (it_row) or adds them atomically into a zeroed output; other
+// leaves store.  Targets go 64 to a
 // round; a round of r targets runs as two power-of-two pieces (r = 40 as
 // 32 + 8, r = 20 as 16 + 4), each piece's targets replicated over 64 / p
 // lane slices that take alternate sources of every staged chunk, so fewer
@@ -398,7 +399,7 @@ __device__ __forceinline__ void p2p_item(int it, int nitems, const int* __restri
                                          const int* __restrict__ rng_start, const int* __restrict__ rng_len,
                                          const double* __restrict__ px, const double* __restrict__ py,
                                          const double* __restrict__ pz, const double* __restrict__ pS, int split,
-                                         double* __restrict__ F, double* sx, double* sy, double* sz, T* sS,
+                                         const int* __restrict__ it_row, double* __restrict__ F, double* sx, double* sy, double* sz, T* sS,
                                          int* sid) {
   constexpr bool kKahan = sizeof(T) == 4;
   const int lane = threadIdx.x;
@@ -406,8 +407,9 @@ __device__ __forceinline__ void p2p_item(int it, int nitems, const int* __restri
   const int t0 = pstart[A], nt = pcount[A];
   const int rb = rng_off[A], re = rng_off[A + 1];
   // a leaf cut into several items accumulates atomically
-  // (the items of a leaf are contiguous)
+  // (the items of a leaf are contiguous), unless every item has its own rows
   const bool atomic = split && ((it > 0 && it_leaf[it - 1] == A) || (it + 1 < nitems && it_leaf[it + 1] == A));
+  if (it_row) F += (ptrdiff_t)(it_row[it] - t0) * OUT;
   for (int tb = 0; tb < nt; tb += 64) {
     // this round's r targets as two power-of-two pieces: pa = the largest
     // power of two <= r (64 at most) and pb = r - pa rounded up to a power
@@ -513,7 +515,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const int* __restrict__ it_n, const int* __restrict__ pstart, const int* __restrict__ pcount,
     const int* __restrict__ rng_off, const int* __restrict__ rng_start, const int* __restrict__ rng_len,
     const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
-    const double* __restrict__ pS, int split, double* __restrict__ F) {
+    const double* __restrict__ pS, int split, const int* __restrict__ it_row, double* __restrict__ F) {
   __shared__ double sx[kP2PChunk], sy[kP2PChunk], sz[kP2PChunk];
   __shared__ T sS[kP2PChunk * SS];
   __shared__ int sid[kP2PChunk];
@@ -521,7 +523,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const int it = ((k / kP2PRun) * 8 + (int)(blockIdx.x & 7)) * kP2PRun + k % kP2PRun;
   if (it < nitems)
     p2p_item<T>(it, nitems, it_leaf, it_r, it_o, it_n, pstart, pcount, rng_off, rng_start, rng_len, px, py, pz, pS,
-                split, F, sx, sy, sz, sS, sid);
+                split, it_row, F, sx, sy, sz, sS, sid);
 }
 
 __global__ void k_fill_zero(long long n, double* __restrict__ a) {
@@ -533,7 +535,10 @@ void near_field(Tree& t, int mode, hipStream_t st) {
   const P2PItems& I = t.p2p_items(mode == 0);
   const int ni = (int)I.count;
   PhaseTimer pt(t, kTP2P, st);
-  if (I.split) {
+  const bool rows = near_rows(t, mode);
+  if (rows) {
+    t.Fseg.alloc((size_t)I.rows * OUT);
+  } else if (I.split) {
     const long long m = (long long)t.n * OUT;
     k_fill_zero<<<(int)((m + 255) / 256), 256, 0, st>>>(m, t.Fp2p.get());
   }
@@ -542,7 +547,8 @@ void near_field(Tree& t, int mode, hipStream_t st) {
   auto launch = [&](auto kern) {
     kern<<<grid, 64, 0, st>>>(ni, I.leaf.get(), I.r.get(), I.o.get(), I.n.get(), t.pstart.get(), t.pcount.get(),
                               t.rng_off.get(), t.rng_start.get(), t.rng_len.get(), t.px.get(), t.py.get(),
-                              t.pz.get(), t.pS.get(), I.split, t.Fp2p.get());
+                              t.pz.get(), t.pS.get(), rows ? 0 : I.split, rows ? I.row.get() : nullptr,
+                              rows ? t.Fseg.get() : t.Fp2p.get());
   };
   if (mode == 0) launch(k_p2p_leaf<double>);
   else launch(k_p2p_leaf<float>);

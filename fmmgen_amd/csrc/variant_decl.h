@@ -55,6 +55,9 @@ inline bool m2l_harmonic(const Tree& t, int mode, int p) {
   return p >= kHarmMinOrder || t.sched.ngroups >= kHarmMinGroups;
 }
 
+// Whether the near field of an evaluation stores its sums by items.
+inline bool near_rows(const Tree& t, int mode) { return mode == 0 && t.p2p_items(true).rows > 0; }
+
 // Order-independent phases (defined in the base translation unit).
 void near_field(Tree& t, int mode, hipStream_t st);
 

@@ -325,20 +325,33 @@ __global__ __launch_bounds__(256) void k_l2l_wave(int beg, int end, const int* _
   for (int j = lane; j < LS; j += 64) Lc[j] += sB[w][j];
 }
 
+// Near plus far field.  Fnear: a row a particle, or with row_off a row a work
+// item and target (the items of leaf c from row_off[c], pcount[c] rows each),
+// added in the items' order.  (Rows instead of atomics into one output, for the
+// sake of repeatable sums: 2000 particles 53.8 -> 54.5 us an evaluation, 10^5 516
+// -> 520 us, 2^20 7.16 -> 7.12 ms.)
 template <int P>
 __global__ __launch_bounds__(64) void k_l2p_final(int n, const int* __restrict__ leaf_of, const int* __restrict__ perm,
                             const double* __restrict__ cx, const double* __restrict__ cy,
                             const double* __restrict__ cz, const double* __restrict__ px,
                             const double* __restrict__ py, const double* __restrict__ pz,
-                            const double* __restrict__ L, const double* __restrict__ Fnear, int use_l2p,
-                            double* __restrict__ F) {
+                            const double* __restrict__ L, const double* __restrict__ Fnear,
+                            const long long* __restrict__ row_off, const int* __restrict__ pstart,
+                            const int* __restrict__ pcount, int use_l2p, double* __restrict__ F) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   double acc[OUT];
+  const int c = leaf_of[j];
 #pragma unroll
-  for (int k = 0; k < OUT; ++k) acc[k] = Fnear ? Fnear[(size_t)j * OUT + k] : 0.0;
+  for (int k = 0; k < OUT; ++k) acc[k] = Fnear && !row_off ? Fnear[(size_t)j * OUT + k] : 0.0;
+  if (Fnear && row_off) {
+    const int nt = pcount[c];
+#pragma unroll 4
+    for (long long r = row_off[c] + (j - pstart[c]); r < row_off[c + 1]; r += nt)
+#pragma unroll
+      for (int k = 0; k < OUT; ++k) acc[k] += Fnear[(size_t)r * OUT + k];
+  }
   if (use_l2p) {
-    const int c = leaf_of[j];
     fmmgen_ops::L2P_o<P, double>(px[j] - cx[c], py[j] - cy[c], pz[j] - cz[c], L + (size_t)c * Op<P>::LS, acc);
   }
   const int i = perm[j];
@@ -472,10 +485,12 @@ void l2p_final_order(Tree& t, int mode, int mask, double* F, hipStream_t st) {
   }
   const int n = (int)t.n;
   PhaseTimer pt(t, kTL2P, st);
+  const bool rows = near_rows(t, mode);
   k_l2p_final<P><<<nblk(n, 64), 64, 0, st>>>(n, t.leaf_of.get(), t.perm.get(), t.cx.get(), t.cy.get(),
                                                t.cz.get(), t.px.get(), t.py.get(), t.pz.get(), t.L.get(),
-                                               (mask & kPhaseP2P) ? t.Fp2p.get() : nullptr,
-                                               (mask & kPhaseL2P) ? 1 : 0, F);
+                                               !(mask & kPhaseP2P) ? nullptr : rows ? t.Fseg.get() : t.Fp2p.get(),
+                                               rows ? t.p2p64.row_off.get() : nullptr, t.pstart.get(),
+                                               t.pcount.get(), (mask & kPhaseL2P) ? 1 : 0, F);
 }
 
 }  // namespace FMM_VARIANT_NS

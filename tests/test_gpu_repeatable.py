@@ -1,0 +1,47 @@
+"""Plain FP64 evaluations of sets whose leaves are cut into several near-field
+items give the same bits every time, and agree with the oracle's sums."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests import util
+
+pytestmark = pytest.mark.gpu
+P2P = 8
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _tree(n, ncrit, so, order=3):
+    from fmmgen_amd import build_tree
+    pot = so != 1
+    pos = util.blobs(n, 21)
+    S = np.random.default_rng(22).normal(size=(n, {0: 1, 1: 3, 2: 6}[so]))
+    return pos, S, build_tree(_dev(pos), _dev(S), n, ncrit, order, 0.5, source_order=so, potential=pot)
+
+
+def _repeat(t, n, outsz, times, **kw):
+    """The first result, after showing that the later ones equal it (with other work between them)."""
+    first = None
+    for _ in range(times):
+        F = torch.full((n, outsz), float("nan"), dtype=torch.float64, device="cuda")
+        t.compute_field_fmm(F, mode="plain", **kw)
+        if first is None:
+            first = F.clone()
+        assert torch.equal(F, first)
+        t.compute_field_fmm(F, mode="f32")
+    return first.cpu().numpy()
+
+
+@pytest.mark.parametrize("n,ncrit,so", [(129, 200, 0), (2000, 64, 0), (2000, 8, 0), (9000, 1000, 0), (60000, 64, 0),
+                                        (9000, 64, 1), (9000, 64, 2)])
+def test_near_field_repeats(gpu, n, ncrit, so):
+    pos, S, t = _tree(n, ncrit, so)
+    outsz = 3 if so == 1 else 4
+    print(f"near field so={so} n={n} ncrit={ncrit}", flush=True)
+    got = _repeat(t, n, outsz, 8, phases=P2P)
+    want = O.OracleTree(pos, S, ncrit, 3, 0.5, source_order=so, outputsize=outsz).compute_field_fmm(mask=P2P)
+    assert util.rel_norm(got, want) <= 1e-12
