@@ -178,7 +178,13 @@ struct M2LSchedule {
   int nchunks = 0, nchunks64 = 0;
   DevBuf<int> chunk_tile, chunk_g0, chunk_g1;
   DevBuf<int> chunk64_tile, chunk64_g0, chunk64_g1;
+  DevBuf<int> chunk64_first;     // [ntiles + 1] first of a tile's finer chunks
+  DevBuf<int> cell_slot;         // [ncells] tile * kTile + column (-1: no M2L sources)
 };
+// From this order on the MFMA steps are dealt to a block's waves so that
+// several waves hold sums of one row of L (m2l_gemm.h); below it a row is one
+// wave's.
+constexpr int kM2LBalancedOrder = 6;
 constexpr int kGroupsPerChunk = 96;  // measured: 48 -> 96 cut the learned M2L by 11%
 // The FP64 M2L of sets with fewer than kChunkTarget such chunks is cut finer, so
 // that the chip fills: 2000 particles at order 4 (383 groups) 50 -> 8 us, 10^5
@@ -304,6 +310,7 @@ struct Tree {
   int m2l_form = 0;
   DevBuf<float> Mhf, Lhf;
   DevBuf<double> Mh64, Lh64;
+  DevBuf<double> Lpart;           // FP64 M2L: the finer chunks' sums (m2l_parts)
   DevBuf<double> Qbh;             // Barnes-Hut: solid-harmonic coefficient rows of every cell (bh.h)
   DevBuf<double> Mtop, Ltop;
   DevBuf<double> Fp2p;            // per-target near-field result, sorted order

@@ -64,15 +64,14 @@ __global__ void k_tile_keys(int nc, const int* __restrict__ off, const int* __re
 // Tiles of 16 in key order, starting anew on every level: level l holds sorted
 // entries from cnt[l] and tiles from base[l].
 __global__ void k_assign_tiles(int total, const unsigned long long* __restrict__ key_sorted,
-                               const int* __restrict__ cnt, const int* __restrict__ base, int* __restrict__ tile_of,
-                               int* __restrict__ col_of, int* __restrict__ tile_cells) {
+                               const int* __restrict__ cnt, const int* __restrict__ base, int* __restrict__ slot,
+                               int* __restrict__ tile_cells) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= total) return;
   const unsigned long long k = key_sorted[i];
   const int c = (int)(k & 0xffffffffu), l = (int)(k >> 42);
   const int j = i - cnt[l], t = base[l] + j / kTile, col = j % kTile;
-  tile_of[c] = t;
-  col_of[c] = col;
+  slot[c] = t * kTile + col;
   tile_cells[t * kTile + col] = c;
 }
 
@@ -135,9 +134,9 @@ __global__ void k_key_ids(long long m, const int* __restrict__ flag, const int* 
 }
 
 __global__ void k_group_keys(long long m, int kb, const int* __restrict__ tgt, const int* __restrict__ keyid,
-                             const int* __restrict__ tile_of, unsigned long long* __restrict__ comp) {
+                             const int* __restrict__ slot, unsigned long long* __restrict__ comp) {
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i < m) comp[i] = ((unsigned long long)(unsigned)tile_of[tgt[i]] << kb) | (unsigned)keyid[i];
+  if (i < m) comp[i] = ((unsigned long long)((unsigned)slot[tgt[i]] / kTile) << kb) | (unsigned)keyid[i];
 }
 
 // Groups and the first group of every tile (every tile has one: its cells all
@@ -145,7 +144,7 @@ __global__ void k_group_keys(long long m, int kb, const int* __restrict__ tgt, c
 __global__ void k_fill_groups(long long m, int kb, int ntiles, const unsigned long long* __restrict__ comp,
                               const int* __restrict__ order, const int* __restrict__ flag,
                               const int* __restrict__ pos, const int* __restrict__ tgt,
-                              const int* __restrict__ src, const int* __restrict__ col_of,
+                              const int* __restrict__ src, const int* __restrict__ slot,
                               int* __restrict__ group_key, int* __restrict__ group_src,
                               int* __restrict__ tile_first) {
   const long long j = blockIdx.x * (long long)blockDim.x + threadIdx.x;
@@ -159,7 +158,7 @@ __global__ void k_fill_groups(long long m, int kb, int ntiles, const unsigned lo
     if (j == 0 || (int)(comp[j - 1] >> kb) != t) tile_first[t] = g;
   }
   if (j == m - 1) tile_first[ntiles] = g + 1;
-  group_src[(long long)g * kTile + col_of[tgt[i]]] = src[i];
+  group_src[(long long)g * kTile + (unsigned)slot[tgt[i]] % kTile] = src[i];
 }
 
 // Work items of a tile: its groups cut into equal runs of at most
@@ -223,9 +222,9 @@ void build_m2l_schedule(Tree& t, hipStream_t st) {
   const long long m = t.n_m2l;
   FMM_CHECK(m < (1LL << 31), kOutOfMemory, "more than 2^31 M2L pairs");
   // tiles of every level
-  DevBuf<int> tile_of, col_of, rank, lvl;
-  tile_of.alloc(nc);
-  col_of.alloc(nc);
+  DevBuf<int> rank, lvl;
+  S.cell_slot.alloc(nc);
+  FMM_HIP(hipMemsetAsync(S.cell_slot.get(), 0xff, sizeof(int) * nc, st));
   {
     const int D = t.depth;
     rank.alloc(nc + 1);
@@ -263,7 +262,7 @@ void build_m2l_schedule(Tree& t, hipStream_t st) {
     FMM_HIP(rocprim::radix_sort_keys(nullptr, bytes, k0.get(), k1.get(), (size_t)nc, 0, 47, st));
     tmp = t.scratch.get(bytes);
     FMM_HIP(rocprim::radix_sort_keys(tmp, bytes, k0.get(), k1.get(), (size_t)nc, 0, 47, st));
-    k_assign_tiles<<<blocks(cnt[D], 256), 256, 0, st>>>(cnt[D], k1.get(), lcnt, lbase, tile_of.get(), col_of.get(),
+    k_assign_tiles<<<blocks(cnt[D], 256), 256, 0, st>>>(cnt[D], k1.get(), lcnt, lbase, S.cell_slot.get(),
                                                         S.tile_cells.get());
     FMM_HIP(hipStreamSynchronize(st));  // base, k0 and k1 end here
   }
@@ -291,7 +290,7 @@ void build_m2l_schedule(Tree& t, hipStream_t st) {
                                             keyid.get(), S.key_dx.get(), S.key_r.get(), S.key_dlevel.get());
   // groups = runs of (tile, key)
   const int kb = bits_for((unsigned long long)S.nkeys - 1);
-  k_group_keys<<<blocks(m, 256), 256, 0, st>>>(m, kb, tgt.get(), keyid.get(), tile_of.get(), key.get());
+  k_group_keys<<<blocks(m, 256), 256, 0, st>>>(m, kb, tgt.get(), keyid.get(), S.cell_slot.get(), key.get());
   sort_order(t, key.get(), key_sorted.get(), order.get(), m, kb + bits_for((unsigned long long)S.ntiles - 1), st);
   k_run_flags64<<<blocks(m + 1, 256), 256, 0, st>>>(m, key_sorted.get(), fl.get());
   scan_ex(t.scratch, fl.get(), pos.get(), m + 1, st);
@@ -300,13 +299,13 @@ void build_m2l_schedule(Tree& t, hipStream_t st) {
   S.group_src.alloc((size_t)S.ngroups * kTile);
   FMM_HIP(hipMemsetAsync(S.group_src.get(), 0xff, sizeof(int) * (size_t)S.ngroups * kTile, st));
   k_fill_groups<<<blocks(m, 256), 256, 0, st>>>(m, kb, S.ntiles, key_sorted.get(), order.get(), fl.get(), pos.get(),
-                                                tgt.get(), t.m2l_src.get(), col_of.get(), S.group_key.get(),
+                                                tgt.get(), t.m2l_src.get(), S.cell_slot.get(), S.group_key.get(),
                                                 S.group_src.get(), S.tile_group_off.get());
   // work items: runs of groups of one tile
-  DevBuf<int> nch, first;
+  DevBuf<int> nch, first32;
   nch.alloc(S.ntiles + 1);
-  first.alloc(S.ntiles + 1);
-  auto cut = [&](int len, int& count, DevBuf<int>& tile, DevBuf<int>& g0, DevBuf<int>& g1) {
+  auto cut = [&](int len, int& count, DevBuf<int>& first, DevBuf<int>& tile, DevBuf<int>& g0, DevBuf<int>& g1) {
+    first.alloc(S.ntiles + 1);
     k_chunk_count<<<blocks(S.ntiles + 1, 256), 256, 0, st>>>(S.ntiles, len, S.tile_group_off.get(), nch.get());
     scan_ex(t.scratch, nch.get(), first.get(), S.ntiles + 1, st);
     count = read_int(first.get() + S.ntiles, st);
@@ -316,10 +315,10 @@ void build_m2l_schedule(Tree& t, hipStream_t st) {
     k_chunk_fill<<<blocks(S.ntiles, 256), 256, 0, st>>>(S.ntiles, S.tile_group_off.get(), nch.get(), first.get(),
                                                         tile.get(), g0.get(), g1.get());
   };
-  cut(kGroupsPerChunk, S.nchunks, S.chunk_tile, S.chunk_g0, S.chunk_g1);
+  cut(kGroupsPerChunk, S.nchunks, first32, S.chunk_tile, S.chunk_g0, S.chunk_g1);
   const int len = std::max(kGroupsPerChunkMin, S.ngroups / kChunkTarget);
   S.nchunks64 = 0;
-  if (len < kGroupsPerChunk) cut(len, S.nchunks64, S.chunk64_tile, S.chunk64_g0, S.chunk64_g1);
+  if (len < kGroupsPerChunk) cut(len, S.nchunks64, S.chunk64_first, S.chunk64_tile, S.chunk64_g0, S.chunk64_g1);
   FMM_HIP(hipStreamSynchronize(st));
 }
 

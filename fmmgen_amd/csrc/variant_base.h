@@ -606,11 +606,12 @@ void evaluate(Tree& t, int mode, int mask, double* F, hipStream_t st) {
   {
     PhaseTimer pt(t, kTPrep, st);
     k_gather_S<<<nblk(n, 256), 256, 0, st>>>(n, t.perm.get(), t.user_S, t.pS.get());
-    // P2M and M2M write every multipole slot and the harmonic form's unfold
-    // every local slot: cleared only when one of those is left out
+    // P2M and M2M write every multipole slot, and the harmonic form's unfold or
+    // the sum over chunks every local slot: cleared only when those are left out
     if (mode == 0 && !((mask & kPhaseP2M) && (mask & kPhaseM2M)))
       FMM_HIP(hipMemsetAsync(t.M.get(), 0, sizeof(double) * nc * ms, st));
-    if (mode == 0 && !((mask & kPhaseM2L) && t.sched.ngroups > 0 && m2l_harmonic(t, mode, t.order)))
+    if (mode == 0 && !((mask & kPhaseM2L) && t.sched.ngroups > 0 &&
+                       (m2l_harmonic(t, mode, t.order) || m2l_parts(t, t.order))))
       FMM_HIP(hipMemsetAsync(t.L.get(), 0, sizeof(double) * nc * ls, st));
   }
   OrderTable<PMIN>::far(t.order, t, mode, mask, st);

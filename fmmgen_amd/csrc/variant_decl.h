@@ -55,6 +55,10 @@ inline bool m2l_harmonic(const Tree& t, int mode, int p) {
   return p >= kHarmMinOrder || t.sched.ngroups >= kHarmMinGroups;
 }
 
+// Whether the FP64 M2L stores every chunk's sums and adds a tile's chunks in
+// order, so that an evaluation repeats bit for bit, instead of adding them into L
+// with atomics: the finer chunk list at the orders whose rows are one wave's.
+inline bool m2l_parts(const Tree& t, int p) { return p < kM2LBalancedOrder && t.sched.nchunks64 > 0; }
 // Whether the near field of an evaluation stores its sums by items.
 inline bool near_rows(const Tree& t, int mode) { return mode == 0 && t.p2p_items(true).rows > 0; }
 

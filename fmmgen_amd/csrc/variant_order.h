@@ -219,22 +219,24 @@ const unsigned* ensure_index_table(Tree& t, hipStream_t st) {
 }
 
 // Harmonic-layout M2L around the GEMM: fold every cell's multipole (M,
-// graded, stride ms) into Mh and clear Lh (rows of order PS), then, after
-// the GEMM, store the unfolded rows into L (graded, stride ls).
+// graded, stride ms) into Mh and clear Lh (rows of order PS; with `parts` the
+// GEMM writes rows of its own instead), then, after the GEMM, store the unfolded
+// rows into L (graded, stride ls).
 template <int PS, typename T>
-void harm_fold(Tree& t, const T* M, int ms, DevBuf<T>& Mh, DevBuf<T>& Lh, hipStream_t st) {
-  const int nc = t.ncells, hs = harm_msize(PS, SO), ls = harm_lsize(PS, SO);
+void harm_fold(Tree& t, const T* M, int ms, DevBuf<T>& Mh, DevBuf<T>& Lh, hipStream_t st, bool parts = false) {
+  const int nc = t.ncells, hs = harm_msize(PS, SO), ls = parts ? 0 : harm_lsize(PS, SO);
   Mh.alloc((size_t)nc * hs);
-  Lh.alloc((size_t)nc * ls);
+  if (!parts) Lh.alloc((size_t)nc * ls);
   if (nc == 0) return;
   constexpr int per = 4 * kHarmCellsPerWave;
   k_harm_fold<PS, SO, T><<<(nc + per - 1) / per, 256, 0, st>>>(nc, M, ms, Mh.get(), hs, Lh.get(), ls);
 }
-template <int PS, typename T>
+template <int PS, typename T, bool PART = false>
 void harm_unfold(Tree& t, const DevBuf<T>& Lh, T* L, int ls, hipStream_t st) {
   if (t.ncells == 0) return;
   constexpr int per = 4 * kHarmCellsPerWave;
-  k_harm_unfold<PS - SO, T><<<(t.ncells + per - 1) / per, 256, 0, st>>>(t.ncells, Lh.get(), harm_lsize(PS, SO), L, ls);
+  k_harm_unfold<PS - SO, T, PART><<<(t.ncells + per - 1) / per, 256, 0, st>>>(
+      t.ncells, Lh.get(), harm_lsize(PS, SO), L, ls, t.sched.cell_slot.get(), t.sched.chunk64_first.get());
 }
 
 template <int P, int W, int LAY = kGraded>
@@ -251,6 +253,37 @@ const unsigned* ensure_index_table32(Tree& t, hipStream_t st) {
   return S.idxtab32[LAY][P].get();
 }
 
+// FP64 M2L of the given chunks; PART: the chunks' sums are stored and a tile's
+// chunks added in order (m2l_parts).
+template <int P, bool PART>
+void m2l_plain_run(Tree& t, int n, const int* tile, const int* g0, const int* g1, hipStream_t st) {
+  M2LSchedule& S = t.sched;
+  const int grid = ((n + 7) / 8) * 8;
+  auto run = [&](auto kern, int W, const unsigned* idx, int mstride, int lstride, const double* M, double* L) {
+    kern<<<grid, 64 * W, 0, st>>>(n, grid, S.tile_cells.get(), tile, g0, g1, S.group_key.get(), S.group_src.get(),
+                                  S.key_dlevel.get(), S.Dtab64.get(), idx, t.tile_order_ptr(), nullptr, Op<P>::MS,
+                                  mstride, lstride, M, L);
+  };
+  if (m2l_harmonic(t, 0, P)) {
+    constexpr int W = m2l_waves<P, SO, double, kHarmonic>(), HL = harm_lsize(P, SO);
+    const unsigned* idx = ensure_index_table<P, W, kHarmonic>(t, st);
+    harm_fold<P, double>(t, t.M.get(), Op<P>::MS, t.Mh64, t.Lh64, st, PART);
+    if (PART) t.Lpart.alloc((size_t)n * kTile * HL);
+    DevBuf<double>& Lh = PART ? t.Lpart : t.Lh64;
+    run(k_m2l_gemm<P, SO, double, false, W, kHarmonic, PART>, W, idx, harm_msize(P, SO), HL, t.Mh64.get(), Lh.get());
+    harm_unfold<P, double, PART>(t, Lh, t.L.get(), Op<P>::LS, st);
+    return;
+  }
+  constexpr int W = m2l_waves<P, SO, double>(), LS = Op<P>::LS;
+  const unsigned* idx = ensure_index_table<P, W>(t, st);
+  if (PART) t.Lpart.alloc((size_t)n * kTile * LS);
+  run(k_m2l_gemm<P, SO, double, false, W, kGraded, PART>, W, idx, Op<P>::MS, LS, t.M.get(),
+      PART ? t.Lpart.get() : t.L.get());
+  if (PART)
+    k_chunk_sum<double><<<nblk((long long)t.ncells * LS, 256), 256, 0, st>>>(
+        t.ncells, LS, S.cell_slot.get(), S.chunk64_first.get(), t.Lpart.get(), t.L.get());
+}
+
 template <int P>
 void m2l_plain(Tree& t, hipStream_t st) {
   M2LSchedule& S = t.sched;
@@ -258,27 +291,17 @@ void m2l_plain(Tree& t, hipStream_t st) {
   S.Dtab64.alloc((size_t)S.nkeys * Op<P>::MS);
   k_dtab<P, double, false><<<nblk(S.nkeys, 64), 64, 0, st>>>(S.nkeys, S.key_dx.get(), S.key_r.get(), S.Dtab64.get());
   const bool fine = S.nchunks64 > 0;
-  const int n = fine ? S.nchunks64 : S.nchunks, grid = ((n + 7) / 8) * 8;
+  const int n = fine ? S.nchunks64 : S.nchunks;
   const int* tile = fine ? S.chunk64_tile.get() : S.chunk_tile.get();
   const int* g0 = fine ? S.chunk64_g0.get() : S.chunk_g0.get();
   const int* g1 = fine ? S.chunk64_g1.get() : S.chunk_g1.get();
-  if (m2l_harmonic(t, 0, P)) {
-    constexpr int W = m2l_waves<P, SO, double, kHarmonic>();
-    const unsigned* idx = ensure_index_table<P, W, kHarmonic>(t, st);
-    harm_fold<P, double>(t, t.M.get(), Op<P>::MS, t.Mh64, t.Lh64, st);
-    k_m2l_gemm<P, SO, double, false, W, kHarmonic><<<grid, 64 * W, 0, st>>>(
-        n, grid, S.tile_cells.get(), tile, g0, g1,
-        S.group_key.get(), S.group_src.get(), S.key_dlevel.get(), S.Dtab64.get(), idx, t.tile_order_ptr(), nullptr,
-        Op<P>::MS, harm_msize(P, SO), harm_lsize(P, SO), t.Mh64.get(), t.Lh64.get());
-    harm_unfold<P, double>(t, t.Lh64, t.L.get(), Op<P>::LS, st);
-    return;
+  if constexpr (P < kM2LBalancedOrder) {
+    if (m2l_parts(t, P)) {
+      m2l_plain_run<P, true>(t, n, tile, g0, g1, st);
+      return;
+    }
   }
-  constexpr int W = m2l_waves<P, SO, double>();
-  const unsigned* idx = ensure_index_table<P, W>(t, st);
-  k_m2l_gemm<P, SO, double, false, W><<<grid, 64 * W, 0, st>>>(
-      n, grid, S.tile_cells.get(), tile, g0, g1, S.group_key.get(),
-      S.group_src.get(), S.key_dlevel.get(), S.Dtab64.get(), idx, t.tile_order_ptr(), nullptr, Op<P>::MS,
-      Op<P>::MS, Op<P>::LS, t.M.get(), t.L.get());
+  m2l_plain_run<P, false>(t, n, tile, g0, g1, st);
 }
 
 // L2L (example/calculate.cpp:219-234), x = child - parent, one thread per

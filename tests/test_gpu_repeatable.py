@@ -1,5 +1,6 @@
 """Plain FP64 evaluations of sets whose leaves are cut into several near-field
-items give the same bits every time, and agree with the oracle's sums."""
+items, and below order 6 whose M2L tiles are cut into several chunks, give the
+same bits every time and agree with the oracle's sums."""
 import numpy as np
 import pytest
 import torch
@@ -44,4 +45,18 @@ def test_near_field_repeats(gpu, n, ncrit, so):
     print(f"near field so={so} n={n} ncrit={ncrit}", flush=True)
     got = _repeat(t, n, outsz, 8, phases=P2P)
     want = O.OracleTree(pos, S, ncrit, 3, 0.5, source_order=so, outputsize=outsz).compute_field_fmm(mask=P2P)
+    assert util.rel_norm(got, want) <= 1e-12
+
+
+@pytest.mark.parametrize("n,ncrit,so,order,form", [
+    (2000, 64, 0, 4, "auto"), (2000, 8, 0, 1, "auto"), (2000, 64, 0, 5, "harmonic"), (700, 64, 0, 5, "full"),
+    (30000, 32, 0, 3, "auto"), (30000, 32, 0, 5, "full"), (9000, 64, 1, 2, "auto"), (9000, 64, 1, 5, "harmonic"),
+    (9000, 64, 2, 3, "auto"), (9000, 64, 2, 5, "harmonic")])
+def test_evaluation_repeats(gpu, n, ncrit, so, order, form):
+    pos, S, t = _tree(n, ncrit, so, order)
+    t.set_m2l_form(form)
+    outsz = 3 if so == 1 else 4
+    print(f"so={so} n={n} order={order} {form}: {t.info()['m2l_groups']} groups", flush=True)
+    got = _repeat(t, n, outsz, 8)
+    want = O.OracleTree(pos, S, ncrit, order, 0.5, source_order=so, outputsize=outsz).compute_field_fmm()
     assert util.rel_norm(got, want) <= 1e-12
