@@ -62,8 +62,9 @@ __host__ __device__ constexpr int sourcesize(int so) { return nterms(so) - nterm
 //   * inside a build (MemScope) a freed block is reused by the same thread on
 //     the same stream only, in stream order;
 //   * at most kIdleBytes are kept (the oldest go first), none longer than
-//     kIdleBuilds builds and destroyed trees without use, and all are given back when an
-//     allocation fails;
+//     kIdleBuilds builds and destroyed trees without use; when an allocation fails, they
+//     and those the running build has freed are given back, and the exact size is
+//     asked for if its size class still does not fit;
 //   * blocks belong to the device they were allocated on; every function may
 //     be called from any thread.
 constexpr size_t kIdleBytes = (size_t)4 << 30;

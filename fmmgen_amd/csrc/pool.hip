@@ -88,18 +88,31 @@ void* device_alloc(size_t bytes) {
     }
   }
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, want);
-  if (e == hipErrorOutOfMemory) {  // give the kept blocks back and try again
+  size_t got = want;
+  hipError_t e = hipMalloc(&p, got);
+  if (e == hipErrorOutOfMemory) {  // give back what is kept, then ask for no more than is needed
     (void)hipGetLastError();
     {
       std::lock_guard<std::mutex> lock(P.mu);
       while (!P.idle.empty()) drop(P, P.idle.begin());
+      for (MemScope* s = t_scope; s; s = s->outer) {  // hipFree waits for the work on them
+        for (auto& f : s->free) {
+          P.blocks.erase(f.second);
+          (void)hipFree(f.second);
+        }
+        s->free.clear();
+      }
     }
-    e = hipMalloc(&p, want);
+    e = hipMalloc(&p, got);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      got = std::max<size_t>(bytes, 1);
+      e = hipMalloc(&p, got);
+    }
   }
   FMM_HIP(e);
   std::lock_guard<std::mutex> lock(P.mu);
-  P.blocks[p] = Block{want, dev};
+  P.blocks[p] = Block{got, dev};
   return p;
 }
 
