@@ -8,12 +8,12 @@
 from .codegen import generate_code, Nterms, Msize, Lsize, generate_mappings
 
 __all__ = ["generate_code", "Nterms", "Msize", "Lsize", "generate_mappings", "build_tree", "Tree",
-           "direct_sum"]
+           "direct_sum", "trim_memory"]
 
 
 def __getattr__(name):
     # torch is imported lazily so the generator works without it
-    if name in ("build_tree", "Tree", "direct_sum", "op_batch"):
+    if name in ("build_tree", "Tree", "direct_sum", "op_batch", "trim_memory"):
         from . import tree
         return getattr(tree, name)
     raise AttributeError(name)

@@ -32,6 +32,7 @@ OPS = {"P2M": 0, "M2M": 1, "M2L": 2, "L2L": 3, "L2P": 4, "M2P": 5, "P2P": 6, "P2
 # Every symbol include/fmm_hip.h declares.
 EXPORTS = (
     "fmm_last_error", "fmm_abi_version", "fmm_variant_orders", "fmm_tree_build", "fmm_tree_destroy",
+    "fmm_trim_memory",
     "fmm_tree_info", "fmm_tree_set_sources", "fmm_evaluate", "fmm_evaluate_phases", "fmm_evaluate_bh",
     "fmm_direct_sampled",
     "fmm_op_batch", "fmm_export_cells", "fmm_export_particles", "fmm_export_lists", "fmm_export_expansions",
@@ -79,6 +80,7 @@ def load(path=None):
     L.fmm_variant_orders.argtypes = [ci, ci, i_p, i_p]
     L.fmm_tree_build.argtypes = [vp, vp, sz, sz, ci, cd, ci, ci, vp, ctypes.POINTER(vp)]
     L.fmm_tree_destroy.argtypes = [vp]
+    L.fmm_trim_memory.argtypes = [sz, ctypes.POINTER(sz)]
     L.fmm_tree_info.argtypes = [vp, ll_p]
     L.fmm_tree_set_sources.argtypes = [vp, vp]
     L.fmm_evaluate.argtypes = [vp, ci, vp, vp]

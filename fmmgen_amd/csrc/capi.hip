@@ -168,6 +168,13 @@ int fmm_tree_destroy(fmm_tree_t tree) {
   });
 }
 
+int fmm_trim_memory(size_t keep_bytes, size_t* kept_bytes) {
+  return guarded([&] {
+    const size_t kept = trim_memory(keep_bytes);
+    if (kept_bytes) *kept_bytes = kept;
+  });
+}
+
 int fmm_timing_enable(fmm_tree_t tree, int enable) {
   return guarded([&] {
     FMM_CHECK(tree, kInvalidArgument, "NULL tree");

@@ -65,12 +65,16 @@ __host__ __device__ constexpr int sourcesize(int so) { return nterms(so) - nterm
 //     kIdleBuilds builds and destroyed trees without use; when an allocation fails, they
 //     and those the running build has freed are given back, and the exact size is
 //     asked for if its size class still does not fit;
+//   * trim_memory gives them back on request (fmm_trim_memory), the oldest first,
+//     until at most `keep` bytes stay, and returns what stays: other users of the
+//     device, a framework's own allocator above all, cannot reach them otherwise;
 //   * blocks belong to the device they were allocated on; every function may
 //     be called from any thread.
 constexpr size_t kIdleBytes = (size_t)4 << 30;
 constexpr unsigned kIdleBuilds = 32;
 void* device_alloc(size_t bytes);
 void device_free(void* p);
+size_t trim_memory(size_t keep);
 
 // Buffers that this thread allocates and frees while it lives belong to work on
 // one stream.

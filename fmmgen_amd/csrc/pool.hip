@@ -51,6 +51,15 @@ void drop(Pool& P, Map::iterator it) {
   P.idle.erase(it);
 }
 
+void shrink_to(Pool& P, size_t bytes) {  // the oldest go first
+  while (P.idle_bytes > bytes) {
+    auto old = P.idle.begin();
+    for (auto it = P.idle.begin(); it != P.idle.end(); ++it)
+      if (P.epoch - it->second.epoch > P.epoch - old->second.epoch) old = it;
+    drop(P, old);
+  }
+}
+
 void keep_idle(Pool& P, void* p) {  // no work on the block is pending
   const Block b = P.blocks[p];
   if (b.bytes > kIdleBytes) {
@@ -58,12 +67,7 @@ void keep_idle(Pool& P, void* p) {  // no work on the block is pending
     (void)hipFree(p);
     return;
   }
-  while (P.idle_bytes + b.bytes > kIdleBytes) {  // the oldest go first
-    auto old = P.idle.begin();
-    for (auto it = P.idle.begin(); it != P.idle.end(); ++it)
-      if (P.epoch - it->second.epoch > P.epoch - old->second.epoch) old = it;
-    drop(P, old);
-  }
+  shrink_to(P, kIdleBytes - b.bytes);
   P.idle.insert({{b.device, b.bytes}, {p, P.epoch}});
   P.idle_bytes += b.bytes;
 }
@@ -94,7 +98,7 @@ void* device_alloc(size_t bytes) {
     (void)hipGetLastError();
     {
       std::lock_guard<std::mutex> lock(P.mu);
-      while (!P.idle.empty()) drop(P, P.idle.begin());
+      shrink_to(P, 0);
       for (MemScope* s = t_scope; s; s = s->outer) {  // hipFree waits for the work on them
         for (auto& f : s->free) {
           P.blocks.erase(f.second);
@@ -128,6 +132,13 @@ void device_free(void* p) {
     P.blocks.erase(p);
   }
   (void)hipFree(p);  // waits for the device: nothing is known about pending work
+}
+
+size_t trim_memory(size_t keep) {
+  Pool& P = pool();
+  std::lock_guard<std::mutex> lock(P.mu);
+  shrink_to(P, keep);
+  return P.idle_bytes;
 }
 
 MemScope::MemScope(hipStream_t s) : st(s), outer(t_scope) {

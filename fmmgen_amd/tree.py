@@ -328,6 +328,16 @@ def build_tree(pos, S, nparticles, ncrit, order, theta, source_order=0, potentia
     return Tree(h, pos, S, n, int(ncrit), int(order), float(theta), int(source_order), potential, field)
 
 
+def trim_memory(keep_bytes=0):
+    """Gives device memory that the library keeps for later trees (4 GiB at
+    most, include/fmm_hip.h) back to the device until at most ``keep_bytes``
+    stay, for other users of the GPU, torch's allocator among them; returns
+    the bytes that stay.  Live trees are not touched."""
+    kept = ctypes.c_size_t()
+    _lib.check(_lib.load().fmm_trim_memory(int(keep_bytes), ctypes.byref(kept)))
+    return kept.value
+
+
 def direct_sum(pos, S, targets, F=None, source_order=0, outsz=4):
     """FP64 direct sum at ``targets`` over every particle (self excluded)."""
     _check_dev(pos, "pos", 3)

@@ -92,6 +92,17 @@ int fmm_tree_build(const double* d_pos, const double* d_S, size_t n, size_t ncri
                    int source_order, int output_size, void* stream, fmm_tree_t* out);
 int fmm_tree_destroy(fmm_tree_t tree);
 
+/* Device memory kept between trees.  Buffers that a build or a destroyed tree
+ * no longer needs stay with the library for the next trees (allocating and
+ * freeing them anew took two thirds of a build of 3e5 particles): at most 4
+ * GiB, none longer than 32 builds and destroyed trees without use, all given back when one of
+ * the library's own allocations fails.  Other users of the device, a framework's
+ * allocator among them, cannot reach that memory: this call gives it back until
+ * at most keep_bytes stay (0: all of it) and reports what stays (kept_bytes may be NULL).
+ * It may be called at any time and from any thread; live trees are not touched.
+ * No counterpart in the reference. */
+int fmm_trim_memory(size_t keep_bytes, size_t* kept_bytes);
+
 /* info must hold FMM_TREE_INFO_LEN entries:
  * info[0..12] = ncells, nleaves, levels, n_m2l, n_p2p, n, order,
  * source_order, P2P particle pairs (self pairs excluded), ncrit,

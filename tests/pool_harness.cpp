@@ -139,6 +139,19 @@ static int threads() {
   return 0;
 }
 
+// On request: all of it, or down to a size.
+static int trim() {
+  build({40 * MB});
+  build({20 * MB, 30 * MB});
+  CHECK(trim_memory(60 * MB) <= 60 * MB && in_use <= 60 * MB && in_use >= 50 * MB);  // the oldest went
+  void* p = device_alloc(5 * MB);
+  CHECK(trim_memory(0) == 0);
+  CHECK(in_use >= 5 * MB && in_use < 7 * MB);  // what is in use stays
+  device_free(p);
+  CHECK(in_use == 0);
+  return 0;
+}
+
 // A block goes to builds on its own device only.
 static int devices() {
   build({50 * MB});
@@ -155,7 +168,8 @@ static int devices() {
 int main(int argc, char** argv) {
   const std::map<std::string, int (*)()> checks = {
       {"scope_gives_back", scope_gives_back}, {"exact_size", exact_size}, {"idle_gives_back", idle_gives_back},
-      {"bounded", bounded},                   {"threads", threads},       {"devices", devices}};
+      {"bounded", bounded},                   {"threads", threads},       {"devices", devices},
+      {"trim", trim}};
   auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   try {

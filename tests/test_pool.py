@@ -23,7 +23,13 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["scope_gives_back", "exact_size", "idle_gives_back", "bounded", "threads", "devices"])
+@pytest.mark.parametrize("check", ["scope_gives_back", "exact_size", "idle_gives_back", "bounded", "threads", "devices",
+                                   "trim"])
 def test_pool(harness, check):
     r = subprocess.run([harness, check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout
+
+
+def test_trim_without_kept_memory():
+    import fmmgen_amd
+    assert fmmgen_amd.trim_memory() == 0
