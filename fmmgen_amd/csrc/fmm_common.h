@@ -216,6 +216,15 @@ struct P2PItems {
   DevBuf<long long> row_off;  // [ncells + 1] first row of a leaf's items
 };
 
+// Entries of the M2L list's buffer that a build of n particles begins with (half
+// as many for P2P; both double when they run full).  16 a particle hold the lists
+// at 64 particles a leaf and theta 0.5 with at most one doubling.  Not more than
+// 2 GiB of keys: a list has less than 2^31 entries however many particles there are, and
+// large sets with large leaves need few.
+constexpr long long list_entries(size_t n) {
+  return std::min<long long>(std::max<long long>(1 << 16, 16LL * (long long)n), 1LL << 28);
+}
+
 // ------------------------------------------------------------ tree handle
 struct Tree {
   // configuration (example/tree.hpp:78-95 + generated macros)

@@ -996,8 +996,7 @@ void build_lists_device(Tree& t, hipStream_t st) {
   DevBuf<int> maxq;
   const int kb = bits_for((unsigned long long)t.ncells - 1);
   long long n_m2l = 0, n_p2p = 0;
-  // about 27 M2L and 9 P2P entries a particle at 64 particles a leaf
-  long long cap_m2l = std::max<long long>(1 << 16, 16LL * (long long)t.n), cap_p2p = cap_m2l / 2;
+  long long cap_m2l = list_entries(t.n), cap_p2p = cap_m2l / 2;
   m2l.alloc(cap_m2l);
   p2p.alloc(cap_p2p);
   cur.alloc(1);

@@ -165,11 +165,20 @@ static int devices() {
   return 0;
 }
 
+// The list buffers of a build: proportional to small sets, a few GiB for the largest.
+static int list_buffers() {
+  CHECK(list_entries(1) == 1 << 16);
+  CHECK(list_entries((size_t)1 << 20) == 16LL << 20);
+  CHECK(list_entries((size_t)1 << 24) == 16LL << 24);
+  CHECK(8 * list_entries(((size_t)1 << 31) - 1) <= 2LL << 30);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, int (*)()> checks = {
       {"scope_gives_back", scope_gives_back}, {"exact_size", exact_size}, {"idle_gives_back", idle_gives_back},
       {"bounded", bounded},                   {"threads", threads},       {"devices", devices},
-      {"trim", trim}};
+      {"trim", trim},                         {"list_buffers", list_buffers}};
   auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   try {

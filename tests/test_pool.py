@@ -1,5 +1,6 @@
 """Device memory kept between trees (csrc/pool.hip): what is kept, for how long
-and when it is given back, with a host allocator in the place of the device's."""
+and when it is given back, with a host allocator in the place of the device's;
+and the sizes of a build's first list buffers."""
 import os
 import subprocess
 
@@ -24,7 +25,7 @@ def harness(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["scope_gives_back", "exact_size", "idle_gives_back", "bounded", "threads", "devices",
-                                   "trim"])
+                                   "trim", "list_buffers"])
 def test_pool(harness, check):
     r = subprocess.run([harness, check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout
