@@ -53,7 +53,9 @@ def _adds_in_place(out, size, inp):
             or out.numel() != size or size == 0 or not out.is_contiguous()
             or out.requires_grad or out.is_inference() or out.is_neg()):
         return False
-    return out.untyped_storage().data_ptr() != inp.untyped_storage().data_ptr()
+    # by address: one allocation can be reached through several storages (dlpack)
+    a, b = out.data_ptr(), inp.data_ptr()
+    return a + 8 * size <= b or b + inp.element_size() * inp.numel() <= a
 
 
 class Library:
