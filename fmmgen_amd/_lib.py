@@ -33,7 +33,7 @@ OPS = {"P2M": 0, "M2M": 1, "M2L": 2, "L2L": 3, "L2P": 4, "M2P": 5, "P2P": 6, "P2
 EXPORTS = (
     "fmm_last_error", "fmm_abi_version", "fmm_variant_orders", "fmm_tree_build", "fmm_tree_destroy",
     "fmm_trim_memory",
-    "fmm_tree_info", "fmm_tree_set_sources", "fmm_evaluate", "fmm_evaluate_phases", "fmm_evaluate_bh",
+    "fmm_tree_info", "fmm_tree_items_f64", "fmm_tree_set_sources", "fmm_evaluate", "fmm_evaluate_phases", "fmm_evaluate_bh",
     "fmm_direct_sampled",
     "fmm_op_batch", "fmm_export_cells", "fmm_export_particles", "fmm_export_lists", "fmm_export_expansions",
     "fmm_timing_enable", "fmm_timing_read",
@@ -82,6 +82,7 @@ def load(path=None):
     L.fmm_tree_destroy.argtypes = [vp]
     L.fmm_trim_memory.argtypes = [sz, ctypes.POINTER(sz)]
     L.fmm_tree_info.argtypes = [vp, ll_p]
+    L.fmm_tree_items_f64.argtypes = [vp, ll_p, ll_p]
     L.fmm_tree_set_sources.argtypes = [vp, vp]
     L.fmm_evaluate.argtypes = [vp, ci, vp, vp]
     L.fmm_evaluate_phases.argtypes = [vp, ci, ci, vp, vp]

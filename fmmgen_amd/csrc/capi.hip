@@ -223,6 +223,15 @@ int fmm_tree_info(fmm_tree_t tree, long long* info) {
   });
 }
 
+int fmm_tree_items_f64(fmm_tree_t tree, long long* p2p, long long* m2l) {
+  return guarded([&] {
+    FMM_CHECK(tree && p2p && m2l, kInvalidArgument, "NULL argument");
+    const Tree& t = tree->t;
+    *p2p = t.p2p_items(true).count;
+    *m2l = t.sched.nchunks64 > 0 ? t.sched.nchunks64 : t.sched.nchunks;
+  });
+}
+
 int fmm_tree_set_sources(fmm_tree_t tree, const double* d_S) {
   return guarded([&] {
     FMM_CHECK(tree && d_S, kInvalidArgument, "NULL argument");

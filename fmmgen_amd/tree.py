@@ -215,7 +215,11 @@ class Tree:
         keys = ("ncells", "nleaves", "levels", "n_m2l", "n_p2p", "n", "order", "source_order",
                 "p2p_particle_pairs", "ncrit", "m2l_tiles", "m2l_groups", "m2l_keys", "p2p_items",
                 "m2l_chunks")
-        return dict(zip(keys, list(a)))
+        out = dict(zip(keys, list(a)))
+        p2p, m2l = ctypes.c_longlong(), ctypes.c_longlong()
+        _lib.check(_lib.load().fmm_tree_items_f64(self._h, ctypes.byref(p2p), ctypes.byref(m2l)))
+        out.update(p2p_items_f64=p2p.value, m2l_chunks_f64=m2l.value)
+        return out
 
     def timing(self, enable):
         """Switches stream-ordered per-phase hipEvent timing on or off (resets totals)."""

@@ -107,11 +107,14 @@ int fmm_trim_memory(size_t keep_bytes, size_t* kept_bytes);
  * info[0..12] = ncells, nleaves, levels, n_m2l, n_p2p, n, order,
  * source_order, P2P particle pairs (self pairs excluded), ncrit,
  * M2L target tiles, M2L (tile, offset) groups, distinct M2L offsets;
- * info[13] = P2P work items (source segments of the target leaves);
- * info[14] = M2L work items (runs of groups of one tile);
- * info[15] = 0 (reserved) */
+ * info[13] = P2P work items (source segments of the target leaves) and
+ * info[14] = M2L work items (runs of groups of one tile) of the mixed and
+ * learned modes; info[15] = 0 (reserved) */
 #define FMM_TREE_INFO_LEN 16
 int fmm_tree_info(fmm_tree_t tree, long long* info);
+/* Work items of the plain FP64 evaluation, which are cut finer on small sets:
+ * P2P and M2L. */
+int fmm_tree_items_f64(fmm_tree_t tree, long long* p2p, long long* m2l);
 
 /* Rebinds the borrowed source strengths (same geometry, new sources). */
 int fmm_tree_set_sources(fmm_tree_t tree, const double* d_S);

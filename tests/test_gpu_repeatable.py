@@ -60,3 +60,14 @@ def test_evaluation_repeats(gpu, n, ncrit, so, order, form):
     got = _repeat(t, n, outsz, 8)
     want = O.OracleTree(pos, S, ncrit, order, 0.5, source_order=so, outputsize=outsz).compute_field_fmm()
     assert util.rel_norm(got, want) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [2000, 60000])
+def test_small_sets_are_cut_finer_in_fp64(gpu, n):
+    """The lists that the tests above are about: the FP32 ones stay as they are
+    (their sums depend on the cut)."""
+    inf = _tree(n, 64, 0)[2].info()
+    print(inf, flush=True)
+    # an item a leaf, or a segment of 8192 sources beside a dense cluster
+    assert inf["nleaves"] <= inf["p2p_items"] < inf["p2p_items_f64"]
+    assert inf["m2l_chunks"] < inf["m2l_chunks_f64"]
