@@ -1,8 +1,7 @@
 // Order-selection network: a 3-layer perceptron (F inputs, two hidden ReLU
-// layers of H units, O outputs) with FP32 weights.  Training kernels
-// (forward with saved activations, masked mean-square loss, backward,
-// weight gradients, Adam) run in FP32; inference runs in FP16 with FP32
-// accumulation.  The network has no counterpart in the reference: it picks
+// layers of H units, O outputs) with FP32 weights.  Training (the gradient of
+// the masked mean-square loss, forward and backward in one kernel, and Adam)
+// runs in FP32; inference runs in FP16 with FP32 accumulation.  The network has no counterpart in the reference: it picks
 // per leaf cell the lowest expansion order whose predicted error meets a
 // field tolerance.
 //
@@ -21,11 +20,28 @@ constexpr int kMlpOrder0 = 2;  // order of output 0 (orders 2 .. 12)
 constexpr int kMlpW1 = 0, kMlpB1 = kMlpW1 + kMlpH * kMlpF, kMlpW2 = kMlpB1 + kMlpH, kMlpB2 = kMlpW2 + kMlpH * kMlpH,
               kMlpW3 = kMlpB2 + kMlpH, kMlpB3 = kMlpW3 + kMlpO * kMlpH, kMlpParams = kMlpB3 + kMlpO;
 
-// Workspace of one training batch of B samples (device floats).
-constexpr size_t mlp_work_floats(int B) { return (size_t)B * (2 * kMlpH + kMlpO) * 2 + 1; }
+// Blocks of the gradient: runs of sample tiles, two tiles at least and kGradBlocks
+// runs at most; a block leaves a row of sums (the gradient, its loss, its count of
+// valid outputs) in the workspace.  Batches of up to kGradOneBlock samples (three
+// tiles) run in one block, which finishes by itself (a call with 32 samples 12.3
+// us, with 41 in one block 15.8 us, with 42 in two blocks and two launches 15.2 us).
+constexpr int kGradTile = 16, kGradBlocks = 128, kGradOneBlock = 41, kGradRow = kMlpParams + 2;
+struct GradGrid {
+  int blocks, per;  // tiles a block
+};
+constexpr GradGrid mlp_grad_grid(int B) {
+  const int tiles = B / kGradTile + (B % kGradTile > 0);
+  if (B <= kGradOneBlock) return GradGrid{1, tiles};
+  const int run = (tiles + kGradBlocks - 1) / kGradBlocks, per = run > 2 ? run : 2;
+  return GradGrid{(tiles + per - 1) / per, per};
+}
 
-// Largest batch of the allocation-free gradient (its workspace is a fixed
-// device array of mlp_work_floats(kMlpScratchBatch) floats, 9.1 MB).
+// Workspace of the gradient of B samples (device floats).
+constexpr size_t mlp_work_floats(int B) { return (size_t)mlp_grad_grid(B).blocks * kGradRow; }
+
+// Largest batch of the allocation-free gradient.  Its workspace, a fixed device
+// array of kGradBlocks rows (2.9 MB), would hold any batch; larger ones stay
+// refused, as callers know the call.
 constexpr int kMlpScratchBatch = 8192;
 
 // FP32 forward: Y[B][O].

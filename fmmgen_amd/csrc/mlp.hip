@@ -1,7 +1,6 @@
 // Kernels of the order-selection network (layout and semantics in mlp.h).
 #include "mlp.h"
 
-#include <algorithm>
 #include <mutex>
 
 namespace fmm {
@@ -67,9 +66,8 @@ __global__ __launch_bounds__(64) void k_mlp_fwd(int B, const float* __restrict__
 // 5.6e-7 to 1.1e-7.
 // Operand layout of the 16x16x4 MFMA: lane l holds A[l%16][l/16],
 // B[l/16][l%16] and rows 4 (l/16) + r of column l%16 of the result.
-constexpr int kGradWaves = 4, kGradTile = 16;
-constexpr int kGradRow = kMlpParams + 2;  // a block's row: the gradient, its loss, its count
-constexpr int kOP = 16;                   // outputs padded to a tile
+constexpr int kGradWaves = 4;
+constexpr int kOP = 16;  // outputs padded to a tile
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) {
@@ -304,7 +302,7 @@ inline int nb(long long n, int bs) { return (int)((n + bs - 1) / bs); }
 // a host-side stand-in, never the device array: host code uses only the
 // per-device address from hipGetSymbolAddress.  Nothing in it has to start
 // at zero (every kernel writes what it later reads).
-static __device__ __align__(256) float scratch[mlp_work_floats(kMlpScratchBatch)];
+static __device__ __align__(256) float scratch[kGradBlocks * kGradRow];
 
 constexpr int kMaxDevices = 64;
 
@@ -331,19 +329,12 @@ void mlp_forward(int B, const float* X, const float* params, float* Y, hipStream
   k_mlp_fwd<<<nb(B, 64), 64, 0, st>>>(B, X, params, Y);
 }
 
-// Blocks of the gradient: two sample tiles each, at most kGradBlocks of them, and no more rows than the workspace
-// holds; a batch whose rows would not fit (below 42 samples) runs in one block.
-constexpr int kGradBlocks = 128;
-
 void mlp_grad(int B, const float* X, const float* T, const float* mask, const float* params, float* grad,
               float* loss, float* work, hipStream_t st) {
   FMM_CHECK(B > 0, kInvalidArgument, "empty batch");
-  const int tiles = nb(B, kGradTile);
-  const int rows = (int)std::min<size_t>(kGradBlocks, mlp_work_floats(B) / kGradRow);
-  const int per = std::max(2, nb(tiles, std::max(rows, 1)));
-  const int blocks = rows < 2 ? 1 : nb(tiles, per);
-  k_mlp_grad<<<blocks, 64 * kGradWaves, 0, st>>>(B, blocks == 1 ? tiles : per, X, T, mask, params, work, grad, loss);
-  if (blocks > 1) k_mlp_grad_sum<<<nb(kMlpParams + 1, 64), 256, 0, st>>>(blocks, work, grad, loss);
+  const GradGrid g = mlp_grad_grid(B);
+  k_mlp_grad<<<g.blocks, 64 * kGradWaves, 0, st>>>(B, g.per, X, T, mask, params, work, grad, loss);
+  if (g.blocks > 1) k_mlp_grad_sum<<<nb(kMlpParams + 1, 64), 256, 0, st>>>(g.blocks, work, grad, loss);
 }
 
 void mlp_adam(const float* grad, float* params, float* m, float* v, float lr, float beta1, float beta2, float eps,

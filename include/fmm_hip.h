@@ -205,7 +205,7 @@ int fmm_mlp_grad(const float* d_X, const float* d_T, const float* d_mask, int B,
  * cannot allocate device memory (code under HIP graph capture, tight
  * training loops).  The workspace is a fixed array inside the library, one
  * per device, of fmm_mlp_work_floats(FMM_MLP_NOALLOC_MAX_BATCH) floats
- * (9.1 MB, held until the process ends); B above FMM_MLP_NOALLOC_MAX_BATCH
+ * (2.9 MB, held until the process ends); B above FMM_MLP_NOALLOC_MAX_BATCH
  * is FMM_ERR_INVALID_ARGUMENT.  Calls that overlap on one device share the
  * array and race; calls ordered on one stream do not. */
 #define FMM_MLP_NOALLOC_MAX_BATCH 8192
