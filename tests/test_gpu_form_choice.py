@@ -48,3 +48,19 @@ def test_mixed_choice_by_groups(gpu, so, n, many, mode):
     print(f"so={so} n={n} {mode} {t.info()['m2l_groups']} groups", flush=True)
     t.compute_field_fmm(F, mode=mode)
     assert util.rel_norm(F.cpu().numpy()[:, pot:], want[:, pot:]) < 1e-6
+
+
+@pytest.mark.parametrize("pot,field,order", [(True, False, 0), (True, False, 1), (True, True, 1), (False, True, 1)])
+@pytest.mark.parametrize("n,form", [(700, "harmonic"), (30000, "auto"), (30000, "full")])
+def test_lowest_orders(gpu, pot, field, order, n, form):
+    """The automatic form is harmonic on large sets at every order, the lowest ones included."""
+    from fmmgen_amd import build_tree
+    pos, S = util.blobs(n, 71), np.random.default_rng(72).uniform(-1, 1, (n, 1))
+    outsz = int(pot) + 3 * int(field)
+    t = build_tree(_dev(pos), _dev(S), n, 32, order, 0.5, potential=pot, field=field)
+    t.set_m2l_form(form)
+    want = O.OracleTree(pos, S, 32, order, 0.5, outputsize=outsz).compute_field_fmm()
+    F = torch.empty(n, outsz, dtype=torch.float64, device="cuda")
+    print(f"order {order} n={n} {form}", flush=True)
+    t.compute_field_fmm(F, mode="plain")
+    assert util.rel_norm(F.cpu().numpy(), want) < 1e-12
