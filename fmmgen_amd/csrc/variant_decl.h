@@ -39,7 +39,8 @@ void m2l_class(Tree& t, int mode, const int* chunks, int nch, int ps, hipStream_
 // Whether the M2L of an evaluation runs in the harmonic layout (p: the order
 // the expansions are stored at).  Automatic: charges in the mixed and learned
 // modes always; otherwise where the shorter GEMM pays for the fold and unfold
-// launches, which is everywhere but at few groups and low order.  Measured
+// launches, which is everywhere but at few groups and low order, and, for dipoles
+// and quadrupoles in the mixed modes, only where it rounds no worse.  Measured
 // (full -> harmonic, one evaluation, theta 0.5, ncrit 64):
 //   FP64 charges   2^22 blobs, order 10 147 -> 66.6 ms; 2^20 uniform, order 8
 //                  11.2 -> 8.9 ms, order 2 6.73 -> 6.55 ms; 10^5 (156k groups)
@@ -47,11 +48,19 @@ void m2l_class(Tree& t, int mode, const int* chunks, int nch, int ps, hipStream_
 //                  us, order 6 318 -> 313 us
 //   FP32 dipoles   10^6 Plummer, theta 0.4, order 6 18.5 -> 13.5 ms; 10^5
 //                  order 4 927 -> 917 us; 2000 302 -> 311 us
+// Far-field error of the harmonic over the full form against FP64, mean of 12
+// sets (uniform, blobs, Plummer, mixed; theta 0.4 to 0.55):
+//   FP32    dipoles order 2 1.00, orders 3 to 8 0.85 to 0.95; quadrupoles orders
+//           3 to 5 0.79 to 0.93, 6 1.07, 7 and 8 0.90
+//   BF16x3  dipoles 1.00 to 1.01 (up to 1.03), quadrupoles 1.08 to 1.10 (up to
+//           1.17): a folded multipole is split as one value
 constexpr int kHarmMinOrder = 6, kHarmMinGroups = 1 << 14, kHarmMinGroupsMixed = 1 << 17;
 inline bool m2l_harmonic(const Tree& t, int mode, int p) {
   if (t.m2l_form == kM2LFull) return false;
   if (t.m2l_form == kM2LHarmonic) return true;
-  if (mode != 0) return SO == 0 || t.sched.ngroups >= kHarmMinGroupsMixed;
+  if (mode != 0 && SO > 0)
+    return mode == 1 && p >= 3 && !(SO == 2 && p == 6) && t.sched.ngroups >= kHarmMinGroupsMixed;
+  if (mode != 0) return true;
   return p >= kHarmMinOrder || t.sched.ngroups >= kHarmMinGroups;
 }
 

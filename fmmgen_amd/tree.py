@@ -67,9 +67,11 @@ class Tree:
             self._h = None
 
     def set_m2l_form(self, form):
-        """Operand form of the M2L translation: "auto" (the faster
-        one: harmonic, except for plain FP64 at orders below 6, and for the
-        mixed modes of dipoles and quadrupoles, on small sets), "full" (the generated
+        """Operand form of the M2L translation: "auto" (harmonic where it is the
+        faster one and rounds no worse: charges in the mixed and learned modes,
+        plain FP64 from order 6 or 2^14 groups on, FP32 dipoles and quadrupoles
+        from order 3 and 2^17 groups on, order 6 of quadrupoles excepted; else
+        full), "full" (the generated
         operator's sums over every multi-index) or "harmonic" (folded
         multipoles and the local rows with n_z <= 1: the same expansions by
         the harmonicity of 1/R, (p+1)^2 rows and columns instead of

@@ -220,9 +220,10 @@ int fmm_mlp_adam(const float* d_grad, float* d_params, float* d_m, float* d_v, f
 int fmm_tree_set_order(fmm_tree_t tree, int order);
 /* Operand form of the M2L translation (no counterpart in the reference,
  * whose M2L is the generated operator, fmmgen/expansions.py:144-172):
- *   FMM_M2L_AUTO (default): the faster of the two for the mode, order and
- *     size: harmonic, except for plain FP64 and for dipoles and quadrupoles
- *     on small sets;
+ *   FMM_M2L_AUTO (default): harmonic where it is the faster one and rounds no
+ *     worse: charges in the mixed and learned modes; plain FP64 from order 6 or
+ *     2^14 groups on; FP32 dipoles and quadrupoles from order 3 and 2^17 groups on,
+ *     order 6 of quadrupoles excepted; else the full form;
  *   FMM_M2L_FULL: the generated operator's sums over every multi-index;
  *   FMM_M2L_HARMONIC: the same local expansions from folded multipoles and
  *     the rows with n_z <= 1 only ((p+1)^2 instead of C(p+3,3) per side,

@@ -10,6 +10,7 @@ from oracle import oracle as O
 from tests import util
 
 pytestmark = pytest.mark.gpu
+P2P = 8
 
 
 def _dev(a):
@@ -64,3 +65,26 @@ def test_lowest_orders(gpu, pot, field, order, n, form):
     print(f"order {order} n={n} {form}", flush=True)
     t.compute_field_fmm(F, mode="plain")
     assert util.rel_norm(F.cpu().numpy(), want) < 1e-12
+
+
+@pytest.mark.parametrize("mode,so,order,took", [
+    ("f32", 1, 3, "harmonic"), ("f32", 1, 8, "harmonic"), ("f32", 2, 3, "harmonic"),
+    ("f32", 2, 5, "harmonic"), ("f32", 2, 6, "full"), ("f32", 2, 7, "harmonic"),
+    ("bf16x3", 1, 8, "full"), ("bf16x3", 2, 3, "full"), ("bf16x3", 2, 8, "full"), ("f32", 0, 4, "harmonic"),
+    ("bf16x3", 0, 4, "harmonic")])
+def test_mixed_choice_by_rounding(gpu, mode, so, order, took):
+    """Above the size limit, dipoles and quadrupoles take the harmonic form in the
+    mixed modes only where it rounds no worse.  The far field of the automatic form
+    is nearer to that of the form it takes (the same roundings but for the order of
+    some additions) than to that of the other."""
+    n = 60000
+    _, _, t = _tree(n, 32, order, so)
+    assert t.info()["m2l_groups"] >= 1 << 17
+    out = {}
+    for form in ("full", "harmonic", "auto"):
+        t.set_m2l_form(form)
+        F = torch.empty(n, 3 if so == 1 else 4, dtype=torch.float64, device="cuda")
+        out[form] = t.compute_field_fmm(F, mode=mode, phases=63 & ~P2P)
+    d = {f: (out["auto"] - out[f]).norm().item() for f in ("full", "harmonic")}
+    print(f"so={so} order={order} {mode} distance to {d}", flush=True)
+    assert min(d, key=d.get) == took
