@@ -73,7 +73,9 @@ def harmonic_m2l(form, mode, so, order, ngroups):
         return False
     if form == "harmonic" or (mode != "plain" and so == 0):
         return True
-    return ngroups >= 1 << 17 if mode != "plain" else order >= 6 or ngroups >= 1 << 14
+    if mode == "plain":
+        return order >= 6 or ngroups >= 1 << 14
+    return mode == "f32" and order >= 3 and not (so == 2 and order == 6) and ngroups >= 1 << 17
 
 
 def cpu_baseline(cfg):
