@@ -585,15 +585,23 @@ __device__ __forceinline__ T chunk_sum(int slot, int n, int ls, const int* __res
   if (slot < 0) return v;
   const int t = slot / kTile, e = first[t + 1];
   const T* p = part + (size_t)(slot % kTile) * ls + n;
-#pragma unroll 4
-  for (int k = first[t]; k < e; ++k) v += p[(size_t)k * kTile * ls];
+  constexpr int B = 8;  // loads in flight (past the last chunk: that chunk again, not added)
+  for (int k = first[t]; k < e; k += B) {
+    T x[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) x[u] = p[(size_t)min(k + u, e - 1) * kTile * ls];
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (k + u < e) v += x[u];
+  }
   return v;
 }
 
 // Every cell's local row from the chunks' sums (the full form; the unfold of the
-// harmonic form adds them itself).  Takes the place of clearing L: 2000 particles,
-// order 4 54.5 -> 55.3 us an evaluation against atomic sums, 10^5 (unfold) 493 ->
-// 485 us.
+// harmonic form adds them itself).  Takes the place of clearing L.  Bound by the
+// latency of the chunks' loads, hence eight in flight: 2000 particles, order 4 55.3
+// (four and a remainder one by one) -> 53.5 us an evaluation, with the near field's
+// rows; 54.0 us with atomic sums of both.
 template <typename T>
 __global__ __launch_bounds__(256) void k_chunk_sum(int nc, int ls, const int* __restrict__ cell_slot,
                                                    const int* __restrict__ first, const T* __restrict__ part,

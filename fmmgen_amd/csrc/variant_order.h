@@ -351,8 +351,8 @@ __global__ __launch_bounds__(256) void k_l2l_wave(int beg, int end, const int* _
 // Near plus far field.  Fnear: a row a particle, or with row_off a row a work
 // item and target (the items of leaf c from row_off[c], pcount[c] rows each),
 // added in the items' order.  (Rows instead of atomics into one output, for the
-// sake of repeatable sums: 2000 particles 53.8 -> 54.5 us an evaluation, 10^5 516
-// -> 520 us, 2^20 7.16 -> 7.12 ms.)
+// sake of repeatable sums, with the M2L's by chunks: 2000 particles 54.0 -> 53.5 us
+// an evaluation, 10^5 493 -> 484 us, 2^20 7.06 -> 7.00 ms.)
 template <int P>
 __global__ __launch_bounds__(64) void k_l2p_final(int n, const int* __restrict__ leaf_of, const int* __restrict__ perm,
                             const double* __restrict__ cx, const double* __restrict__ cy,
@@ -368,11 +368,22 @@ __global__ __launch_bounds__(64) void k_l2p_final(int n, const int* __restrict__
 #pragma unroll
   for (int k = 0; k < OUT; ++k) acc[k] = Fnear && !row_off ? Fnear[(size_t)j * OUT + k] : 0.0;
   if (Fnear && row_off) {
-    const int nt = pcount[c];
-#pragma unroll 4
-    for (long long r = row_off[c] + (j - pstart[c]); r < row_off[c + 1]; r += nt)
+    const int nt = pcount[c], m = (int)((row_off[c + 1] - row_off[c]) / nt);  // items of the leaf
+    const double* row = Fnear + (size_t)(row_off[c] + (j - pstart[c])) * OUT;
+    constexpr int B = 4;  // rows in flight (past the last one: that one again, not added)
+    for (int i = 0; i < m; i += B) {
+      double x[B][OUT];
 #pragma unroll
-      for (int k = 0; k < OUT; ++k) acc[k] += Fnear[(size_t)r * OUT + k];
+      for (int u = 0; u < B; ++u)
+#pragma unroll
+        for (int k = 0; k < OUT; ++k) x[u][k] = row[(size_t)min(i + u, m - 1) * nt * OUT + k];
+#pragma unroll
+      for (int u = 0; u < B; ++u)
+        if (i + u < m) {
+#pragma unroll
+          for (int k = 0; k < OUT; ++k) acc[k] += x[u][k];
+        }
+    }
   }
   if (use_l2p) {
     fmmgen_ops::L2P_o<P, double>(px[j] - cx[c], py[j] - cy[c], pz[j] - cz[c], L + (size_t)c * Op<P>::LS, acc);
