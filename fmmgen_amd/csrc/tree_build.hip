@@ -51,10 +51,13 @@ __device__ __forceinline__ double rmax_of(double r) { return sqrt_rn((3.0 * r) *
 // any order first, which gives each run's range of s up to the bound E of
 // k_mean_scan; a run whose range lies in one binade is composed in parallel
 // (k_mean_steps), and k_mean_walk applies the pairs in order, 64 at a time,
-// adding one by one only in the runs that may leave their binade (a few of
-// them where s grows steadily).
+// adding one by one only in the runs that may leave their binade, and run by run
+// in their batches of 64: a dozen runs an axis where s grows steadily, but a
+// twentieth to a half of them where the set is centred and s wanders about zero.
 // The chain of additions, one lane per axis, took 1936 us at 300007 particles
-// and 27 ms at 2^22; this takes 110 us at 300007 (k_mean_walk 82).
+// and 27 ms at 2^22.  This takes 110 us at 300007 blob particles (k_mean_walk 89)
+// and 460 us at 2^22 (327); k_mean_walk alone takes 1341 us on 300007 and 3.8 ms on
+// 10^6 particles of a Plummer sphere about the origin.
 constexpr int kMeanChunk = 256;  // one wave per axis, 4 additions a lane
 constexpr int kMeanUnsafe = -100000;
 

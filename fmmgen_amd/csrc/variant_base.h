@@ -505,8 +505,8 @@ __device__ __forceinline__ void p2p_item(int it, int nitems, const int* __restri
 // in turn, so that dense regions are spread over all of them: at 2^22 blobs one
 // eighth of the items per XCD took 13.3 ms (FP32), runs of 256, 64 and 16 items
 // 11.1, 11.1 and 11.0 ms.  (Waves that stay and take items from eight counters
-// took 12.2 ms, and the counters themselves up to half the time of small sets:
-// 10^5 particles 547 us, now 255.)
+// took 12.2 ms, and the counters themselves took a third of the time of small
+// sets: 10^5 particles, FP32, 547 -> 344 us.)
 // FP64: four waves a SIMD (128 registers) against three, 18.5 -> 17.8 ms.
 constexpr int kP2PRun = 16;
 template <typename T>

@@ -131,11 +131,15 @@ class Tree:
         _lib.check(_lib.load().fmm_tree_leaf_error(self._h, _ptr(F), _ptr(Fref), _ptr(e), _stream()))
         return e
 
-    # Learned opening angle.  Costs of one learned evaluation in seconds per
-    # unit, measured on MI355X at 2^22 blobs (FP32 harmonic-form M2L, FP32
-    # near field): an M2L multiply-add of the harmonic form (full form), a
-    # near-field particle pair, and a (cell, expansion slot) of the upward
-    # and downward passes, which run at the largest order in use.
+    # Learned opening angle.  Prices of one learned evaluation in seconds per
+    # unit: an M2L multiply-add of the harmonic form (full form), a near-field
+    # particle pair, and a (cell, expansion slot) of the upward and downward
+    # passes, which run at the largest order in use.  They were measured on
+    # MI355X at 2^22 blobs with earlier kernels; the present ones take 4e-14 to
+    # 1e-13 a multiply-add and 4.8e-13 to 6.6e-13 a pair (uniform, Plummer, blob
+    # and mixed sets of 2^20 to 2^24).  Only their ratios decide: of nine sets of
+    # 2^17 to 2^24, six run on the faster of 0.5 and 0.55, three on an angle up to
+    # 12% slower, and a price of 5.8e-13 a pair changes one choice, to the slower.
     COST_M2L_HARMONIC = 8.0e-14
     COST_M2L_FULL = 5.9e-14
     COST_P2P_PAIR = 6.4e-13
