@@ -12,7 +12,8 @@
 //   * a group is (tile, key): at most one source per tile column (the
 //     source of a target at a given key is unique), so the group is one
 //     16-column operand of the tile's GEMM; the tile's group list is cut
-//     into chunks (one wavefront each) whose results add atomically.
+//     into chunks (a block each) whose results add atomically, or are stored
+//     and added in order (m2l_parts).
 #include <cstring>
 
 #include <rocprim/rocprim.hpp>
